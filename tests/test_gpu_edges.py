@@ -34,3 +34,38 @@ def test_relax_reports_the_largest_overlap(n):
     assert it == 1
     # the same operations in another order: a few ulps of the cell edge
     assert abs(ov - best) <= 16 * np.finfo(float).eps * cell
+
+
+@pytest.mark.parametrize("n,fill,periodic", [(513, .3, True), (2049, .3, False), (4100, .5, True), (3000, 1e-3, True),
+                                              (3000, 2e-6, True), (3000, 1e-5, False)])
+def test_pair_set_over_cells_per_sphere(n, fill, periodic):
+    # dense cells (ordered by counting), a few cells per sphere, and far more cells than spheres
+    # (ordered by sorting, or hashed): the potential pairs are those of an all-pairs test, and a
+    # second refresh of the same positions keeps them
+    from woo_amd._native import SPHERE, Device
+
+    rng = np.random.default_rng(n)
+    r = rng.uniform(2e-3, 3e-3, n)
+    L = (float(np.sum(4 / 3. * np.pi * r ** 3)) / fill) ** (1 / 3.)
+    pos = rng.uniform(0., L, (n, 3))
+    # half of the spheres close to another, so that sparse scenes have pairs too
+    pos[1::2] = pos[0::2][:len(pos[1::2])] + rng.normal(0., 2e-3, (len(pos[1::2]), 3))
+    d = Device(0)
+    d.set_field(periodic=periodic, cell=(L,) * 3)
+    d.set_materials([dict(kind=0, density=1., young=1., ktDivKn=.2, tanPhi=.5, surfEnergy=0., alpha=0.)])
+    d.upload_particles(shape=np.full(n, SPHERE, np.int32), pos=pos, radius=r, mass=np.ones(n),
+                       inertia=np.ones((n, 3)), vel=np.zeros((n, 3)))
+    vd = .05 * float(r.min())
+    want = set()
+    for k in range(0, n, 500):
+        dx = pos[k:k + 500, None] - pos[None]
+        if periodic:
+            dx -= L * np.round(dx / L)
+        hit = np.all(np.abs(dx) <= (r[k:k + 500, None] + r[None] + 2 * vd)[..., None], axis=-1)
+        i, j = np.nonzero(hit)
+        want |= {(a + k, b) for a, b in zip(i.tolist(), j.tolist()) if a + k < b}
+    for _ in range(2):
+        d.collide(-.05, forceInit=True)
+        ids = d.contacts(real_only=False, data=False)[0]
+        assert {(min(a, b), max(a, b)) for a, b in ids.tolist()} == want
+    np.testing.assert_array_equal(d.get("pos"), pos)

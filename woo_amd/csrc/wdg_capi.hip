@@ -567,7 +567,7 @@ int wdg_ctx_destroy(wdg_ctx* ctx) {
       c.snapEp[k].release();
     }
     c.snapMatch.release();
-    c.sortHist.release(); c.scanAux.release(); c.red.release(); c.xfer.release(); c.dflags.release();
+    c.sortHist.release(); c.scanWords.release(); c.scanTicket.release(); c.cellCnt.release(); c.cellRank.release(); c.red.release(); c.xfer.release(); c.dflags.release();
     if (c.hflags) (void)hipHostFree(c.hflags);
     if (c.stream) (void)hipStreamDestroy(c.stream);
   });

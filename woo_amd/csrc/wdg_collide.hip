@@ -274,20 +274,57 @@ __device__ __forceinline__ void scene_cell(const double p[3], const SceneGrid& G
 // cell key of every sphere (storage [s0,n)); value = current storage index
 __global__ void k_keys(int64_t s0, int64_t n, const double* __restrict__ px, const double* __restrict__ py,
                        const double* __restrict__ pz, Grid g, const uint32_t* __restrict__ scene, uint32_t* key,
-                       uint32_t* idx) {
+                       uint32_t* idx, uint32_t* cnt, uint32_t* rank) {
   int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int64_t s = s0 + t;
   if (s >= n) return;
   double p[3] = {px[s], py[s], pz[s]};
+  uint32_t k;
   if (g.sg) {
     const SceneGrid& G = g.sg[scene[s]];
     int c[3];
     scene_cell(p, G, c);
-    key[t] = G.off + (uint32_t)(((int64_t)c[2] * G.nc[1] + c[1]) * G.nc[0] + c[0]);
+    k = G.off + (uint32_t)(((int64_t)c[2] * G.nc[1] + c[1]) * G.nc[0] + c[0]);
   } else {
-    key[t] = cell_key(p, g);
+    k = cell_key(p, g);
   }
-  idx[t] = (uint32_t)s;
+  key[t] = k;
+  if (cnt) rank[t] = atomicAdd(&cnt[k], 1u);
+  else idx[t] = (uint32_t)s;
+}
+
+// Spheres in cell order by counting, with the spheres of a cell in their previous order (what a
+// stable sort by cell gives). k_keys counts the spheres of each cell (a sphere's place in the
+// count depends on the race), the counts are scanned, k_cell_place puts each sphere into its
+// cell's range and k_cell_rank ranks it there among its cell's few by its previous place. The
+// scanned counts are the cells' starts that the pair pass reads. Five launches, bound by latency;
+// the radix passes it replaces (histogram, scan, scatter, each three times), the search for the
+// cells' starts and the storage-index and record kernels took 190 us of a refresh of 150,000
+// spheres, these with the permutation 60 us.
+__global__ void k_cell_place(int64_t nSph, int64_t nW, const uint32_t* __restrict__ key,
+                             const uint32_t* __restrict__ rank, const uint32_t* __restrict__ cbeg, uint32_t* placed) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < nSph) placed[cbeg[key[t]] - (uint32_t)nW + rank[t]] = (uint32_t)t;
+}
+// perm[new storage] = old storage, its inverse, and the key of each sphere in the new order;
+// boundary bodies keep their place
+__global__ void k_cell_rank(int64_t n, int64_t nW, const uint32_t* __restrict__ key,
+                            const uint32_t* __restrict__ cbeg, const uint32_t* __restrict__ placed, uint32_t* perm,
+                            uint32_t* invPerm, uint32_t* sortedKey) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  if (i < nW) {
+    perm[i] = (uint32_t)i;
+    invPerm[i] = (uint32_t)i;
+    return;
+  }
+  const uint32_t w = (uint32_t)nW, v = placed[i - nW], k = key[v];
+  const uint32_t b = cbeg[k], e = cbeg[k + 1];
+  uint32_t s = b;
+  for (uint32_t q = b; q < e; q++) s += placed[q - w] < v ? 1u : 0u;
+  perm[s] = v + w;
+  invPerm[v + w] = s;
+  sortedKey[s - w] = k;
 }
 
 // bounding box and sphere count of every scene (ordered bits of the bounds, as k_bbox): per
@@ -346,47 +383,51 @@ struct PermArgs {
   double* dd[NPD];
   const uint32_t* su[NPU];
   uint32_t* du[NPU];
+  // the refresh positions and the pair pass's float records, and the storage index of each user id
+  Grid g;
+  double absDf, vd0;
+  const double* vdS;
+  double *lx, *ly, *lz;
+  float4* pf;
+  uint32_t* sto;
 };
+// Every particle array in the new storage order; with the values in registers also the refresh
+// positions, the user ids' storage index, and per particle the float record the pair kernel
+// filters candidates with: position relative to the grid (wrapped into the cell when periodic) and
+// the AABB half-size |distFactor|*r + verletDist. Bound by its 464 bytes per particle at the rate
+// of a copy (1M: 95 us; as three kernels 116 us).
 __global__ __launch_bounds__(256) void k_permute(PermArgs a) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.n) return;
   const uint32_t o = a.perm[i];
+  double d[NPD];
+  uint32_t u[NPU];
 #pragma unroll
-  for (int k = 0; k < NPD; k++) a.dd[k][i] = a.sd[k][o];
+  for (int k = 0; k < NPD; k++) d[k] = a.sd[k][o];
 #pragma unroll
-  for (int k = 0; k < NPU; k++) a.du[k][i] = a.su[k][o];
-}
-
-__global__ void k_sto(int64_t n, const uint32_t* __restrict__ uid, uint32_t* sto) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) sto[uid[i]] = (uint32_t)i;
-}
-
-// refresh positions, and per particle the float record the pair kernel filters candidates
-// with: position relative to the grid (wrapped into the cell when periodic) and the
-// AABB half-size |distFactor|*r + verletDist
-__global__ void k_last_pos(int64_t n, const double* __restrict__ px, const double* __restrict__ py,
-                           const double* __restrict__ pz, const double* __restrict__ rad, Grid g, double absDf,
-                           double vd0, const double* __restrict__ vdS, const uint32_t* __restrict__ scene,
-                           const uint32_t* __restrict__ flags, double* lx, double* ly, double* lz, float4* pf) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double p[3] = {px[i], py[i], pz[i]};
-  lx[i] = p[0];
-  ly[i] = p[1];
-  lz[i] = p[2];
+  for (int k = 0; k < NPU; k++) u[k] = a.su[k][o];
+#pragma unroll
+  for (int k = 0; k < NPD; k++) a.dd[k][i] = d[k];
+#pragma unroll
+  for (int k = 0; k < NPU; k++) a.du[k][i] = u[k];
+  // the order of the arrays: pos first, radius last; flags, mask, uid, mat, scene
+  a.sto[u[2]] = (uint32_t)i;
+  a.lx[i] = d[0];
+  a.ly[i] = d[1];
+  a.lz[i] = d[2];
   float f[3];
   // relative to the origin of the sphere's grid (its scene's, with scene grids; the boundary
   // bodies' records are not read)
-  const double* org = g.org;
-  if (g.sg && !((flags[i] >> F_SHAPE_SHIFT) & 3u)) org = g.sg[scene[i]].org;
+  const double* org = a.g.org;
+  if (a.g.sg && !((u[0] >> F_SHAPE_SHIFT) & 3u)) org = a.g.sg[u[4]].org;
+#pragma unroll
   for (int k = 0; k < 3; k++) {
-    double x = p[k] - org[k];
-    if (g.periodic) x = x - floor(x / g.L[k]) * g.L[k];
+    double x = d[k] - org[k];
+    if (a.g.periodic) x = x - floor(x / a.g.L[k]) * a.g.L[k];
     f[k] = (float)x;
   }
-  const double vd = vd_at(vdS, scene, i, vd0);
-  pf[i] = make_float4(f[0], f[1], f[2], (float)(absDf * rad[i] + vd));
+  const double vd = a.vdS ? a.vdS[u[4]] : a.vd0;  // the scene's Verlet distance (vd_at)
+  a.pf[i] = make_float4(f[0], f[1], f[2], (float)(a.absDf * d[NPD - 1] + vd));
 }
 
 // enlarged AABB of every boundary body from its refresh position: Bo1_Wall_Aabb
@@ -1616,6 +1657,10 @@ static void refresh(Ctx& c) {
   c.cellKeyTmp.ensure(nSph + 1); c.sortIdxTmp.ensure(nSph + 1);
   c.perm.ensure(n + 1); c.invPerm.ensure(n + 1);
   c.scount.ensure(nSph + 1); c.soff.ensure(nSph + 1);
+  // by counting while the cells are no more than a few per sphere (a scan over them is then
+  // cheaper than the passes of a sort), else by sorting the keys: a periodic cell that is nearly
+  // empty. All-pairs keeps the order.
+  const bool counting = !brute && nSph > 0 && ncells <= std::max<int64_t>(16 * nSph, 4096);
   if (nSph > 0) {
     Grid gk = g;
     if (brute) {
@@ -1624,16 +1669,37 @@ static void refresh(Ctx& c) {
       gk.hashed = 0;
       gk.sg = nullptr;
     }
+    uint32_t* cnt = nullptr;
+    if (counting) {
+      c.cellCnt.ensure(ncells + 1);  // and a zero after them, so that the scan also gives the end
+      c.cellStart.ensure(ncells + 1);
+      c.cellRank.ensure(nSph + 1);
+      WDG_HIP(hipMemsetAsync(c.cellCnt.p, 0, (ncells + 1) * sizeof(uint32_t), c.stream));
+      cnt = c.cellCnt.p;
+    }
+    uint32_t* key = counting ? c.cellKeyTmp.p : c.cellKey.p;
     hipLaunchKernelGGL(k_keys, dim3(nblocks(nSph, 256)), dim3(256), 0, c.stream, nW, n, c.pos[0].p, c.pos[1].p,
-                       c.pos[2].p, gk, (const uint32_t*)c.scene.p, c.cellKey.p, c.sortIdx.p);
+                       c.pos[2].p, gk, (const uint32_t*)c.scene.p, key, c.sortIdx.p, cnt, c.cellRank.p);
     WDG_LAUNCH_CHECK();
-    if (!brute)
+    if (counting) {
+      scan_exclusive(c, c.cellCnt.p, c.cellStart.p, ncells + 1, c.dflags.p + 3, (uint32_t)nW);
+      const uint32_t* cb = c.cellStart.p;
+      hipLaunchKernelGGL(k_cell_place, dim3(nblocks(nSph, 256)), dim3(256), 0, c.stream, nSph, nW,
+                         (const uint32_t*)key, (const uint32_t*)c.cellRank.p, cb, c.sortIdx.p);
+      WDG_LAUNCH_CHECK();
+      hipLaunchKernelGGL(k_cell_rank, dim3(nblocks(n, 256)), dim3(256), 0, c.stream, n, nW, (const uint32_t*)key, cb,
+                         (const uint32_t*)c.sortIdx.p, c.perm.p, c.invPerm.p, c.cellKey.p);
+      WDG_LAUNCH_CHECK();
+    } else if (!brute) {
       radix_sort_pairs<uint32_t>(c, c.cellKey.p, c.sortIdx.p, c.cellKeyTmp.p, c.sortIdxTmp.p, nSph,
                                  bits_for((uint64_t)(ncells > 1 ? ncells - 1 : 1)));
+    }
   }
-  hipLaunchKernelGGL(k_build_perm, dim3(nblocks(n, 256)), dim3(256), 0, c.stream, nW, n, c.sortIdx.p, c.perm.p,
-                     c.invPerm.p);
-  WDG_LAUNCH_CHECK();
+  if (!counting) {
+    hipLaunchKernelGGL(k_build_perm, dim3(nblocks(n, 256)), dim3(256), 0, c.stream, nW, n, c.sortIdx.p, c.perm.p,
+                       c.invPerm.p);
+    WDG_LAUNCH_CHECK();
+  }
   {
     PermArgs pa{};
     pa.n = n;
@@ -1653,18 +1719,19 @@ static void refresh(Ctx& c) {
       pa.su[k] = u[k]->p;
       pa.du[k] = c.spareU[k].p;
     }
+    c.posf.ensure(n + 1);
+    pa.g = g;
+    pa.absDf = absDf;
+    pa.vd0 = vd;
+    pa.vdS = vdS;
+    pa.lx = c.lastPos[0].p; pa.ly = c.lastPos[1].p; pa.lz = c.lastPos[2].p;
+    pa.pf = c.posf.p;
+    pa.sto = c.sto.p;
     hipLaunchKernelGGL(k_permute, dim3(nblocks(n, 256)), dim3(256), 0, c.stream, pa);
     WDG_LAUNCH_CHECK();
     for (int k = 0; k < NPD; k++) d[k]->swap(c.spareD[k]);
     for (int k = 0; k < NPU; k++) u[k]->swap(c.spareU[k]);
   }
-  hipLaunchKernelGGL(k_sto, dim3(nblocks(n, 256)), dim3(256), 0, c.stream, n, c.uid.p, c.sto.p);
-  WDG_LAUNCH_CHECK();
-  c.posf.ensure(n + 1);
-  hipLaunchKernelGGL(k_last_pos, dim3(nblocks(n, 256)), dim3(256), 0, c.stream, n, c.pos[0].p, c.pos[1].p,
-                     c.pos[2].p, c.radius.p, g, absDf, vd, vdS, (const uint32_t*)c.scene.p,
-                     (const uint32_t*)c.flags.p, c.lastPos[0].p, c.lastPos[1].p, c.lastPos[2].p, c.posf.p);
-  WDG_LAUNCH_CHECK();
   if (nW > 0) {
     c.bnd.ensure((size_t)6 * nW);
     hipLaunchKernelGGL(k_bnd_bounds, dim3(nblocks(nW, 256)), dim3(256), 0, c.stream, nW, c.lastPos[0].p,
@@ -1672,7 +1739,7 @@ static void refresh(Ctx& c) {
                        c.bnd.p);
     WDG_LAUNCH_CHECK();
   }
-  if (nSph > 0 && !brute) {
+  if (nSph > 0 && !brute && !counting) {
     c.cellStart.ensure(ncells + 1);
     hipLaunchKernelGGL(k_cell_begin, dim3(nblocks(ncells + 1, 256)), dim3(256), 0, c.stream, nSph, nW, c.cellKey.p,
                        ncells, c.cellStart.p);

@@ -346,7 +346,12 @@ struct Ctx {
   // adjacency of high-degree particles (boundary bodies), sorted by one radix sort
   DBuf<uint32_t> bigOff, bigRank, bigVal, bigValTmp, bigDest, bigList;
   DBuf<uint64_t> bigKey, bigKeyTmp;
-  DBuf<uint32_t> sortHist, scanAux;
+  DBuf<uint32_t> sortHist;
+  // prefix scans: a word per tile, the number of the last scan, the tile tickets given out so far
+  DBuf<uint64_t> scanWords;
+  DBuf<uint32_t> scanTicket;
+  uint32_t scanEpoch = 0, scanTickets = 0;
+  DBuf<uint32_t> cellCnt, cellRank;  // spheres per cell, each sphere's place in its cell's count
   DBuf<uint32_t> act;     // slot of each state index (contact loop), per-slot flags (relaxation)
   DBuf<uint4> desc;       // contact loop: the filter's record of each real slot, by state index
   DBuf<uint64_t> descDist;
@@ -424,7 +429,8 @@ struct Ctx {
 };
 
 // ------------------------------------------------------------------ internal API
-void scan_exclusive(Ctx& c, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* dTotal);
+// out[i] = first + the sum of in[0 .. i-1], *dTotal = first + the sum of all (in may be out)
+void scan_exclusive(Ctx& c, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* dTotal, uint32_t first = 0);
 template <class K>
 void radix_sort_pairs(Ctx& c, K* keys, uint32_t* vals, K* keysTmp, uint32_t* valsTmp, int64_t n, int bits);
 uint32_t read_u32(Ctx& c, const uint32_t* d);
