@@ -69,3 +69,32 @@ def test_pair_set_over_cells_per_sphere(n, fill, periodic):
         ids = d.contacts(real_only=False, data=False)[0]
         assert {(min(a, b), max(a, b)) for a, b in ids.tolist()} == want
     np.testing.assert_array_equal(d.get("pos"), pos)
+
+
+@pytest.mark.parametrize("n", [3, 511, 512, 39999, 40001, 100001])
+def test_pairs_over_lanes_per_sphere(n):
+    # the pair pass's lanes per sphere change with the size; the real contacts of a jittered lattice
+    # are those found cell by cell on the host
+    from scipy.spatial import cKDTree
+
+    from woo_amd._native import SPHERE, Device
+
+    rng = np.random.default_rng(n)
+    m = int(np.ceil(n ** (1 / 3.)))
+    pos = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n] * 2e-3
+    pos = pos + rng.uniform(-1e-4, 1e-4, pos.shape)
+    r = rng.uniform(.9e-3, 1.05e-3, n)
+    mass = 1e-5 * np.ones(n)
+    d = Device(0)
+    d.set_field(periodic=False)
+    d.set_materials([dict(kind=0, density=1., young=1e6, ktDivKn=.2, tanPhi=.5, surfEnergy=0., alpha=0.)])
+    d.upload_particles(shape=np.full(n, SPHERE, np.int32), pos=pos, radius=r, mass=mass,
+                       inertia=np.repeat((.4 * mass * r * r)[:, None], 3, 1), vel=np.zeros((n, 3)))
+    d.collide(-.05)
+    d.contact_loop(0, 1e-7)
+    got = d.contacts(real_only=True, data=False)[0]
+    p = cKDTree(pos).query_pairs(2.2e-3, output_type="ndarray")
+    p = p[np.linalg.norm(pos[p[:, 0]] - pos[p[:, 1]], axis=1) < r[p[:, 0]] + r[p[:, 1]]]
+    want = np.sort(p, axis=1)
+    assert len(want) > n // 4 or n == 3
+    np.testing.assert_array_equal(np.sort(got, axis=1), want[np.lexsort((want[:, 1], want[:, 0]))])

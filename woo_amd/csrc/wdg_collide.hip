@@ -538,53 +538,59 @@ constexpr int BLIST = 256;
 // and every wall. Each pair is emitted once, by its sphere of lower storage index. With
 // OUT_STAGE the sphere also records every neighbour (j < s too, with the same test, whose
 // arithmetic follows the canonical pA/pB roles and so gives the same answer from either
-// side), which is its adjacency list. A float test on the grid-relative positions rejects
-// far candidates before the exact test; its margin keeps it from rejecting any pair.
-constexpr int PAIR_Q = 16;  // candidates queued per sphere for the exact test
+// side), which is its adjacency list. A float test on the grid-relative positions decides most
+// candidates; its margin keeps it from rejecting any pair or accepting anything else.
+//
+// G lanes share a sphere: each walks a part of its candidates and queues those that pass the
+// float test; the queues are worked off by the whole wavefront together, a group's finds placed
+// one after the other by ballots (a fixed order: rounds of the queue, lanes within a round).
+// Bound by the latency of the loads and of the instructions between them (a sphere has about 70
+// candidates in 27 cells, some 5,000 instructions): one lane a sphere left 2 wavefronts a SIMD
+// at 150,000 spheres and less below; before, each lane loaded one candidate at a time and tested
+// every queued one in FP64: 72 us for 300 spheres, 60 us for 20,000, 107 us for 150,000, 293 us
+// for 1M. pair_lanes gives the figures now.
+constexpr int PAIR_Q = 12;  // candidates queued per lane
+constexpr int PAIR_B = 4;   // candidates read together
+constexpr uint32_t PAIR_SURE = 0x80000000u;  // queued candidate: a pair for certain
+// the cells of the spheres: none (all pairs), rows along x (one grid or a grid per scene), Morton
+// codes, hashed
+enum { CELL_NONE = 0, CELL_ROWS = 1, CELL_MORTON = 2, CELL_HASHED = 3 };
 
-template <int OUT, int MODE>
+template <int OUT, int MODE, int KIND, int G>
 __global__ __launch_bounds__(256) void k_pairs(PairArgs a) {
-  // Candidates that pass the float test wait in a per-thread LDS queue and get the exact test
-  // in a batch: a wavefront then runs the exact test for most of its lanes at once, instead of
-  // at nearly every candidate step for the few lanes whose candidate passed.
   __shared__ uint32_t sq[PAIR_Q][256];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, g = threadIdx.x & (G - 1);
   // consecutive workgroups on one XCD: a sphere's neighbour cells are mostly in its own XCD's L2
-  const int64_t s = a.nW + (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const int64_t s = a.nW + ((int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x) / G;
   const bool live = s < a.n;
-  uint32_t cnt = 0, ndeg = 0;
-  // enlarged AABB of this sphere, and of the wavefront's and the workgroup's spheres: the
-  // workgroup lists the boundary bodies its box meets (in body order), each wavefront skips
-  // those its own box misses, each sphere tests the rest
+  const int64_t sl = live ? s : a.n - 1;  // a sphere to read for the lanes past the end
+  const int64_t t = sl - a.nW;
+  uint32_t cnt = 0, ndeg = 0;  // pairs and neighbours of the sphere so far (the same in its lanes)
+  const double ps[3] = {a.px[sl], a.py[sl], a.pz[sl]};
+  const double rs = a.rad[sl];
+  const uint32_t ms = a.mask[sl], us = a.uid[sl];
+  const uint32_t scs = a.scene ? a.scene[sl] : 0u;
+  const float4 fs = a.pf[sl];
+  // this sphere's Verlet distance (its scene's; the pairs never cross scenes)
+  const double vds = vd_at(a.vdS, a.scene, sl, a.P.vd);
+  // enlarged AABB of the wavefront's and the workgroup's spheres: the workgroup lists the boundary
+  // bodies its box meets (in body order), each wavefront skips those its own box misses, each
+  // sphere tests the rest
   __shared__ uint32_t blist[BLIST];
   __shared__ uint32_t bwc[4];
   __shared__ double bbox[4][6];
   __shared__ int bcount;
-  double slo[3] = {INFINITY, INFINITY, INFINITY}, shi[3] = {-INFINITY, -INFINITY, -INFINITY};
-  double wlo[3], whi[3];
   int nb = 0;
   bool bfull = false;
-  // this sphere's Verlet distance (its scene's; the pairs never cross scenes)
-  const double vds = live ? vd_at(a.vdS, a.scene, s, a.P.vd) : a.P.vd;
-  if (a.nW > 0 && live && a.sceneBodyOff) {
-    const double p[3] = {a.px[s], a.py[s], a.pz[s]};
-    const double h = a.P.absDf * a.rad[s];
-    for (int k = 0; k < 3; k++) sph_bounds(p[k], h, vds, slo[k], shi[k]);
-  }
   if (a.nW > 0 && !a.sceneBodyOff) {
-    if (live) {
-      const double p[3] = {a.px[s], a.py[s], a.pz[s]};
-      const double h = a.P.absDf * a.rad[s];
-      for (int k = 0; k < 3; k++) sph_bounds(p[k], h, vds, slo[k], shi[k]);
-    }
+    double wlo[3], whi[3];
     for (int k = 0; k < 3; k++) {
-      wlo[k] = slo[k];
-      whi[k] = shi[k];
+      sph_bounds(ps[k], a.P.absDf * rs, vds, wlo[k], whi[k]);
       for (int off = 32; off > 0; off >>= 1) {
         wlo[k] = fmin(wlo[k], __shfl_xor(wlo[k], off));
         whi[k] = fmax(whi[k], __shfl_xor(whi[k], off));
       }
     }
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (lane == 0)
       for (int k = 0; k < 3; k++) {
         bbox[wv][k] = wlo[k];
@@ -620,229 +626,261 @@ __global__ __launch_bounds__(256) void k_pairs(PairArgs a) {
     nb = bcount;
     bfull = nb > BLIST;  // too many for the list: every body is tested
   }
-  if (live) {
-    const double ps[3] = {a.px[s], a.py[s], a.pz[s]};
-    const double rs = a.rad[s];
-    const uint32_t ms = a.mask[s], us = a.uid[s];
-    const float4 fs = a.pf[s];
-    const int64_t t = s - a.nW;
-    const int64_t o = (OUT == OUT_SLOTS || OUT == OUT_KEYS) ? (int64_t)a.off[t] : t;
-    // staged arrays are neighbour-major: entry q of sphere t at q * nSph + t
-    auto emit = [&](uint32_t partner, uint32_t lo, uint32_t hi, uint32_t info, uint64_t cd, uint64_t ukey) {
+  const int64_t o = (OUT == OUT_SLOTS || OUT == OUT_KEYS) ? (int64_t)a.off[t] : t;
+  const unsigned long long gmask = (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << (lane & ~(G - 1));
+  const unsigned long long below = gmask & ((1ull << lane) - 1ull);
+  // One find of each lane (hit): neighbour j, and with gen the pair itself. Every lane of the
+  // wavefront calls it. Staged arrays are neighbour-major: entry q of sphere t at q * nSph + t.
+  auto emit = [&](bool hit, bool gen, uint32_t partner, uint32_t lo, uint32_t hi, uint32_t info, uint64_t cd,
+                  uint64_t ukey) {
+    const unsigned long long H = __ballot(hit), P = __ballot(hit && gen);
+    if (hit && OUT == OUT_STAGE) {
+      const uint32_t d = ndeg + (uint32_t)__popcll(H & below);
+      if (d < (uint32_t)a.nbStage) a.nb[(int64_t)d * a.nSph + t] = partner;
+    }
+    if (hit && gen) {
+      const uint32_t c = cnt + (uint32_t)__popcll(P & below);
       if (OUT == OUT_STAGE) {
-        if (cnt < (uint32_t)a.stage) {
-          const int64_t e = (int64_t)cnt * a.nSph + o;
+        if (c < (uint32_t)a.stage) {
+          const int64_t e = (int64_t)c * a.nSph + o;
           a.sA[e] = partner;
           a.sInfo[e] = info;
           if (a.P.periodic) a.sDist[e] = cd;
         }
       } else if (OUT == OUT_SLOTS) {
-        a.sA[o + cnt] = lo;
-        a.sB[o + cnt] = hi;
-        a.sInfo[o + cnt] = info;
-        a.sCarry[o + cnt] = 0u;
-        if (a.P.periodic) a.sDist[o + cnt] = cd;
+        a.sA[o + c] = lo;
+        a.sB[o + c] = hi;
+        a.sInfo[o + c] = info;
+        a.sCarry[o + c] = 0u;
+        if (a.P.periodic) a.sDist[o + c] = cd;
       } else if (OUT == OUT_KEYS) {
-        a.pkey[o + cnt] = ukey;
-        if (a.P.periodic) a.pdist[o + cnt] = cd;
+        a.pkey[o + c] = ukey;
+        if (a.P.periodic) a.pdist[o + c] = cd;
       }
-      cnt++;
-    };
-    auto neighbour = [&](uint32_t j) {
-      if (OUT == OUT_STAGE) {
-        if (ndeg < (uint32_t)a.nbStage) a.nb[(int64_t)ndeg * a.nSph + t] = j;
-        ndeg++;
-      }
-    };
-    // the exact test of a candidate that passed the float test (the periodic image is found
-    // again in FP64 by sph_overlap)
-    auto exact = [&](int64_t j) {
-      if (!may_collide(ms, a.mask[j], a.P.loneMask)) return;
-      if (a.scene && a.scene[j] != a.scene[s]) return;
-      const double pj[3] = {a.px[j], a.py[j], a.pz[j]};
-      const double rj = a.rad[j];
+    }
+    ndeg += (uint32_t)__popcll(H & gmask);
+    cnt += (uint32_t)__popcll(P & gmask);
+  };
+  // the exact test of a candidate that the float test left open (the periodic image is found
+  // again in FP64 by sph_overlap)
+  auto exact = [&](int64_t j, bool sIsA, const double (&pj)[3], uint64_t& pcd) {
+    const double rj = a.rad[j];
+    // canonical roles: the smaller user id is pA
+    const double* pa = sIsA ? ps : pj;
+    const double* pb = sIsA ? pj : ps;
+    const double ra = sIsA ? rs : rj, rb = sIsA ? rj : rs;
+    int cd[3], nimg;
+    if (!sph_overlap(pa, a.P.absDf * ra, pb, a.P.absDf * rb, a.P, vds, cd, nimg)) return false;
+    if (a.P.periodic && nimg > 1) {
+      atomicOr(&a.dflags[1], ERR_DOUBLE_IMAGE);
+      return false;
+    }
+    if (MODE == MODE_NEAR) {
+      // centres within reach before the next refresh
+      d3 d = mk3(pb[0] + a.P.L[0] * cd[0] * a.P.periodic - pa[0], pb[1] + a.P.L[1] * cd[1] * a.P.periodic - pa[1],
+                 pb[2] + a.P.L[2] * cd[2] * a.P.periodic - pa[2]);
+      double reach = a.P.absDf * (ra + rb) + 2 * vds;
+      if (sqn3(d) > reach * reach * (1 + 1e-9)) return false;
+    }
+    pcd = a.P.periodic ? pack_cd(cd[0], cd[1], cd[2]) : 0ull;
+    return true;
+  };
+  int nq = 0;
+  // Works off the queues. A candidate that the float test accepted for certain needs its periodic
+  // image only: the pair is far nearer than half a period on every axis, so the nearest integer is
+  // that of near_img.
+  auto flush = [&]() {
+    for (int k = 0; __any(k < nq); k++) {
+      bool hit = k < nq;
+      const uint32_t e = hit ? sq[k][threadIdx.x] : (uint32_t)sl;
+      const uint32_t j = e & ~PAIR_SURE;
       const uint32_t uj = a.uid[j];
-      // canonical roles: the smaller user id is pA
       const bool sIsA = us < uj;
-      const double* pa = sIsA ? ps : pj;
-      const double* pb = sIsA ? pj : ps;
-      const double ra = sIsA ? rs : rj, rb = sIsA ? rj : rs;
-      int cd[3], nimg;
-      if (!sph_overlap(pa, a.P.absDf * ra, pb, a.P.absDf * rb, a.P, vds, cd, nimg)) return;
-      if (a.P.periodic && nimg > 1) {
-        atomicOr(&a.dflags[1], ERR_DOUBLE_IMAGE);
-        return;
-      }
-      if (MODE == MODE_NEAR) {
-        // centres within reach before the next refresh
-        d3 d = mk3(pb[0] + a.P.L[0] * cd[0] * a.P.periodic - pa[0], pb[1] + a.P.L[1] * cd[1] * a.P.periodic - pa[1],
-                   pb[2] + a.P.L[2] * cd[2] * a.P.periodic - pa[2]);
-        double reach = a.P.absDf * (ra + rb) + 2 * vds;
-        if (sqn3(d) > reach * reach * (1 + 1e-9)) return;
-      }
-      neighbour((uint32_t)j);
-      if (j < s) return;
-      const uint64_t pcd = a.P.periodic ? pack_cd(cd[0], cd[1], cd[2]) : 0ull;
-      emit((uint32_t)j, (uint32_t)s, (uint32_t)j, (uint32_t)CT_SS | CI_NEAR | (sIsA ? 0u : CI_SWAP), pcd,
-           sIsA ? (((uint64_t)us << 32) | uj) : (((uint64_t)uj << 32) | us));
-    };
-    int nq = 0;
-    auto flush = [&]() {
-      for (int k = 0; k < nq; k++) exact((int64_t)sq[k][threadIdx.x]);
-      nq = 0;
-    };
-    // the float test of candidate j with the periodic shift of its cell; passing candidates
-    // are queued in scan order, so pairs and neighbours come out in that order
-    auto consider = [&](int64_t j, float sx, float sy, float sz) {
-      if (OUT == OUT_STAGE ? j == s : j <= s) return;
-      const float4 fj = a.pf[j];
-      const float dx = (fj.x + sx) - fs.x, dy = (fj.y + sy) - fs.y, dz = (fj.z + sz) - fs.z;
-      const float R = (fs.w + fj.w) + a.margin;
-      if (fabsf(dx) > R || fabsf(dy) > R || fabsf(dz) > R) return;
-      // the centre-distance test must not hide a pair whose AABBs overlap through two
-      // periodic images (an error below); that needs fewer than 3 cells along an axis,
-      // which is the all-pairs path
-      if (MODE == MODE_NEAR && !a.brute && (dx * dx + dy * dy) + dz * dz > R * R) return;
-      sq[nq][threadIdx.x] = (uint32_t)j;
-      if (++nq == PAIR_Q) flush();
-    };
-    if (a.brute) {
-      for (int64_t j = a.nW; j < a.n; j++) {
-        float sh[3] = {0.f, 0.f, 0.f};
-        if (a.P.periodic) {
-          const float4 fj = a.pf[j];
-          const float d[3] = {fj.x - fs.x, fj.y - fs.y, fj.z - fs.z};
-          for (int m = 0; m < 3; m++) sh[m] = -(float)a.P.L[m] * rintf(d[m] / (float)a.P.L[m]);
-        }
-        consider(j, sh[0], sh[1], sh[2]);
-      }
-    } else if (a.g.hashed) {
-      // the 27 neighbour cells one by one (their buckets are not consecutive); a bucket shared
-      // by two of them (a hash collision) is walked once, at the first; a sphere of a far cell
-      // in a walked bucket fails the float test
-      int c[3];
-      const double pc[3] = {a.px[s], a.py[s], a.pz[s]};
-      cell_coords(pc, a.g, c);
-      for (int m = 0; m < 27; m++) {
-        const int q0 = c[0] + m % 3 - 1, q1 = c[1] + (m / 3) % 3 - 1, q2 = c[2] + m / 9 - 1;
-        if (q0 < 0 || q1 < 0 || q2 < 0 || q0 >= a.g.nc[0] || q1 >= a.g.nc[1] || q2 >= a.g.nc[2]) continue;
-        const uint32_t b = cell_hash(q0, q1, q2, a.g.hmask);
-        bool seen = false;
-        for (int m2 = 0; m2 < m && !seen; m2++) {
-          const int r0 = c[0] + m2 % 3 - 1, r1 = c[1] + (m2 / 3) % 3 - 1, r2 = c[2] + m2 / 9 - 1;
-          if (r0 < 0 || r1 < 0 || r2 < 0 || r0 >= a.g.nc[0] || r1 >= a.g.nc[1] || r2 >= a.g.nc[2]) continue;
-          seen = cell_hash(r0, r1, r2, a.g.hmask) == b;
-        }
-        if (seen) continue;
-        const uint32_t t0 = a.cbeg[b], t1 = a.cbeg[b + 1];
-        for (uint32_t tt = t0; tt < t1; tt++) consider(tt, 0.f, 0.f, 0.f);
-      }
-    } else if (a.g.morton) {
-      // Morton keys: the 27 neighbour cells one by one (a row's cells are not consecutive
-      // keys); a cell across a periodic boundary is its image, one period away (every axis
-      // has at least 3 cells, so the 27 are distinct)
-      const uint32_t k = a.key[t];
-      const int c0 = (int)gather_bits3(k), c1 = (int)gather_bits3(k >> 1), c2 = (int)gather_bits3(k >> 2);
-      for (int m = 0; m < 27; m++) {
-        int q[3] = {c0 + m % 3 - 1, c1 + (m / 3) % 3 - 1, c2 + m / 9 - 1};
-        float sh[3] = {0.f, 0.f, 0.f};
-        bool ok = true;
-        for (int d = 0; d < 3; d++)
-          if (q[d] < 0 || q[d] >= a.g.nc[d]) {
-            ok = ok && a.g.periodic;
-            sh[d] = q[d] < 0 ? -(float)a.g.L[d] : (float)a.g.L[d];
-            q[d] = (q[d] + a.g.nc[d]) % a.g.nc[d];
+      hit = hit && may_collide(ms, a.mask[j], a.P.loneMask) && (!a.scene || a.scene[j] == scs);
+      uint64_t pcd = 0ull;
+      if (hit && (a.P.periodic || !(e & PAIR_SURE))) {
+        const double pj[3] = {a.px[j], a.py[j], a.pz[j]};
+        if (!(e & PAIR_SURE)) {
+          hit = exact((int64_t)j, sIsA, pj, pcd);
+        } else {
+          int cd[3];
+#pragma unroll
+          for (int d = 0; d < 3; d++) {
+            const int c = (int)rint((pj[d] - ps[d]) / a.P.L[d]);
+            cd[d] = sIsA ? -c : c;
           }
-        if (!ok) continue;
-        const uint32_t b = morton3(q[0], q[1], q[2]);
-        const uint32_t t0 = a.cbeg[b], t1 = a.cbeg[b + 1];
-        for (uint32_t tt = t0; tt < t1; tt++) consider(tt, sh[0], sh[1], sh[2]);
+          pcd = pack_cd(cd[0], cd[1], cd[2]);
+        }
       }
+      emit(hit, (int64_t)j > s, j, (uint32_t)s, j, (uint32_t)CT_SS | CI_NEAR | (sIsA ? 0u : CI_SWAP), pcd,
+           sIsA ? (((uint64_t)us << 32) | uj) : (((uint64_t)uj << 32) | us));
+    }
+    nq = 0;
+  };
+  // The float test of candidate j with the periodic shift of its cell. Its margin covers the
+  // rounding of the float positions many times over, so a candidate beyond reach plus margin is
+  // no pair, one within reach minus margin is one, and only those between need the exact test.
+  auto consider = [&](int64_t j, const float4& fj, float sx, float sy, float sz) {
+    if (OUT == OUT_STAGE ? j == s : j <= s) return;
+    if (KIND == CELL_NONE && a.P.periodic) {
+      const float d[3] = {fj.x - fs.x, fj.y - fs.y, fj.z - fs.z};
+      sx = -(float)a.P.L[0] * rintf(d[0] / (float)a.P.L[0]);
+      sy = -(float)a.P.L[1] * rintf(d[1] / (float)a.P.L[1]);
+      sz = -(float)a.P.L[2] * rintf(d[2] / (float)a.P.L[2]);
+    }
+    const float dx = (fj.x + sx) - fs.x, dy = (fj.y + sy) - fs.y, dz = (fj.z + sz) - fs.z;
+    const float R = (fs.w + fj.w) + a.margin;
+    const float mx = fmaxf(fmaxf(fabsf(dx), fabsf(dy)), fabsf(dz));
+    if (mx > R) return;
+    const float d2 = (dx * dx + dy * dy) + dz * dz;
+    // the centre-distance test must not hide a pair whose AABBs overlap through two
+    // periodic images (an error below); that needs fewer than 3 cells along an axis,
+    // which is the all-pairs path
+    if (MODE == MODE_NEAR && KIND != CELL_NONE && d2 > R * R) return;
+    const float Ri = R - 2.f * a.margin;
+    const bool sure = KIND != CELL_NONE && Ri > 0.f && (MODE == MODE_NEAR ? d2 < Ri * Ri : mx < Ri);
+    sq[nq++][threadIdx.x] = (uint32_t)j | (sure ? PAIR_SURE : 0u);
+  };
+  // The candidates as M storage ranges [t0, t1), each with the periodic shift of its cells; the
+  // lane takes ranges m0 .. m1 - 1 (all pairs: a part of the one range).
+  struct Range {
+    uint32_t t0, t1;
+    float sx, sy, sz;
+  };
+  int M = G;
+  int c[3] = {0, 0, 0}, nc[3] = {a.g.nc[0], a.g.nc[1], a.g.nc[2]};
+  uint32_t kbase = 0u;
+  int xlo = 0, xhi = 0, xw = -1;
+  float xwsh = 0.f;
+  if (KIND == CELL_HASHED) {
+    cell_coords(ps, a.g, c);
+    M = 27;
+  } else if (KIND == CELL_MORTON) {
+    const uint32_t k = a.key[t];
+    for (int d = 0; d < 3; d++) c[d] = (int)gather_bits3(k >> d);
+    M = 27;
+  } else if (KIND == CELL_ROWS) {
+    // the sphere's grid: its scene's (keys from the scene's offset), or the one grid
+    uint32_t k = a.key[t];
+    if (a.g.sg) {
+      const SceneGrid& S = a.g.sg[scs];
+      kbase = S.off;
+      for (int d = 0; d < 3; d++) nc[d] = S.nc[d];
+      k -= kbase;
+    }
+    c[0] = (int)(k % (uint32_t)nc[0]);
+    c[1] = (int)((k / (uint32_t)nc[0]) % (uint32_t)nc[1]);
+    c[2] = (int)(k / ((uint32_t)nc[0] * (uint32_t)nc[1]));
+    xlo = c[0] > 0 ? c[0] - 1 : 0;
+    xhi = c[0] + 1 < nc[0] ? c[0] + 1 : nc[0] - 1;
+    if (a.g.periodic && c[0] == 0) { xw = nc[0] - 1; xwsh = -(float)a.g.L[0]; }
+    if (a.g.periodic && c[0] == nc[0] - 1) { xw = 0; xwsh = (float)a.g.L[0]; }
+    M = a.g.periodic ? 18 : 9;
+  }
+  const int m1 = live ? (g + 1) * M / G : 0;
+  auto range = [&](int m) {
+    Range r{0u, 0u, 0.f, 0.f, 0.f};
+    if (m >= m1) return r;
+    if (KIND == CELL_NONE) {
+      r.t0 = (uint32_t)(a.nW + a.nSph * m / G);
+      r.t1 = (uint32_t)(a.nW + a.nSph * (m + 1) / G);
+      return r;
+    }
+    // The 27 neighbour cells one by one where their keys are not consecutive (Morton, hashed).
+    // Else as 9 rows along x: cells x-1..x+1 of a row are consecutive keys, so their spheres are
+    // one storage range; across a periodic x boundary the wrapped cell is a second range.
+    const bool rows = KIND == CELL_ROWS;
+    const bool wrap = rows && a.g.periodic && (m & 1);
+    const int row = rows ? (a.g.periodic ? m >> 1 : m) : m / 3;
+    int q[3] = {rows ? 0 : c[0] + m % 3 - 1, c[1] + row % 3 - 1, c[2] + row / 3 - 1};
+    // a cell across a periodic boundary is its image, one period away on this side (every axis
+    // has at least 3 cells, so the 27 are distinct)
+    float sh[3] = {0.f, 0.f, 0.f};
+    bool ok = !wrap || xw >= 0;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      const bool lo = q[d] < 0, hi = q[d] >= nc[d];
+      ok = ok && (!(lo || hi) || a.g.periodic);
+      sh[d] = lo ? -(float)a.g.L[d] : (hi ? (float)a.g.L[d] : 0.f);
+      q[d] += lo ? nc[d] : (hi ? -nc[d] : 0);
+    }
+    if (!ok) return r;
+    uint32_t b0, b1;
+    if (KIND == CELL_HASHED) {
+      b0 = cell_hash(q[0], q[1], q[2], a.g.hmask);
+      // a bucket shared by two of the cells (a hash collision) is walked once, at the first; a
+      // sphere of a far cell in a walked bucket fails the float test
+      for (int m2 = 0; m2 < m; m2++) {
+        const int r0 = c[0] + m2 % 3 - 1, r1 = c[1] + (m2 / 3) % 3 - 1, r2 = c[2] + m2 / 9 - 1;
+        if (r0 < 0 || r1 < 0 || r2 < 0 || r0 >= nc[0] || r1 >= nc[1] || r2 >= nc[2]) continue;
+        if (cell_hash(r0, r1, r2, a.g.hmask) == b0) return r;
+      }
+      b1 = b0;
+    } else if (KIND == CELL_MORTON) {
+      b0 = b1 = morton3(q[0], q[1], q[2]);
     } else {
-      // The 27 neighbour cells as 9 rows along x: cells x-1..x+1 of a row are consecutive keys,
-      // so their spheres are one storage range; across a periodic x boundary the wrapped cell
-      // is a second range, one period away. The 9 ranges are loaded before any candidate.
-      // the sphere's grid: its scene's (keys from the scene's offset), or the one grid
-      uint32_t k = a.key[t], kbase = 0u;
-      int nx = a.g.nc[0], ny = a.g.nc[1], nz = a.g.nc[2];
-      if (a.g.sg) {
-        const SceneGrid& G = a.g.sg[a.scene[s]];
-        kbase = G.off;
-        nx = G.nc[0]; ny = G.nc[1]; nz = G.nc[2];
-        k -= kbase;
-      }
-      const int c0 = (int)(k % (uint32_t)nx), c1 = (int)((k / (uint32_t)nx) % (uint32_t)ny),
-                c2 = (int)(k / ((uint32_t)nx * (uint32_t)ny));
-      const int xlo = c0 > 0 ? c0 - 1 : 0, xhi = c0 + 1 < nx ? c0 + 1 : nx - 1;
-      int xw = -1;
-      float xwsh = 0.f;
-      if (a.g.periodic && c0 == 0) { xw = nx - 1; xwsh = -(float)a.g.L[0]; }
-      if (a.g.periodic && c0 == nx - 1) { xw = 0; xwsh = (float)a.g.L[0]; }
-      // neighbour row m = 3 (dz + 1) + dy + 1: its first cell key, periodic shifts, and whether
-      // it exists; the next row's range is loaded while the current one is walked
-      auto row = [&](int m, uint32_t& rb, float& sy, float& sz) {
-        int q1 = c1 + (m % 3) - 1, q2 = c2 + (m / 3) - 1;
-        bool ok = true;
-        sy = 0.f;
-        sz = 0.f;
-        // a wrapped row lies one period away on this side
-        if (q1 < 0 || q1 >= ny) {
-          ok = ok && a.g.periodic;
-          sy = q1 < 0 ? -(float)a.g.L[1] : (float)a.g.L[1];
-          q1 = (q1 + ny) % ny;
-        }
-        if (q2 < 0 || q2 >= nz) {
-          ok = ok && a.g.periodic;
-          sz = q2 < 0 ? -(float)a.g.L[2] : (float)a.g.L[2];
-          q2 = (q2 + nz) % nz;
-        }
-        rb = kbase + (uint32_t)(((int64_t)q2 * ny + q1) * nx);
-        return ok;
-      };
-      uint32_t nb0 = 0u, nb1 = 0u, rbn;
-      float syn, szn;
-      bool okn = row(0, rbn, syn, szn);
-      if (okn) { nb0 = a.cbeg[rbn + xlo]; nb1 = a.cbeg[rbn + xhi + 1]; }
-      for (int m = 0; m < 9; m++) {
-        const uint32_t t0 = nb0, t1 = nb1, rb = rbn;
-        const float sy = syn, sz = szn;
-        const bool ok = okn;
-        if (m < 8) {
-          okn = row(m + 1, rbn, syn, szn);
-          nb0 = okn ? a.cbeg[rbn + xlo] : 0u;
-          nb1 = okn ? a.cbeg[rbn + xhi + 1] : 0u;
-        }
-        for (uint32_t tt = t0; tt < t1; tt++) consider(tt, 0.f, sy, sz);
-        if (xw >= 0 && ok) {
-          const uint32_t w0 = a.cbeg[rb + xw], w1 = a.cbeg[rb + xw + 1];
-          for (uint32_t tt = w0; tt < w1; tt++) consider(tt, xwsh, sy, sz);
-        }
+      const uint32_t rb = kbase + (uint32_t)(((int64_t)q[2] * nc[1] + q[1]) * nc[0]);
+      b0 = rb + (uint32_t)(wrap ? xw : xlo);
+      b1 = rb + (uint32_t)(wrap ? xw : xhi);
+      sh[0] = wrap ? xwsh : 0.f;
+    }
+    r = Range{a.cbeg[b0], a.cbeg[b1 + 1], sh[0], sh[1], sh[2]};
+    return r;
+  };
+  // One batch of PAIR_B candidates a turn, every lane in its own ranges, the bounds of the next
+  // range loaded while the current one is walked
+  {
+    int m = g * M / G;
+    Range ra = range(m), rb = range(m + 1);
+    uint32_t tt = ra.t0;
+    while (__any(m < m1)) {
+      if (__any(nq > PAIR_Q - PAIR_B)) flush();
+      float4 f[PAIR_B];
+#pragma unroll
+      for (int q = 0; q < PAIR_B; q++) f[q] = a.pf[tt + q < ra.t1 ? (int64_t)(tt + q) : sl];
+#pragma unroll
+      for (int q = 0; q < PAIR_B; q++)
+        if (tt + q < ra.t1) consider(tt + q, f[q], ra.sx, ra.sy, ra.sz);
+      tt += PAIR_B;
+      if (tt >= ra.t1) {
+        m++;
+        ra = rb;
+        tt = ra.t0;
+        rb = range(m + 1);
       }
     }
-    flush();
-    // boundary bodies (storage [0,nW): walls, facets) against every sphere, the body as pA:
-    // AABB overlap (InsertionSortCollider.cpp:67-73) of the body's enlarged AABB and the
-    // sphere's. The AABB of a wall is infinite except along its axis (Wall.cpp:25-38).
-    // batched scenes: the sphere's own scene's bodies; else the workgroup's list
+  }
+  flush();
+  // boundary bodies (storage [0,nW): walls, facets) against every sphere, the body as pA:
+  // AABB overlap (InsertionSortCollider.cpp:67-73) of the body's enlarged AABB and the
+  // sphere's. The AABB of a wall is infinite except along its axis (Wall.cpp:25-38).
+  // batched scenes: the sphere's own scene's bodies; else the workgroup's list; the lanes of a
+  // sphere take them in turn
+  if (a.nW > 0) {
     const bool own = a.sceneBodyOff != nullptr;
-    const int64_t q0 = own ? (int64_t)a.sceneBodyOff[a.scene[s]] : 0;
-    const int64_t q1 = own ? (int64_t)a.sceneBodyOff[a.scene[s] + 1] : (bfull ? a.nW : nb);
-    for (int64_t q = q0; q < q1; q++) {
-      const int64_t w = own ? (int64_t)a.sceneBody[q] : (bfull ? q : (int64_t)blist[q]);
-      const double* b = a.bnd + 6 * w;
-      // the whole wavefront misses this body (uniform branch)
-      if (!own && !(b[0] <= whi[0] && b[3] >= wlo[0] && b[1] <= whi[1] && b[4] >= wlo[1] && b[2] <= whi[2] &&
-                    b[5] >= wlo[2]))
-        continue;
-      if (!(b[0] <= shi[0] && b[3] >= slo[0] && b[1] <= shi[1] && b[4] >= slo[1] && b[2] <= shi[2] &&
-            b[5] >= slo[2]))
-        continue;
-      if (!may_collide(a.mask[w], ms, a.P.loneMask)) continue;
-      if (a.scene && a.scene[w] != a.scene[s]) continue;
-      const uint32_t type = flag_shape(a.flags[w]) == WDG_FACET ? CT_FS : CT_WS;
-      neighbour((uint32_t)w);
-      emit((uint32_t)w, (uint32_t)w, (uint32_t)s, type | CI_NEAR, pack_cd(0, 0, 0), ((uint64_t)a.uid[w] << 32) | us);
+    const double* wb = bbox[wv];  // the wavefront's box
+    double slo[3], shi[3];
+    for (int k = 0; k < 3; k++) sph_bounds(ps[k], a.P.absDf * rs, vds, slo[k], shi[k]);
+    const int64_t q0 = own ? (int64_t)a.sceneBodyOff[scs] : 0;
+    const int64_t q1 = !live ? 0 : (own ? (int64_t)a.sceneBodyOff[scs + 1] : (bfull ? a.nW : nb));
+    for (int64_t q = q0 + g; __any(q < q1); q += G) {
+      bool hit = q < q1;
+      int64_t w = 0;
+      if (hit) {
+        w = own ? (int64_t)a.sceneBody[q] : (bfull ? q : (int64_t)blist[q]);
+        const double* b = a.bnd + 6 * w;
+        hit = own || (b[0] <= wb[3] && b[3] >= wb[0] && b[1] <= wb[4] && b[4] >= wb[1] && b[2] <= wb[5] &&
+                      b[5] >= wb[2]);
+        hit = hit && b[0] <= shi[0] && b[3] >= slo[0] && b[1] <= shi[1] && b[4] >= slo[1] && b[2] <= shi[2] &&
+              b[5] >= slo[2];
+        hit = hit && may_collide(a.mask[w], ms, a.P.loneMask) && (!a.scene || a.scene[w] == scs);
+      }
+      const uint32_t type = hit && flag_shape(a.flags[w]) == WDG_FACET ? CT_FS : CT_WS;
+      emit(hit, true, (uint32_t)w, (uint32_t)w, (uint32_t)s, type | CI_NEAR, pack_cd(0, 0, 0),
+           hit ? (((uint64_t)a.uid[w] << 32) | us) : 0ull);
     }
+  }
+  if (live && g == 0) {
     if (OUT == OUT_COUNT || OUT == OUT_STAGE) a.count[t] = cnt;
     if (OUT == OUT_STAGE) a.deg[t] = ndeg;
   }
@@ -865,6 +903,30 @@ __global__ __launch_bounds__(256) void k_pairs(PairArgs a) {
       a.bmax[2 * blockIdx.x + k] = max(max(wm[0][k], wm[1][k]), max(wm[2][k], wm[3][k]));
     }
   }
+}
+
+// Lanes per sphere: as many as fill the chip's 1,024 SIMDs with a few wavefronts. Measured (us):
+// all pairs of 300 spheres 73 / 46 / 34 / 24 with 1 / 2 / 4 / 8 lanes, 2,000 in cells 46 / 30 / 19 /
+// 15, 20,000: 56 / 35 / 23 / 18, 150,000: 94 / 92 / 85 / 92, 186,000 sparse in 64 scenes 36 / 46 /
+// 59 / 80, 1M: 309 / 328 / 377 / 481 (the passes over queues and cells that more lanes repeat then
+// cost more than the latency they hide).
+static int pair_lanes(int64_t nSph) { return nSph <= 40000 ? 8 : (nSph <= 100000 ? 4 : 1); }
+template <int OUT, int MODE, int G>
+static void launch_pairs_g(Ctx& c, const PairArgs& a) {
+  const dim3 grid(nblocks(a.nSph * G, 256)), block(256);
+  if (a.brute) hipLaunchKernelGGL((k_pairs<OUT, MODE, CELL_NONE, G>), grid, block, 0, c.stream, a);
+  else if (a.g.hashed) hipLaunchKernelGGL((k_pairs<OUT, MODE, CELL_HASHED, G>), grid, block, 0, c.stream, a);
+  else if (a.g.morton) hipLaunchKernelGGL((k_pairs<OUT, MODE, CELL_MORTON, G>), grid, block, 0, c.stream, a);
+  else hipLaunchKernelGGL((k_pairs<OUT, MODE, CELL_ROWS, G>), grid, block, 0, c.stream, a);
+  WDG_LAUNCH_CHECK();
+}
+template <int OUT, int MODE>
+static void launch_pairs(Ctx& c, const PairArgs& a) {
+  // (the passes besides the refresh's own, which are rare, all take 4)
+  const int G = OUT == OUT_STAGE ? pair_lanes(a.nSph) : 4;
+  if (OUT == OUT_STAGE && G == 1) launch_pairs_g<OUT, MODE, OUT == OUT_STAGE ? 1 : 4>(c, a);
+  else if (OUT == OUT_STAGE && G == 8) launch_pairs_g<OUT, MODE, OUT == OUT_STAGE ? 8 : 4>(c, a);
+  else launch_pairs_g<OUT, MODE, 4>(c, a);
 }
 
 // largest of the per-workgroup maxima of k_pairs, one workgroup
@@ -937,6 +999,21 @@ __global__ __launch_bounds__(US_BS) void k_unstage(int64_t nW, int64_t nSph, con
   }
 }
 
+// the slot among the n from g0 whose partner is p (0xFFFFFFFF: none), four read at a time so that
+// the search costs one memory latency for most spheres instead of one per slot
+__device__ __forceinline__ uint32_t find_partner(const uint32_t* __restrict__ B, uint32_t g0, uint32_t n, uint32_t p) {
+  uint32_t slot = 0xFFFFFFFFu;
+  for (uint32_t u = 0; u < n && slot == 0xFFFFFFFFu; u += 4) {
+    uint32_t b[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) b[q] = B[g0 + (u + q < n ? u + q : u)];
+#pragma unroll
+    for (int q = 3; q >= 0; q--)
+      if (u + q < n && b[q] == p) slot = g0 + u + q;
+  }
+  return slot;
+}
+
 struct MergeArgs {
   int64_t nOld, nW, nPairs;
   RealView ov;
@@ -961,14 +1038,14 @@ __global__ void k_merge(MergeArgs a) {
   const uint32_t lo = x < y ? x : y, hi = x < y ? y : x;
   const bool ws = (oi & CI_TYPE_MASK) != CT_SS;
   const uint32_t gen = ws ? hi : lo;  // the generating sphere (boundary bodies come first in storage)
-  const uint32_t g0 = a.off[gen - a.nW], g1 = g0 + a.count[gen - a.nW];
-  for (uint32_t t = g0; t < g1; t++) {
-    if (a.A[t] == lo && a.B[t] == hi) {
-      a.carry[t] = (uint32_t)c + 1u;
-      // the contact keeps the periodic image it was created in
-      if (a.periodic) a.dist[t] = a.oDist[c];
-      return;
-    }
+  // its slots with spheres have it as A and a later sphere as B, those with boundary bodies the
+  // other way round
+  const uint32_t found = find_partner(ws ? a.A : a.B, a.off[gen - a.nW], a.count[gen - a.nW], ws ? lo : hi);
+  if (found != 0xFFFFFFFFu) {
+    a.carry[found] = (uint32_t)c + 1u;
+    // the contact keeps the periodic image it was created in
+    if (a.periodic) a.dist[found] = a.oDist[c];
+    return;
   }
   const uint32_t t = (uint32_t)a.nPairs + atomicAdd(a.nExtra, 1u);
   // roles are fixed by user ids: find where the old pA went
@@ -1283,10 +1360,7 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) void k_adj_sym(AdjArgs a) {
         for (uint32_t v = 0; v < q; v++) r += adj_generated(a, p, sj[w][b0 + v]) ? 1u : 0u;
         slot = a.off[tw + L] + r;
       } else {
-        slot = 0xFFFFFFFFu;
-        const uint32_t g0 = a.off[j - a.nW], g1 = g0 + a.count[j - a.nW];
-        for (uint32_t u = g0; u < g1; u++)
-          if (a.B[u] == p) { slot = u; break; }
+        slot = find_partner(a.B, a.off[j - a.nW], a.count[j - a.nW], p);
         if (slot == 0xFFFFFFFFu) {
           // the pair test disagreed between the two spheres: reported, entry kept in bounds
           atomicOr(&a.dflags[1], ERR_ADJ);
@@ -1774,11 +1848,10 @@ static void refresh(Ctx& c) {
     pa.nbStage = NS;
     pa.sA = c.stPartner.p; pa.sInfo = c.stInfo.p; pa.sDist = c.stDist.p;
     pa.deg = c.sdeg.p; pa.nb = c.stNb.p;
-    const int64_t npb = nblocks(nSph, 256);
+    const int64_t npb = nblocks(nSph * pair_lanes(nSph), 256);
     c.pairMax.ensure(2 * npb);
     pa.bmax = c.pairMax.p;
-    hipLaunchKernelGGL((k_pairs<OUT_STAGE, MODE_NEAR>), dim3(npb), dim3(256), 0, c.stream, pa);
-    WDG_LAUNCH_CHECK();
+    launch_pairs<OUT_STAGE, MODE_NEAR>(c, pa);
     hipLaunchKernelGGL(k_block_max, dim3(1), dim3(1024), 0, c.stream, npb, (const uint32_t*)c.pairMax.p,
                        c.dflags.p + 7);
     WDG_LAUNCH_CHECK();
@@ -1807,7 +1880,7 @@ static void refresh(Ctx& c) {
     } else {
       // a sphere generated more pairs than the staging area holds: generate again, in place
       pa.sA = N.A.p; pa.sB = N.B.p; pa.sInfo = N.info.p; pa.sCarry = N.carry.p; pa.sDist = N.dist.p;
-      hipLaunchKernelGGL((k_pairs<OUT_SLOTS, MODE_NEAR>), dim3(nblocks(nSph, 256)), dim3(256), 0, c.stream, pa);
+      launch_pairs<OUT_SLOTS, MODE_NEAR>(c, pa);
     }
     WDG_LAUNCH_CHECK();
   }
@@ -1993,8 +2066,7 @@ void potential_pairs(Ctx& c, std::vector<uint32_t>& ida, std::vector<uint32_t>& 
   P.periodic = c.field.periodic;
   for (int k = 0; k < 3; k++) P.L[k] = c.field.cell[k];
   PairArgs pa = pair_args(c, g, P);
-  hipLaunchKernelGGL((k_pairs<OUT_COUNT, MODE_AABB>), dim3(nblocks(nSph, 256)), dim3(256), 0, c.stream, pa);
-  WDG_LAUNCH_CHECK();
+  launch_pairs<OUT_COUNT, MODE_AABB>(c, pa);
   scan_exclusive(c, c.scount.p, c.soff.p, nSph, c.dflags.p + 4);
   int64_t np = read_u32(c, c.dflags.p + 4);
   if (np == 0) return;
@@ -2002,8 +2074,7 @@ void potential_pairs(Ctx& c, std::vector<uint32_t>& ida, std::vector<uint32_t>& 
   k.ensure(np);
   d.ensure(np);
   pa.pkey = k.p; pa.pdist = d.p;
-  hipLaunchKernelGGL((k_pairs<OUT_KEYS, MODE_AABB>), dim3(nblocks(nSph, 256)), dim3(256), 0, c.stream, pa);
-  WDG_LAUNCH_CHECK();
+  launch_pairs<OUT_KEYS, MODE_AABB>(c, pa);
   std::vector<uint64_t> hk((size_t)np), hd;
   WDG_HIP(hipMemcpyAsync(hk.data(), k.p, np * 8, hipMemcpyDeviceToHost, c.stream));
   if (c.field.periodic) {
