@@ -98,3 +98,34 @@ def test_pairs_over_lanes_per_sphere(n):
     want = np.sort(p, axis=1)
     assert len(want) > n // 4 or n == 3
     np.testing.assert_array_equal(np.sort(got, axis=1), want[np.lexsort((want[:, 1], want[:, 0]))])
+
+
+@pytest.mark.parametrize("n,flat,steps", [(20, False, 1), (300, False, 7), (300, False, 130), (4900, True, 40)])
+@pytest.mark.parametrize("track", [False, True])
+def test_steps_ahead_equal_engine_calls(n, flat, steps, track):
+    # wdg_run's batches of gated steps against the engines called one by one: short wall lists (summed
+    # in the leapfrog) and a floor with more than 2,048 contacts (cut into parts), several refreshes
+    from tests.scenes import GpuRunner, contact_kw, deposition
+
+    sc = deposition(n=n, seed=n, dense=True, vel_sigma=.3)
+    if flat:  # one layer on the floor, slightly in contact with it
+        m = int(round(n ** .5))
+        r = sc["radius"][0]
+        g = np.stack(np.meshgrid(np.arange(m), np.arange(m), indexing="ij"), -1).reshape(-1, 2)
+        sc["pos"] = np.column_stack([(g + .5) * 2.01 * r, np.full(len(g), .999 * r)])
+        for w in sc["walls"][3:]:
+            w["pos"][w["axis"]] = 2.01 * r * m
+    a, b = GpuRunner(sc), GpuRunner(sc)
+    eng = ["Collider", "ContactLoop", "Leapfrog"]
+    if track:
+        a.d.set_energy_tracking(True)
+        b.d.set_energy_tracking(True)
+    a.run(eng, steps)
+    b.d.run(eng, steps, 0, sc["dt"], contact=contact_kw(sc), leapfrog=dict(damping=sc["damping"]), dynDtPeriod=0)
+    for f in ("pos", "vel", "angVel", "ori", "force", "torque"):
+        np.testing.assert_array_equal(a.d.get(f), b.d.get(f), err_msg=f)
+    np.testing.assert_array_equal(a.d.contacts(data=False)[0], b.d.contacts(data=False)[0])
+    sa, sb = a.d.stats(), b.d.stats()
+    assert sa["nSteps"] == sb["nSteps"] and sa["nRefresh"] == sb["nRefresh"]
+    if flat:
+        assert sa["nCandidates"] > 2 * 2048

@@ -517,6 +517,8 @@ int wdg_ctx_create(int device, wdg_ctx** out) {
     ctx->c.dflags.ensure(64);
     WDG_HIP(hipMemset(ctx->c.dflags.p, 0, 64 * sizeof(uint32_t)));
     WDG_HIP(hipHostMalloc((void**)&ctx->c.hflags, 64 * sizeof(uint32_t), hipHostMallocDefault));
+    std::memset(ctx->c.hflags, 0, 64 * sizeof(uint32_t));
+    WDG_HIP(hipHostGetDevicePointer((void**)&ctx->c.hflagsDev, ctx->c.hflags, 0));
     ctx->c.red.ensure(64);
     // the device's copy of the no-allocation entry points' scratch array
     scratch_setup(device);
@@ -555,7 +557,7 @@ int wdg_ctx_destroy(wdg_ctx* ctx) {
     c.adjEnt.release(); c.adjDeg.release(); c.stNb.release(); c.sdeg.release(); c.posf.release();
     c.fgeo.release(); c.bnd.release(); c.pairMax.release(); c.scene.release(); c.dtScene.release();
     c.sceneBodyOff.release(); c.sceneBody.release();
-    c.fnode.release(); c.gbody.release(); c.bndPart.release(); c.vdScene.release(); c.sceneVmax.release();
+    c.fnode.release(); c.gbody.release(); c.gbodyOf.release(); c.bndPart.release(); c.vdScene.release(); c.sceneVmax.release();
     c.sceneBox.release(); c.sgrid.release();
     c.gstate.release();
     if (c.graph.exec) (void)hipGraphExecDestroy(c.graph.exec);
@@ -716,6 +718,10 @@ int wdg_upload_particles(wdg_ctx* ctx, const wdg_particles* p) {
       c.nGBody = (int64_t)gb.size();
       c.gbodyHost = gb;
       c.gbody.ensure(gb.size() + 1);
+      std::vector<uint32_t> of((size_t)nW + 1, NO_STATE);
+      for (size_t k = 0; k < gb.size(); k++) of[gb[k]] = (uint32_t)k;
+      c.gbodyOf.ensure(of.size());
+      WDG_HIP(hipMemcpy(c.gbodyOf.p, of.data(), of.size() * 4, hipMemcpyHostToDevice));
       if (!gb.empty()) WDG_HIP(hipMemcpy(c.gbody.p, gb.data(), gb.size() * 4, hipMemcpyHostToDevice));
       c.bndPart.ensure((size_t)64 * 6 * (gb.size() + 1));
       c.bndParts = 1;
@@ -1074,6 +1080,10 @@ int wdg_run(wdg_ctx* ctx, const wdg_program* prog, int64_t nSteps, int64_t* step
   }
   return guard(ctx, [&] {
     Ctx& c = ctx->c;
+    if (can_run_ahead(c, prog)) {
+      run_ahead(c, prog, nSteps, step, dt);
+      return;
+    }
     std::vector<double> crs, nextScene;
     for (int64_t s = 0; s < nSteps; s++) {
       double nextDt = NAN;

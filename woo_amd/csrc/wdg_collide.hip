@@ -2026,7 +2026,12 @@ void collide(Ctx& c, const wdg_collide_params* p) {
       c.dirtyIdx = 0;
       fresh = false;
     }
-    if (!fresh) {
+    if (!fresh && c.hostWords && c.dirtyIdx >= DIRTY_PP) {
+      // the leapfrog wrote its own answer to the pinned words
+      WDG_HIP(hipStreamSynchronize(c.stream));
+      c.hflags[1] = c.hflags[HOST_ERR];
+      c.hflags[c.dirtyIdx] = c.hflags[HOST_DIRTY] == c.lfNumber ? 1u : 0u;
+    } else if (!fresh) {
       WDG_HIP(hipMemcpyAsync(c.hflags, c.dflags.p, (DIRTY_PP + 2) * sizeof(uint32_t), hipMemcpyDeviceToHost,
                              c.stream));
       WDG_HIP(hipStreamSynchronize(c.stream));

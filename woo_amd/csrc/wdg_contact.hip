@@ -53,9 +53,13 @@ struct ContactArgs {
   // batched scenes: dt of each particle's scene (else null, dt above)
   const double* dtScene;
   const uint32_t* scene;
-  // graph replay: a set stop word skips the kernel; the step's renorm flag from the device
+  // gated steps (wdg_graph.hip): a set stop word skips the kernel; the step's renorm flag from the
+  // device; the filter decides whether the step runs (gs: all the words, dirtyPrev: the word that
+  // the previous step's leapfrog set)
   const uint32_t* gstop;
   const uint32_t* renormPtr;
+  uint32_t* gs;
+  const uint32_t* dirtyPrev;
   int cfBlocks;  // workgroups per group of slots in the force kernel
   // parameters
   double L[3];
@@ -310,9 +314,29 @@ __device__ __forceinline__ bool filter_slot(const ContactArgs& a, int64_t c, Slo
   return keep;
 }
 
+// Whether a gated step is skipped, decided by its first kernel: once a step was skipped, or when
+// the step before it (not the host's collider call, before the batch's first step) left a particle
+// outside its Verlet skin or raised an error. Every workgroup comes to the same answer from words
+// that no other of them writes differently; the first one makes it stick for the kernels and steps
+// after it and sets the step's trsfRenorm flag. The leapfrog counts the step when it ran.
+__device__ __forceinline__ bool step_skipped(const ContactArgs& a) {
+  if (!a.gs) return false;
+  const bool skip = a.gs[0] != 0u || (a.gs[6] == 0u && (*a.dirtyPrev != 0u || a.dflags[1] != 0u));
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (skip) {
+      a.gs[0] = 1u;
+    } else {
+      const int64_t step = (int64_t)(((uint64_t)a.gs[4] << 32) | a.gs[3]) + a.gs[1];
+      const int64_t tr = (int64_t)a.gs[5];
+      a.gs[2] = (tr > 0 && (step % tr) == 0) ? 1u : 0u;
+    }
+  }
+  return skip;
+}
+
 template <bool PERIODIC, int LAW>
 __global__ __launch_bounds__(GROUP_BS) void k_cfilter(ContactArgs a) {
-  if (a.gstop && *a.gstop) return;
+  if (step_skipped(a)) return;
   const uint32_t g = xcd_block(blockIdx.x, gridDim.x);
   const int64_t base = (int64_t)g * GROUP;
   // all slots of the thread first (their loads overlap), then the bookkeeping passes
@@ -736,7 +760,7 @@ __device__ __forceinline__ bool filter_slot32(const ContactArgs& a, int64_t c, S
 
 template <bool PERIODIC, int LAW>
 __global__ __launch_bounds__(GROUP_BS) void k_cfilter32(ContactArgs a) {
-  if (a.gstop && *a.gstop) return;
+  if (step_skipped(a)) return;
   const uint32_t g = xcd_block(blockIdx.x, gridDim.x);
   const int64_t base = (int64_t)g * GROUP;
   constexpr int NP = GROUP / GROUP_BS;
@@ -1028,9 +1052,11 @@ static ContactArgs contact_args(Ctx& c, int from, int to) {
   a.dtScene = c.nScenes > 0 ? c.dtScene.p : nullptr;
   a.scene = c.scene.p;
   a.cfBlocks = c.tune.cfBlocks;
-  if (c.graphCapture) {
+  if (c.gated) {
     a.gstop = c.gstate.p;
     a.renormPtr = c.gstate.p + 2;
+    a.gs = c.gstate.p;
+    a.dirtyPrev = c.dflags.p + DIRTY_PP + (1 - c.lfParity);
   }
   for (int k = 0; k < 3; k++) a.L[k] = c.field.cell[k];
   a.absDf = std::fabs(c.field.distFactor);
@@ -1236,6 +1262,7 @@ void contact_loop(Ctx& c, const wdg_contact_params* p) {
                                      (std::sqrt(std::log(p->en) * std::log(p->en) + M_PI * M_PI))
                                : 0.;
   c.stepNow = p->step;
+  c.hostWords = false;  // error bits of this loop are read again
   c.lastPhysKind = p->physKind;
   c.lastPoisson = p->poisson;
   c.lastEn = p->en;
@@ -1324,7 +1351,7 @@ void contact_loop(Ctx& c, const wdg_contact_params* p) {
     WDG_LAUNCH_CHECK();
     const double vol = c.field.cell[0] * c.field.cell[1] * c.field.cell[2];
     hipLaunchKernelGGL(k_cl_stress_sum, dim3(1), dim3(256), 0, c.stream, ng, (const double*)c.clPart.p, vol,
-                       c.graphCapture ? (const uint32_t*)c.gstate.p : nullptr, c.clStress.p);
+                       c.gated ? (const uint32_t*)c.gstate.p : nullptr, c.clStress.p);
     WDG_LAUNCH_CHECK();
   }
   c.R[to].sidxValid = true;
@@ -1335,7 +1362,7 @@ void contact_loop(Ctx& c, const wdg_contact_params* p) {
   if (energy_per_scene(c)) energy_scenes_contacts(c);
   c.forcesPending = p->applyForces != 0;
   // ContactLoop::run's epilogue (ContactLoop.cpp:265-266): 'once' updates one step only
-  if (c.updatePhys == 2 && !c.graphCapture) c.updatePhys = 0;
+  if (c.updatePhys == 2 && !c.gated) c.updatePhys = 0;
 }
 
 // ------------------------------------------------------------------ real set from per-slot flags

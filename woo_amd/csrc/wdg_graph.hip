@@ -1,14 +1,19 @@
-// Graph replay of the step loop and its autotuner.
+// The step loop ahead of the host's checks: graph replay with its autotuner, and plain launches.
 //
 // The engine list [Collider, ContactLoop, Leapfrog(reset)] runs as: the collider on the
 // host (its dirty test reads one flag word, a rebuild sizes buffers), then K steps of contact
-// loop and leapfrog captured once as a hipGraph and replayed. Before step j > 0 of a replay a
-// one-thread kernel reads the dirty word the leapfrog of step j-1 set: when a particle left
-// its Verlet skin it sets the stop word, and every captured kernel after it returns at once,
-// so the replay ends after step j-1 and the host rebuilds before the next step, exactly as
-// Scene::doOneStep would. The same kernel counts the executed steps and sets the step's
-// trsfRenorm flag from the device-resident step number. Host bookkeeping (which state
-// buffer is current, the parity of the dirty words) advances by the executed count.
+// loop and leapfrog captured once as a hipGraph and replayed, or launched one after the other
+// (wdg_run). The first kernel of step j > 0 (the contact filter; k_gate when there are no slots)
+// reads the dirty word the leapfrog of step j-1 set: when a particle left its Verlet skin, or an
+// error was raised, it sets the stop word, and every kernel after it returns at once, so the
+// batch ends after step j-1 and the host rebuilds before the next step, exactly as
+// Scene::doOneStep would. It also sets the step's trsfRenorm flag from the device-resident step
+// number, and the step's leapfrog counts it. Host bookkeeping (which state buffer is current,
+// the parity of the dirty words) advances by the executed count.
+//
+// Small scenes are bound by launches and the host's round trips: 2,000 spheres between walls took
+// 57 us a step with a round trip and five launches, 40 us (refreshes included) with three and a round
+// trip per batch.
 //
 // A graph is valid while the slot list, the buffers and the parameters it captured stay the
 // same: it is captured again after a rebuild or any change of state layout (Ctx::gen), of
@@ -18,6 +23,7 @@
 // The autotuner times candidate tunings (workgroups per contact group in the force kernel,
 // steps per graph) on the live state: each trial is a run of real steps, timed by the host
 // clock around whole replays, the best kept.
+#include <algorithm>
 #include <chrono>
 
 #include "wdg_internal.hpp"
@@ -28,12 +34,14 @@ namespace wdg {
 // the batch's first step (int64), [5] trsfRenorm, [6] set until the batch's first step starts.
 // A batch is several replays launched back to back: once a gate has stopped, every later kernel
 // of the batch returns at once, so the replays after the stop cost only their launches.
-// dirtyWord: the word the previous step's leapfrog sets (its parity is fixed at capture; K is even)
+// The gate of a step without slots, which has no filter (step_skipped in wdg_contact.hip and the
+// leapfrog do the same in the others). dirtyWord: the word the previous step's leapfrog sets (its
+// parity is fixed at capture; K is even)
 __global__ void k_gate(uint32_t* gs, const uint32_t* dflags, int dirtyWord) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   if (gs[0]) return;
   // the batch's first step follows the host's collider call, which has rebuilt if needed
-  if (!gs[6] && dflags[dirtyWord]) {
+  if (!gs[6] && (dflags[dirtyWord] || dflags[1])) {
     gs[0] = 1u;
     return;
   }
@@ -57,6 +65,11 @@ static void check_program(const wdg_program* prog) {
 }
 
 static void plain_step(Ctx& c, const wdg_program* prog, int64_t step, double dt) {
+  if (c.gated && c.con().n == 0) {
+    hipLaunchKernelGGL(k_gate, dim3(1), dim3(64), 0, c.stream, c.gstate.p, (const uint32_t*)c.dflags.p,
+                       DIRTY_PP + (1 - c.lfParity));
+    WDG_LAUNCH_CHECK();
+  }
   wdg_contact_params cp = prog->contact;
   cp.step = step;
   cp.dt = dt;
@@ -86,13 +99,9 @@ static void restore(Ctx& c, const HostState& h) {
   c.eidxClean = h.eidxClean;
 }
 
-static void capture(Ctx& c, const wdg_program* prog, int K, int64_t step, double dt) {
-  auto& G = c.graph;
-  if (G.exec) {
-    WDG_HIP(hipGraphExecDestroy(G.exec));
-    G.exec = nullptr;
-  }
-  // every buffer a captured launch touches is sized now (no allocation while capturing)
+// every buffer a gated launch touches is sized before the first (no allocation while capturing,
+// and none that would wait for the steps launched ahead)
+static void size_buffers(Ctx& c, const wdg_program* prog) {
   const int64_t nc = c.con().n;
   c.R[0].ensure(nc);
   c.R[1].ensure(nc);
@@ -106,26 +115,29 @@ static void capture(Ctx& c, const wdg_program* prog, int K, int64_t step, double
   if (c.trackEnergy)
     c.enPart.ensure(std::max<size_t>((size_t)4 * ngroups(nc) * c.tune.cfBlocks, (size_t)3 * nblocks(c.n, 256)));
   if (energy_per_scene(c)) energy_scenes_prepare(c, nc);
+}
+
+static void capture(Ctx& c, const wdg_program* prog, int K, int64_t step, double dt) {
+  auto& G = c.graph;
+  if (G.exec) {
+    WDG_HIP(hipGraphExecDestroy(G.exec));
+    G.exec = nullptr;
+  }
+  size_buffers(c, prog);
   const HostState h = save(c);
   hipGraph_t graph = nullptr;
-  c.graphCapture = true;
+  c.gated = true;
   WDG_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
   try {
-    for (int j = 0; j < K; j++) {
-      // the dirty word the previous step's leapfrog sets
-      const int prevWord = DIRTY_PP + (1 - c.lfParity);
-      hipLaunchKernelGGL(k_gate, dim3(1), dim3(64), 0, c.stream, c.gstate.p, (const uint32_t*)c.dflags.p, prevWord);
-      WDG_LAUNCH_CHECK();
-      plain_step(c, prog, step + j, dt);
-    }
+    for (int j = 0; j < K; j++) plain_step(c, prog, step + j, dt);
   } catch (...) {
-    c.graphCapture = false;
+    c.gated = false;
     (void)hipStreamEndCapture(c.stream, &graph);
     if (graph) (void)hipGraphDestroy(graph);
     restore(c, h);
     throw;
   }
-  c.graphCapture = false;
+  c.gated = false;
   WDG_HIP(hipStreamEndCapture(c.stream, &graph));
   WDG_HIP(hipGraphInstantiate(&G.exec, graph, nullptr, nullptr, 0));
   WDG_HIP(hipGraphDestroy(graph));
@@ -160,20 +172,39 @@ static bool graph_valid(const Ctx& c, const wdg_program* prog, int K, double dt)
          a.relRollStiff == b.relRollStiff && a.relTwistStiff == b.relTwistStiff && a.rollTanPhi == b.rollTanPhi;
 }
 
-// one batch of R replays of the K-step graph (up to R*K steps); returns the steps executed. The
-// executed count and the dirty/error words come back in one round trip, and the collider call
-// that follows uses them without reading again.
-static int replay(Ctx& c, const wdg_program* prog, int K, int R, int64_t step, double dt) {
-  // the captured filters keep the per-entry state indices of a clean or current array
+// One batch of up to n steps: R replays of the K-step graph (K > 0), or n steps launched here;
+// returns the steps executed. The executed count and the dirty/error words come back in one round
+// trip, and the collider call that follows uses them without reading again.
+static int batch(Ctx& c, const wdg_program* prog, int K, int n, int64_t step, double dt) {
+  // the filters keep the per-entry state indices of a clean or current array
   if (!c.eidxValid && !c.eidxClean && c.con().n > 0) {
     eidx_clear(c);
     c.eidxClean = true;
   }
-  if (!graph_valid(c, prog, K, dt)) capture(c, prog, K, step, dt);
+  if (K > 0) {
+    if (!graph_valid(c, prog, K, dt)) capture(c, prog, K, step, dt);
+  } else {
+    size_buffers(c, prog);
+  }
   uint32_t w[7] = {0u, 0u, 0u, (uint32_t)((uint64_t)step & 0xFFFFFFFFu), (uint32_t)((uint64_t)step >> 32),
                    (uint32_t)std::max(prog->contact.trsfRenorm, 0), 1u};
   WDG_HIP(hipMemcpyAsync(c.gstate.p, w, sizeof(w), hipMemcpyHostToDevice, c.stream));
-  for (int r = 0; r < R; r++) WDG_HIP(hipGraphLaunch(c.graph.exec, c.stream));
+  if (K > 0) {
+    for (int r = 0; r < n / K; r++) WDG_HIP(hipGraphLaunch(c.graph.exec, c.stream));
+  } else {
+    const HostState h = save(c);
+    c.gated = true;
+    try {
+      for (int j = 0; j < n; j++) plain_step(c, prog, step + j, dt);
+    } catch (...) {
+      c.gated = false;
+      (void)hipStreamSynchronize(c.stream);
+      restore(c, h);
+      throw;
+    }
+    c.gated = false;
+    restore(c, h);
+  }
   WDG_HIP(hipMemcpyAsync(c.hflags + 32, c.gstate.p + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream));
   WDG_HIP(hipMemcpyAsync(c.hflags, c.dflags.p, (DIRTY_PP + 2) * sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream));
   WDG_HIP(hipStreamSynchronize(c.stream));
@@ -194,65 +225,85 @@ static int replay(Ctx& c, const wdg_program* prog, int K, int R, int64_t step, d
     c.lfParity = (c.lfParity + e) & 1;
     c.dirtyIdx = DIRTY_PP + lastParity;
     c.dirtyKnown = true;
+    c.hostWords = false;
     c.forcesPending = false;
     c.forceClean = true;
   }
   return e;
 }
 
-static void run_graph_steps(Ctx& c, const wdg_program* prog, int64_t nSteps, int64_t* step, double* dt) {
-  check_program(prog);
+// K > 0: replays of a K-step graph; 0: steps launched ahead
+static void run_gated(Ctx& c, const wdg_program* prog, int K, int64_t nSteps, int64_t* step, double* dt) {
   c.gstate.ensure(16);
   int64_t done = 0;
-  const int K = c.tune.graphSteps;
   while (done < nSteps) {
     const int64_t nr = c.nRefresh;
     collide(c, &prog->collide);
     if (c.nRefresh != nr) {
       // the run's refresh interval, a running mean over the last few refreshes
-      if (c.lastRefreshStep >= 0) {
-        const double iv = (double)(*step - c.lastRefreshStep);
-        c.refreshEvery = c.refreshEvery > 0 ? 0.75 * c.refreshEvery + 0.25 * iv : iv;
-      }
-      c.lastRefreshStep = *step;
+      const double iv = (double)c.sinceRefresh;
+      if (iv > 0) c.refreshEvery = c.refreshEvery > 0 ? 0.75 * c.refreshEvery + 0.25 * iv : iv;
+      c.sinceRefresh = 0;
     }
-    // a replay starts from a state its capture saw: forces at their reset value, the
+    // a batch starts from a state its capture saw: forces at their reset value, the
     // contact loop's forces gathered; otherwise one plain step
     const int64_t left = nSteps - done;
     // (a periodic scene's step 0 is a plain one when tracking energy: its leapfrog adds no terms,
     // and a graph captured there would skip them at every replay)
     // (updatePhys 'once' is one plain step, after which the loop reads 'never')
-    if (!c.forceClean || c.forcesPending || left < K || c.n == 0 || c.updatePhys == 2 ||
-        (c.trackEnergy && c.field.periodic && *step == 0)) {
+    if (!c.forceClean || c.forcesPending || left < std::max(K, 1) || c.n == 0 || c.updatePhys == 2 ||
+        !(c.verletDist > 0) || (c.trackEnergy && c.field.periodic && *step == 0)) {
+      if (c.trackEnergy && K == 0) energy_step_begin(c);
       plain_step(c, prog, *step, *dt);
       *step += 1;
       done += 1;
+      c.sinceRefresh += 1;
       continue;
     }
-    // replays per batch: up to the next refresh the run's own refresh interval predicts (a
-    // batch that reaches a refresh earlier wastes only the launches of its remaining replays)
-    int R = 1;
-    if (c.refreshEvery > 0) {
-      const double toRefresh = c.refreshEvery - (double)(*step - c.lastRefreshStep);
-      R = (int)std::max(1., std::floor(toRefresh / K));
-    }
-    R = (int)std::min<int64_t>(std::min<int64_t>(R, left / K), 64);
-    const int e = replay(c, prog, K, R, *step, *dt);
-    if (e == 0) throw Error(WDG_E_STATE, "graph replay executed no step");
+    // steps per batch: up to the next refresh the run's own refresh interval predicts (a batch
+    // that reaches a refresh earlier wastes only the launches of its remaining steps; four steps
+    // at a time once the refresh is due)
+    const int u = std::max(K, 1);
+    const double to = c.refreshEvery > 0 ? c.refreshEvery - (double)c.sinceRefresh : 8.;
+    int64_t n = std::max<int64_t>((int64_t)std::floor(to / u), K > 0 ? 1 : 4) * u;
+    n = std::min<int64_t>(std::min<int64_t>(n, left / u * u), 64 * u);
+    const int e = batch(c, prog, K, (int)n, *step, *dt);
+    if (e == 0) throw Error(WDG_E_STATE, "a batch of steps executed none");
+    // a plain loop calls the collider once a step
+    if (K == 0) c.nCollide += e - 1;
     *step += e;
     done += e;
+    c.sinceRefresh += e;
   }
 }
 
-void run_graph(Ctx& c, const wdg_program* prog, int64_t nSteps, int64_t* step, double* dt) {
+static void run_guarded(Ctx& c, const wdg_program* prog, int K, int64_t nSteps, int64_t* step, double* dt) {
   // the host mirror of the flag words serves only the collider call right after a batch
   try {
-    run_graph_steps(c, prog, nSteps, step, dt);
+    run_gated(c, prog, K, nSteps, step, dt);
   } catch (...) {
     c.hflagsFresh = false;
     throw;
   }
   c.hflagsFresh = false;
+}
+
+void run_graph(Ctx& c, const wdg_program* prog, int64_t nSteps, int64_t* step, double* dt) {
+  check_program(prog);
+  run_guarded(c, prog, c.tune.graphSteps, nSteps, step, dt);
+}
+
+// The lists a batch can run, stepped as the plain loop steps them: a collider that rebuilds when a
+// particle leaves its skin only, and a leapfrog that resets
+bool can_run_ahead(const Ctx& c, const wdg_program* prog) {
+  const int n = prog->nEngines;
+  return (n == 3 || n == 4) && prog->engines[0] == WDG_E_COLLIDER && prog->engines[1] == WDG_E_CONTACTLOOP &&
+         (n == 3 || prog->engines[2] == WDG_E_INTRAFORCE) && prog->engines[n - 1] == WDG_E_LEAPFROG &&
+         prog->leapfrog.reset && !prog->collide.forceInit && c.n > 0;
+}
+
+void run_ahead(Ctx& c, const wdg_program* prog, int64_t nSteps, int64_t* step, double* dt) {
+  run_guarded(c, prog, 0, nSteps, step, dt);
 }
 
 // ------------------------------------------------------------------ autotuner

@@ -129,14 +129,26 @@ __device__ __forceinline__ void gather_all(const GatherArgs& g, int64_t i, d3 po
   for (uint32_t k = k0; k < k1; k++) gather_one<PERIODIC, F32>(g, g.adj[k], pos, F, T);
 }
 
+// one adjacency entry, through the per-entry real slots when they are kept
+template <bool PERIODIC, bool F32>
+__device__ __forceinline__ void gather_entry(const GatherArgs& g, uint32_t k, d3 pos, d3& F, d3& T) {
+  if (g.eidx && g.sidx) {
+    const uint32_t v = g.eidx[k];
+    if (v != NO_STATE) gather_record<PERIODIC, F32>(g, g.sidx[v & ~EIDX_PA], (v & EIDX_PA) != 0u, pos, F, T);
+  } else {
+    gather_one<PERIODIC, F32>(g, g.adj[k], pos, F, T);
+  }
+}
+
 // Contact forces on the boundary bodies other than facets (storage [0, nW), listed in
 // gbody), which may touch up to every sphere (a floor under a spread pile): each body's list is
 // cut into `parts` equal parts (set at each refresh from the largest such list), one workgroup
-// each, whose threads sum every 256th entry of their part in order, then a fixed-order tree;
-// k_gather_bnd_sum adds the parts in order to the value in the force arrays (which always hold
-// the current force: the reset value, or the gathered one). The spheres' gathers (k_gather,
-// k_leapfrog) skip these bodies. Deterministic; the summation order differs from the
-// sequential one, by rounding.
+// each, whose threads sum every 256th entry of their part in order, then a fixed-order tree; the
+// parts are added in order to the value in the force arrays (which always hold the current force:
+// the reset value, or the gathered one), by the leapfrog or by k_gather_bnd_sum. A single part
+// (lists of up to 2,048 entries) is summed by a workgroup of the leapfrog itself. The spheres'
+// gathers (k_gather, k_leapfrog) skip these bodies. Deterministic; the summation order differs
+// from the sequential one, by rounding.
 constexpr int BND_PARTS_MAX = 64;
 template <bool PERIODIC, bool F32>
 __global__ __launch_bounds__(256) void k_gather_bnd(GatherArgs g, const uint32_t* __restrict__ gbody, int parts,
@@ -151,7 +163,7 @@ __global__ __launch_bounds__(256) void k_gather_bnd(GatherArgs g, const uint32_t
   const uint32_t a0 = k0 + (uint32_t)p * chunk, a1 = a0 + chunk < k1 ? a0 + chunk : k1;
   const d3 pos = mk3(px[i], py[i], pz[i]);
   d3 F = mk3(0., 0., 0.), T = mk3(0., 0., 0.);
-  for (uint32_t k = a0 + threadIdx.x; k < a1; k += blockDim.x) gather_one<PERIODIC, F32>(g, g.adj[k], pos, F, T);
+  for (uint32_t k = a0 + threadIdx.x; k < a1; k += blockDim.x) gather_entry<PERIODIC, F32>(g, k, pos, F, T);
   double v[6] = {F.x, F.y, F.z, T.x, T.y, T.z};
   block_sum_store<6, 256>(v, part + ((int64_t)b * parts + p) * 6);
 }
@@ -205,7 +217,18 @@ struct LeapArgs {
   uint32_t* dirtyNext;  // cleared for the next launch
   const double* dtScene;  // batched scenes: dt of each particle's scene (else null, dt above)
   const uint32_t* scene;
-  const uint32_t* gstop;  // graph replay: a set stop word skips the kernel
+  // the boundary bodies whose contact forces are gathered: the partial sums of k_gather_bnd (parts
+  // of them each, none when foldBodies), each body's index among them; the last foldBodies
+  // workgroups gather one of them each
+  const double* part;
+  const uint32_t *gbody, *gbodyOf;
+  int parts;
+  uint32_t foldBodies;
+  uint32_t* gs;           // gated steps: the words to count the step in, else null
+  uint32_t* host;         // words of the pinned host mirror, else null
+  uint32_t number;        // of this launch, for them
+  const uint32_t* err;
+  const uint32_t* gstop;  // gated steps: a set stop word skips the kernel
   double* enPart;         // energy tracking: kinetic, grav, nonviscDamp partials per workgroup
   double* enP;            // energy tracking per scene: the three terms of each particle, else null
 };
@@ -218,14 +241,32 @@ __device__ __forceinline__ double max_cmp(double x, double y) { return x < y ? y
 template <bool PERIODIC, bool F32, bool ENERGY>
 __global__ __launch_bounds__(256) void k_leapfrog(LeapArgs a, GatherArgs g) {
   if (a.gstop && *a.gstop) return;
-  const int64_t i = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const uint32_t nPart = gridDim.x - a.foldBodies;
+  int64_t i = (int64_t)xcd_block(blockIdx.x, nPart) * blockDim.x + threadIdx.x;
   bool dirty = false;
   double en[3] = {0., 0., 0.};
+  __shared__ double bsum[6];
+  if (!ENERGY && a.foldBodies) {
+    if (blockIdx.x >= nPart) {
+      // one boundary body: its contact forces by the whole workgroup, then it is its first thread's
+      const int64_t b = a.gbody[blockIdx.x - nPart];
+      const uint32_t k0 = g.adjOff[b], k1 = g.adjOff[b + 1];
+      const d3 pos = mk3(a.px[b], a.py[b], a.pz[b]);
+      d3 F = mk3(0., 0., 0.), T = mk3(0., 0., 0.);
+      for (uint32_t k = k0 + threadIdx.x; k < k1; k += blockDim.x) gather_entry<PERIODIC, F32>(g, k, pos, F, T);
+      double v[6] = {F.x, F.y, F.z, T.x, T.y, T.z};
+      block_sum_store<6, 256>(v, bsum);
+      __syncthreads();
+      i = threadIdx.x == 0 ? b : a.n;
+    } else if (i < g.nW && a.gbodyOf[i] != NO_STATE) {
+      i = a.n;
+    }
+  }
   if (i < a.n) {
     const uint32_t fl = a.flags[i];
     const bool integrated = (fl & F_INTEGRATED) != 0u;
     const bool grav = a.hasGravity && !(fl & F_GRAVITY_SKIP);
-    // a boundary body's contact forces were summed into its arrays by k_gather_bnd
+    // a boundary body (facets take no force from the contact loop)
     const bool pre = a.gather && i < g.nW;
     d3 pos = mk3(a.px[i], a.py[i], a.pz[i]);
     d3 F, T;
@@ -239,8 +280,23 @@ __global__ __launch_bounds__(256) void k_leapfrog(LeapArgs a, GatherArgs g) {
       T = mk3(a.tx[i], a.ty[i], a.tz[i]);
     }
     if (a.gather && !pre) gather_all<PERIODIC, F32>(g, i, pos, F, T);
+    const uint32_t body = pre ? a.gbodyOf[i] : NO_STATE;
+    if (pre && body != NO_STATE && g.adjOff[i] != g.adjOff[i + 1]) {
+      double v[6] = {0., 0., 0., 0., 0., 0.};
+      if (!ENERGY && a.foldBodies) {
+#pragma unroll
+        for (int q = 0; q < 6; q++) v[q] += bsum[q];
+      } else {
+#pragma unroll 4
+        for (int p = 0; p < a.parts; p++)
+#pragma unroll
+          for (int q = 0; q < 6; q++) v[q] += a.part[((int64_t)body * a.parts + p) * 6 + q];
+      }
+      F = add3(F, mk3(v[0], v[1], v[2]));
+      T = add3(T, mk3(v[3], v[4], v[5]));
+    }
     if (!integrated) {
-      if (a.gather && !pre) {
+      if (a.gather && (!pre || body != NO_STATE)) {
         a.fx[i] = F.x; a.fy[i] = F.y; a.fz[i] = F.z;
         a.tx[i] = T.x; a.ty[i] = T.y; a.tz[i] = T.z;
       }
@@ -350,8 +406,18 @@ __global__ __launch_bounds__(256) void k_leapfrog(LeapArgs a, GatherArgs g) {
       a.qw[i] = ori.w / qn; a.qx[i] = ori.x / qn; a.qy[i] = ori.y / qn; a.qz[i] = ori.z / qn;
     }
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) *a.dirtyNext = 0u;
-  if (__ballot(dirty) != 0ull && (threadIdx.x & 63) == 0) atomicOr(a.dirty, 1u);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *a.dirtyNext = 0u;
+    if (a.gs) {
+      a.gs[1] += 1u;
+      a.gs[6] = 0u;
+    }
+    if (a.host) a.host[HOST_ERR] = *a.err;
+  }
+  if (__ballot(dirty) != 0ull && (threadIdx.x & 63) == 0) {
+    atomicOr(a.dirty, 1u);
+    if (a.host) a.host[HOST_DIRTY] = a.number;
+  }
   if (ENERGY && a.enP) {
     if (i < a.n) {
       double* e = a.enP + 3 * i;
@@ -493,20 +559,23 @@ static GatherArgs gather_args(Ctx& c) {
   g.sidx = c.reals().sidxValid ? c.reals().sidx.p : nullptr;
   g.eidx = c.eidxValid ? C.eidx.p : nullptr;
   g.nW = c.nW;
-  if (c.graphCapture) g.gstop = c.gstate.p;
+  if (c.gated) g.gstop = c.gstate.p;
   for (int k = 0; k < 3; k++) g.L[k] = c.field.cell[k];
   return g;
 }
 
-static void gather_boundary(Ctx& c, const GatherArgs& g) {
+static int boundary_parts(const Ctx& c) { return std::min(std::max(c.bndParts, 1), BND_PARTS_MAX); }
+// sum: also added to the force arrays (else by the leapfrog)
+static void gather_boundary(Ctx& c, const GatherArgs& g, bool sum) {
   const int64_t nb = c.nGBody;
   if (nb == 0) return;
-  const int parts = std::min(std::max(c.bndParts, 1), BND_PARTS_MAX);
+  const int parts = boundary_parts(c);
   auto* kern = c.precision == 32 ? k_gather_bnd<false, true>
                                  : (c.field.periodic ? k_gather_bnd<true, false> : k_gather_bnd<false, false>);
   hipLaunchKernelGGL(kern, dim3((unsigned)(nb * parts)), dim3(256), 0, c.stream, g, (const uint32_t*)c.gbody.p, parts,
                      c.bndPart.p, (const double*)c.pos[0].p, (const double*)c.pos[1].p, (const double*)c.pos[2].p);
   WDG_LAUNCH_CHECK();
+  if (!sum) return;
   hipLaunchKernelGGL(k_gather_bnd_sum, dim3(nblocks(nb, 64)), dim3(64), 0, c.stream, nb, (const uint32_t*)c.gbody.p,
                      parts, g.adjOff, g.gstop, (const double*)c.bndPart.p, c.force[0].p, c.force[1].p, c.force[2].p,
                      c.torque[0].p, c.torque[1].p, c.torque[2].p);
@@ -530,7 +599,7 @@ void flush_forces(Ctx& c) {
   c.forceClean = false;
   if (c.con().n == 0 || c.n == 0) return;
   GatherArgs g = gather_args(c);
-  gather_boundary(c, g);
+  gather_boundary(c, g, true);
   dim3 grid(nblocks(c.n, 256)), block(256);
   auto* kern = c.precision == 32 ? k_gather<false, true> : (c.field.periodic ? k_gather<true, false> : k_gather<false, false>);
   hipLaunchKernelGGL(kern, grid, block, 0, c.stream, g, c.force[0].p, c.force[1].p, c.force[2].p, c.torque[0].p,
@@ -561,16 +630,38 @@ void leapfrog(Ctx& c, const wdg_leapfrog_params* p) {
   a.clean = c.forceClean ? 1 : 0;
   a.dtScene = c.nScenes > 0 ? c.dtScene.p : nullptr;
   a.scene = c.scene.p;
-  if (c.graphCapture) a.gstop = c.gstate.p;
+  if (c.gated) a.gstop = c.gstate.p;
   // the flag word of this launch was cleared by the previous launch (or at creation)
   const int s = c.lfParity;
   a.dirty = c.dflags.p + DIRTY_PP + s;
   a.dirtyNext = c.dflags.p + DIRTY_PP + (1 - s);
   GatherArgs g = gather_args(c);
-  if (a.gather) gather_boundary(c, g);
-  dim3 grid(nblocks(c.n, 256)), block(256);
   // Leapfrog.cpp:132: a periodic scene is not tracked at step 0 (gradV is zero here)
   const bool track = c.trackEnergy && (!c.field.periodic || c.stepNow > 0);
+  dim3 grid(nblocks(c.n, 256)), block(256);
+  if (a.gather && c.nGBody > 0) {
+    a.part = c.bndPart.p;
+    a.gbody = c.gbody.p;
+    a.gbodyOf = c.gbodyOf.p;
+    a.parts = boundary_parts(c);
+    // short lists: a workgroup of this launch per body (the energy sums of the tracked variants are
+    // laid out per workgroup of particles); long ones cut into parts by a launch of their own
+    if (!track && a.parts == 1) {
+      a.foldBodies = (uint32_t)c.nGBody;
+      grid.x += a.foldBodies;
+    } else {
+      gather_boundary(c, g, false);
+    }
+  } else if (a.gather) {
+    a.gbodyOf = c.gbodyOf.p;
+  }
+  // a gated step is counted here when its filter ran (without slots k_gate counts it)
+  if (c.gated && c.con().n > 0) a.gs = c.gstate.p;
+  if (!c.gated) {
+    a.host = c.hflagsDev;
+    a.number = ++c.lfNumber;
+    a.err = c.dflags.p + 1;
+  }
   if (track && energy_per_scene(c)) {
     energy_scenes_prepare(c, c.con().n);
     a.enP = c.pe.p;
@@ -598,6 +689,7 @@ void leapfrog(Ctx& c, const wdg_leapfrog_params* p) {
   }
   c.lfParity = 1 - s;
   c.dirtyIdx = DIRTY_PP + s;
+  c.hostWords = !c.gated;
   c.forcesPending = false;
   // after a resetting step the integrated particles hold the reset value
   c.forceClean = p->reset != 0;
@@ -1257,12 +1349,12 @@ void energy_zero(Ctx& c, int term) {
   if (energy_per_scene(c)) {
     energy_scenes_prepare(c, c.con().n);
     hipLaunchKernelGGL(k_energy_zero_scenes, dim3(nblocks(c.nScenes, 256)), dim3(256), 0, c.stream, c.energyS.p,
-                       (int64_t)c.nScenes, term, c.graphCapture ? (const uint32_t*)c.gstate.p : nullptr);
+                       (int64_t)c.nScenes, term, c.gated ? (const uint32_t*)c.gstate.p : nullptr);
     WDG_LAUNCH_CHECK();
     return;
   }
   hipLaunchKernelGGL(k_energy_zero, dim3(1), dim3(64), 0, c.stream, c.energy.p, term,
-                     c.graphCapture ? (const uint32_t*)c.gstate.p : nullptr);
+                     c.gated ? (const uint32_t*)c.gstate.p : nullptr);
   WDG_LAUNCH_CHECK();
 }
 
@@ -1280,7 +1372,7 @@ void energy_add(Ctx& c, int64_t nBlocks, int nTerms, const int* target, int setM
   if (nBlocks <= 0) return;
   const int4 t = make_int4(target[0], nTerms > 1 ? target[1] : 0, nTerms > 2 ? target[2] : 0, nTerms > 3 ? target[3] : 0);
   hipLaunchKernelGGL(k_energy_add, dim3(1), dim3(256), 0, c.stream, c.enPart.p, nBlocks, nTerms, t, setMask,
-                     c.energy.p, c.graphCapture ? (const uint32_t*)c.gstate.p : nullptr);
+                     c.energy.p, c.gated ? (const uint32_t*)c.gstate.p : nullptr);
   WDG_LAUNCH_CHECK();
 }
 
@@ -1338,7 +1430,7 @@ void energy_scenes_prepare(Ctx& c, int64_t nc) {
   c.energyS.ensure((size_t)ns * WDG_EN_N);
   if (c.energySScenes != ns) {
     // another set of scenes (wdg_set_scenes): their terms start at zero
-    if (c.graphCapture) throw Error(WDG_E_STATE, "the scenes' energy terms are not set up while capturing");
+    if (c.gated) throw Error(WDG_E_STATE, "the scenes' energy terms are not set up while capturing");
     energy_scenes_reset(c, 1);
     c.energySScenes = ns;
   }
@@ -1348,7 +1440,7 @@ void energy_scenes_prepare(Ctx& c, int64_t nc) {
   c.sceneOff.ensure((size_t)ns + 1);
   c.enSPart.ensure((size_t)4 * ns * ENS_PARTS_MAX);
   if (c.sceneListGen == c.gen) return;
-  if (c.graphCapture) throw Error(WDG_E_STATE, "the scenes' particle lists are stale while capturing");
+  if (c.gated) throw Error(WDG_E_STATE, "the scenes' particle lists are stale while capturing");
   c.sceneKey.ensure((size_t)std::max<int64_t>(n, 1));
   c.sceneKeyTmp.ensure((size_t)std::max<int64_t>(n, 1));
   c.sceneList.ensure((size_t)std::max<int64_t>(n, 1));
@@ -1445,7 +1537,7 @@ __global__ void k_energy_scenes_sum(const double* __restrict__ sp, int64_t ns, i
 }
 
 static void energy_scenes_sum(Ctx& c, const double* part, int stride, int nTerms, int4 tgt) {
-  const uint32_t* gstop = c.graphCapture ? (const uint32_t*)c.gstate.p : nullptr;
+  const uint32_t* gstop = c.gated ? (const uint32_t*)c.gstate.p : nullptr;
   const int64_t ns = c.nScenes;
   // about 2048 workgroups over the scenes, so that a batch of few scenes still fills the chip
   const int parts = (int)std::min<int64_t>(ENS_PARTS_MAX, std::max<int64_t>(1, (2048 + ns - 1) / ns));
@@ -1459,7 +1551,7 @@ static void energy_scenes_sum(Ctx& c, const double* part, int stride, int nTerms
 
 void energy_scenes_contacts(Ctx& c) {
   Contacts& C = c.con();
-  const uint32_t* gstop = c.graphCapture ? (const uint32_t*)c.gstate.p : nullptr;
+  const uint32_t* gstop = c.gated ? (const uint32_t*)c.gstate.p : nullptr;
   hipLaunchKernelGGL(k_energy_at_pb, dim3(nblocks(c.n, 256)), dim3(256), 0, c.stream, c.n, c.nW, (const uint32_t*)C.adj.p,
                      (const uint32_t*)C.adjOff.p, c.rview(), (const double*)c.enC.p, c.pc.p, gstop);
   WDG_LAUNCH_CHECK();

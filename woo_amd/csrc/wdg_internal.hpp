@@ -81,6 +81,7 @@ __host__ __device__ inline int unpack_cd(uint64_t v, int k) {
 // dflags words: [0] dirty flag of a refresh / k_dirty, [1] error bits, [3..5] scan totals,
 // [DIRTY_PP + 0/1] dirty flags set by alternate leapfrog launches (each launch clears the other)
 constexpr int DIRTY_PP = 12;
+constexpr int HOST_DIRTY = 40, HOST_ERR = 41;  // words of the pinned host mirror only
 
 // device error bits
 enum : uint32_t {
@@ -273,6 +274,7 @@ struct Ctx {
   // out), the parts each one's list is cut into (from the largest list at the last refresh),
   // and their partial sums (up to 64 parts of 6 doubles per body)
   DBuf<uint32_t> gbody;
+  DBuf<uint32_t> gbodyOf;  // per boundary body its index in gbody, or NO_STATE (a facet)
   std::vector<uint32_t> gbodyHost;
   int64_t nGBody = 0;
   int bndParts = 1;
@@ -305,7 +307,9 @@ struct Ctx {
   DBuf<uint32_t> gstate;
   wdg_tuning tune{2, 8, 0};  // until wdg_tune / wdg_set_tuning: 2 force workgroups per group of slots
   int64_t gen = 0;  // bumped whenever buffers a captured graph uses may change
-  bool graphCapture = false;  // kernels being launched are captured for replay
+  // the kernels being launched are gated by the device words of gstate: captured for replay, or
+  // launched ahead of the host's checks (run_ahead)
+  bool gated = false;
   struct GraphCache {
     hipGraphExec_t exec = nullptr;
     int64_t gen = -1;
@@ -387,6 +391,12 @@ struct Ctx {
   DBuf<double> xfer;      // user-id-ordered staging for upload/download
   DBuf<uint32_t> dflags;  // [0] dirty, [1] error bits, [2..] scratch counters
   uint32_t* hflags = nullptr;  // pinned host mirror
+  // Words of the pinned mirror that the leapfrog writes itself, so that a collider call after it
+  // waits for the stream but copies nothing: [HOST_DIRTY] the number of the last leapfrog that left a
+  // particle outside its Verlet skin, [HOST_ERR] the error bits as that launch found them.
+  uint32_t* hflagsDev = nullptr;
+  uint32_t lfNumber = 0;    // leapfrog launches that wrote them
+  bool hostWords = false;   // they describe the last leapfrog
 
   // grid of the last refresh (for the on-demand potential-set report)
   struct GridState {
@@ -415,8 +425,8 @@ struct Ctx {
   bool eidxValid = false, eidxClean = false;
   double verletDist = NAN;
   int64_t nRefresh = 0, nCollide = 0;
-  // graph runner: the step of the last refresh and the running mean of the refresh interval
-  int64_t lastRefreshStep = -1;
+  // gated runs: steps since the last refresh and the running mean of the refresh interval
+  int64_t sinceRefresh = 0;
   double refreshEvery = 0;
   // hflags[0 .. DIRTY_PP + 1] mirror dflags after a graph batch (the next collider call uses them)
   bool hflagsFresh = false;
@@ -449,6 +459,10 @@ void flush_forces(Ctx& c);
 // IntraForce([In2_Facet]): the contact forces of each facet spread to its nodes (fnode)
 void intra_force(Ctx& c);
 void run_graph(Ctx& c, const wdg_program* prog, int64_t nSteps, int64_t* step, double* dt);
+// the same engine lists without a graph: steps launched ahead of the host's checks, gated on the
+// device as the replayed ones are; can_run_ahead says whether a program may be run so
+bool can_run_ahead(const Ctx& c, const wdg_program* prog);
+void run_ahead(Ctx& c, const wdg_program* prog, int64_t nSteps, int64_t* step, double* dt);
 uint32_t read_u32(Ctx& c, const uint32_t* d);
 int64_t tune(Ctx& c, const wdg_program* prog, int64_t* step, double* dt);
 double crit_dt(Ctx& c);
