@@ -100,6 +100,60 @@ def test_pairs_over_lanes_per_sphere(n):
     np.testing.assert_array_equal(np.sort(got, axis=1), want[np.lexsort((want[:, 1], want[:, 0]))])
 
 
+@pytest.mark.parametrize("n", [2, 255, 257, 5000, 262145 + 300])
+@pytest.mark.parametrize("stepped", [False, True])
+def test_observables_over_workgroups(n, stepped):
+    # one workgroup, ragged ones, and more workgroups than one pass of the last reduction takes; the
+    # contacts straight from the refresh, and after steps
+    from woo_amd._native import SPHERE, Device
+
+    rng = np.random.default_rng(n)
+    m = int(np.ceil(n ** (1 / 3.)))
+    pos = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n] * 2e-3
+    r = rng.uniform(.95e-3, 1.05e-3, n)
+    r[0] = r[n - 1] = 1.05e-3
+    mass = rng.uniform(1e-5, 2e-5, n)
+    vel = rng.normal(0., 1e-4, (n, 3))
+    E, kdk = 1e6, .2
+    d = Device(0)
+    d.set_field(periodic=False)
+    d.set_materials([dict(kind=0, density=1., young=E, ktDivKn=kdk, tanPhi=.5, surfEnergy=0., alpha=0.)])
+    d.upload_particles(shape=np.full(n, SPHERE, np.int32), pos=pos, radius=r, mass=mass,
+                       inertia=np.repeat((.4 * mass * r * r)[:, None], 3, 1), vel=vel)
+    d.collide(-.05)
+    d.contact_loop(0, 1e-9)
+    if stepped:
+        d.leapfrog(1e-9)
+        d.contact_loop(1, 1e-9)
+    pos, vel = d.get("pos"), d.get("vel")
+    ids = d.contacts(real_only=True, data=False)[0]
+    assert len(ids)
+    cnt = np.bincount(ids.reshape(-1), minlength=n)
+    o = d.observables((-1., -1., -1.), (1., 1., 1.))
+    n0, n1 = np.sum(cnt == 0), np.sum(cnt == 1)
+    assert o["coordNumber"] == cnt.sum() / n
+    if n > n0 + n1:
+        assert o["coordNumberSkipFree"] == (cnt.sum() - n1) / (n - n0 - n1)
+    eps = np.finfo(float).eps
+    # sums of n terms of one sign over 256-wide trees and a 1,024-wide last stage
+    tol = 32 * eps
+    assert abs(o["solidFraction"] / (np.sum(4 / 3. * np.pi * r ** 3) / 8.) - 1) <= tol
+    ek = np.sum(.5 * mass * np.sum(vel ** 2, 1)) + np.sum(.5 * .4 * mass * r * r * np.sum(d.get("angVel") ** 2, 1))
+    assert abs(d.kinetic_energy() / ek - 1) <= tol
+    # the stiffness of every particle, a few dozen roundings per contact term
+    i, j = ids.T
+    kn = 1 / (1 / (E * np.pi * np.minimum(r[i], r[j]) ** 2 / r[i]) + 1 / (E * np.pi * np.minimum(r[i], r[j]) ** 2 / r[j]))
+    nn = pos[j] - pos[i]
+    n2 = (nn / np.linalg.norm(nn, axis=1)[:, None]) ** 2
+    kt, kr = np.zeros((n, 3)), np.zeros((n, 3))
+    for e in (i, j):
+        np.add.at(kt, e, n2 * (kn * (1 - kdk))[:, None] + (kdk * kn)[:, None])
+        np.add.at(kr, e, (r[e] ** 2 * kdk * kn)[:, None] * (1 - n2))
+    with np.errstate(divide="ignore"):
+        crit = np.sqrt(2 * min(np.min(mass[:, None] / kt), np.min((.4 * mass * r * r)[:, None] / kr)))
+    assert abs(d.crit_dt() / crit - 1) <= 64 * eps
+
+
 @pytest.mark.parametrize("n,flat,steps", [(20, False, 1), (300, False, 7), (300, False, 130), (4900, True, 40)])
 @pytest.mark.parametrize("track", [False, True])
 def test_steps_ahead_equal_engine_calls(n, flat, steps, track):

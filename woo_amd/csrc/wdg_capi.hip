@@ -516,9 +516,11 @@ int wdg_ctx_create(int device, wdg_ctx** out) {
     WDG_HIP(hipStreamCreateWithFlags(&ctx->c.stream, hipStreamNonBlocking));
     ctx->c.dflags.ensure(64);
     WDG_HIP(hipMemset(ctx->c.dflags.p, 0, 64 * sizeof(uint32_t)));
-    WDG_HIP(hipHostMalloc((void**)&ctx->c.hflags, 64 * sizeof(uint32_t), hipHostMallocDefault));
-    std::memset(ctx->c.hflags, 0, 64 * sizeof(uint32_t));
+    WDG_HIP(hipHostMalloc((void**)&ctx->c.hflags, HOST_WORDS * sizeof(uint32_t), hipHostMallocDefault));
+    std::memset(ctx->c.hflags, 0, HOST_WORDS * sizeof(uint32_t));
     WDG_HIP(hipHostGetDevicePointer((void**)&ctx->c.hflagsDev, ctx->c.hflags, 0));
+    ctx->c.hres = reinterpret_cast<double*>(ctx->c.hflags + HOST_RES);
+    ctx->c.hresDev = reinterpret_cast<double*>(ctx->c.hflagsDev + HOST_RES);
     ctx->c.red.ensure(64);
     // the device's copy of the no-allocation entry points' scratch array
     scratch_setup(device);
@@ -569,7 +571,7 @@ int wdg_ctx_destroy(wdg_ctx* ctx) {
       c.snapEp[k].release();
     }
     c.snapMatch.release();
-    c.sortHist.release(); c.scanWords.release(); c.scanTicket.release(); c.cellCnt.release(); c.cellRank.release(); c.red.release(); c.xfer.release(); c.dflags.release();
+    c.sortHist.release(); c.scanWords.release(); c.scanTicket.release(); c.cellCnt.release(); c.cellRank.release(); c.red.release(); c.obsPart.release(); c.dynRec.release(); c.xfer.release(); c.dflags.release();
     if (c.hflags) (void)hipHostFree(c.hflags);
     if (c.stream) (void)hipStreamDestroy(c.stream);
   });

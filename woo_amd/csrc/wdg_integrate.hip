@@ -721,19 +721,30 @@ struct DynArgs {
   const double* fgeo;
   int hertz;
   double poisson, en, viscAlpha;
-  unsigned long long* out;
-  const uint32_t* scene;  // batched scenes: the minimum per scene, out[scene] (else one, out[0])
+  int64_t nc;
+  const uint32_t *eidx, *sidx;  // per-entry real slots and their state indices, when kept
+  double* rec;                  // DYN_REC doubles per state index
+  unsigned long long* out;      // one per workgroup; batched scenes: one per scene
+  const uint32_t* scene;        // batched scenes, else null
 };
 
+// The stiffness of one real contact, once for both of its particles: its translational diagonal
+// (3), its tangential stiffness, the sums of the other two squared normal components (3) that its
+// rotational diagonal takes, and pA's lever arm (pB, always a sphere, has its radius). The particle
+// pass then only adds records up. Bound by the FP64 arithmetic here and the gather there: at
+// 400,000 spheres with 757,000 contacts 71 us together; evaluated per adjacency entry, so
+// twice per contact and as often as the lane of a wavefront with the most contacts, 175 us.
+constexpr int DYN_REC = 8;
 template <int PREC>
-__device__ __forceinline__ void dyn_one(const DynArgs& a, uint32_t e, d3& kt, d3& kr) {
-  const uint32_t s = e & ~ADJ_PA;
+__global__ __launch_bounds__(256) void k_dyn_contacts(DynArgs a) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= a.nc) return;
+  const uint32_t s = (uint32_t)c;
   if (!rv_real(a.rv, s)) return;
   const uint32_t r = rv_index(a.rv, s);
   const uint32_t inf = a.info[s];
   const bool swap = (inf & CI_SWAP) != 0u;
   const uint32_t pA = swap ? a.B[s] : a.A[s], pB = swap ? a.A[s] : a.B[s];
-  const int ix = (e & ADJ_PA) ? 0 : 1;
   double r1, r2;
   contact_radii(inf, pA, pB, a.rad, a.fgeo, r1, r2);
   double l0, l1, A;
@@ -758,13 +769,22 @@ __device__ __forceinline__ void dyn_one(const DynArgs& a, uint32_t e, d3& kt, d3
   q4 q = quat_from_cols(T0, T1, cross3(T0, T1));
   d3 n = quat_rot(q, mk3(1., 0., 0.));
   d3 n2 = mk3(n.x * n.x, n.y * n.y, n.z * n.z);
-  kt = mk3(kt.x + (n2.x * (kn - ktt) + ktt), kt.y + (n2.y * (kn - ktt) + ktt), kt.z + (n2.z * (kn - ktt) + ktt));
-  double l = ix == 0 ? l0 : l1;
-  double lk = (l * l) * ktt;
-  kr = mk3(kr.x + lk * (n2.y + n2.z), kr.y + lk * (n2.z + n2.x), kr.z + lk * (n2.x + n2.y));
+  double2* o = reinterpret_cast<double2*>(a.rec + (int64_t)DYN_REC * r);
+  o[0] = make_double2(n2.x * (kn - ktt) + ktt, n2.y * (kn - ktt) + ktt);
+  o[1] = make_double2(n2.z * (kn - ktt) + ktt, ktt);
+  o[2] = make_double2(n2.y + n2.z, n2.z + n2.x);
+  o[3] = make_double2(n2.x + n2.y, l0);
+}
+// a contact's record added to the stiffness of one of its particles (of radius rad, when it is pB)
+__device__ __forceinline__ void dyn_add(const double* rec, bool isPA, double rad, d3& kt, d3& kr) {
+  const double2* o = reinterpret_cast<const double2*>(rec);
+  const double2 a = o[0], b = o[1], c = o[2], d = o[3];
+  kt = mk3(kt.x + a.x, kt.y + a.y, kt.z + b.x);
+  const double l = isPA ? d.y : rad;
+  const double lk = (l * l) * b.y;
+  kr = mk3(kr.x + lk * c.x, kr.y + lk * c.y, kr.z + lk * d.x);
 }
 
-template <int PREC>
 __global__ __launch_bounds__(256) void k_dyndt(DynArgs a) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   double ret = INFINITY;
@@ -772,7 +792,24 @@ __global__ __launch_bounds__(256) void k_dyndt(DynArgs a) {
     const uint32_t fl = a.flags[i];
     if ((fl & F_INTEGRATED) && (fl & F_DOF_ALL) != F_DOF_ALL) {
       d3 kt = mk3(0., 0., 0.), kr = mk3(0., 0., 0.);
-      for (uint32_t k = a.adjOff[i]; k < a.adjOff[i + 1]; k++) dyn_one<PREC>(a, a.adj[k], kt, kr);
+      const double rad = a.rad[i];
+      const uint32_t k1 = a.adjOff[i + 1];
+      for (uint32_t k = a.adjOff[i]; k < k1; k++) {
+        uint32_t r;
+        bool isPA;
+        if (a.eidx) {
+          const uint32_t v = a.eidx[k];
+          if (v == NO_STATE) continue;
+          isPA = (v & EIDX_PA) != 0u;
+          r = a.sidx[v & ~EIDX_PA];
+        } else {
+          const uint32_t e = a.adj[k], s = e & ~ADJ_PA;
+          if (!rv_real(a.rv, s)) continue;
+          isPA = (e & ADJ_PA) != 0u;
+          r = rv_index(a.rv, s);
+        }
+        dyn_add(a.rec + (int64_t)DYN_REC * r, isPA, rad, kt, kr);
+      }
       const double m = a.mass[i];
       const double I[3] = {a.ix[i], a.iy[i], a.iz[i]};
       const double ktv[3] = {kt.x, kt.y, kt.z}, krv[3] = {kr.x, kr.y, kr.z};
@@ -785,23 +822,66 @@ __global__ __launch_bounds__(256) void k_dyndt(DynArgs a) {
   }
   // non-negative doubles order like their bit patterns
   unsigned long long b = (unsigned long long)__double_as_longlong(ret);
-  uint32_t sc = 0u;
   if (a.scene) {
     // scenes lie in runs of storage order: a wavefront of one scene reduces first, a mixed one
     // (or the tail past n) takes one atomic per particle
-    sc = i < a.n ? a.scene[i] : 0xFFFFFFFFu;
+    const uint32_t sc = i < a.n ? a.scene[i] : 0xFFFFFFFFu;
     const uint32_t s0 = __shfl(sc, 0);
     if (!__all(sc == s0)) {
       if (i < a.n && ret != INFINITY) atomicMin(&a.out[sc], b);
       return;
     }
     if (s0 == 0xFFFFFFFFu) return;
+    for (int off = 32; off > 0; off >>= 1) {
+      unsigned long long o = __shfl_xor(b, off);
+      b = o < b ? o : b;
+    }
+    if ((threadIdx.x & 63) == 0) atomicMin(&a.out[s0], b);
+    return;
   }
+  // one word per workgroup (k_min_words takes their minimum)
+  __shared__ unsigned long long wm[4];
   for (int off = 32; off > 0; off >>= 1) {
     unsigned long long o = __shfl_xor(b, off);
     b = o < b ? o : b;
   }
-  if ((threadIdx.x & 63) == 0) atomicMin(&a.out[sc], b);
+  if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = b;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 4; w++) b = wm[w] < b ? wm[w] : b;
+    a.out[blockIdx.x] = b;
+  }
+}
+
+// Reductions of the workgroups' partial results by one workgroup, in a fixed order, straight into
+// pinned host memory: reading a value back then is the wait for the stream and nothing else
+// (before: a buffer allocated and freed by each call, all partials copied, the sums on the host).
+__global__ __launch_bounds__(1024) void k_min_words(int64_t nb, const unsigned long long* __restrict__ part,
+                                                     unsigned long long* out) {
+  __shared__ unsigned long long wm[16];
+  unsigned long long b = ~0ull;
+  for (int64_t i = threadIdx.x; i < nb; i += blockDim.x) b = part[i] < b ? part[i] : b;
+  for (int off = 32; off > 0; off >>= 1) {
+    const unsigned long long o = __shfl_xor(b, off);
+    b = o < b ? o : b;
+  }
+  if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = b;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; w++) b = wm[w] < b ? wm[w] : b;
+    *out = b;
+  }
+}
+// NT sums over nb rows of NT partials: thread t adds rows t, t + 1024, ..., then a fixed tree
+template <int NT>
+__global__ __launch_bounds__(1024) void k_sum_rows(int64_t nb, const double* __restrict__ part, double* out) {
+  double v[NT];
+#pragma unroll
+  for (int q = 0; q < NT; q++) v[q] = 0.;
+  for (int64_t b = threadIdx.x; b < nb; b += blockDim.x)
+#pragma unroll
+    for (int q = 0; q < NT; q++) v[q] += part[NT * b + q];
+  block_sum_store<NT, 1024>(v, out);
 }
 
 static DynArgs dyn_args(Ctx& c) {
@@ -818,7 +898,21 @@ static DynArgs dyn_args(Ctx& c) {
   if (c.matEpochs > 1) a.hE = R.hE.p;
   a.hertz = c.lastPhysKind == WDG_PHYS_HERTZ;
   a.poisson = c.lastPoisson; a.en = c.lastEn; a.viscAlpha = c.lastViscAlpha;
+  a.nc = C.n;
+  if (c.eidxValid && R.sidxValid) {
+    a.eidx = C.eidx.p;
+    a.sidx = R.sidx.p;
+  }
+  c.dynRec.ensure((size_t)DYN_REC * ngroups(C.n) * GROUP);
+  a.rec = c.dynRec.p;
   return a;
+}
+static void dyn_launch(Ctx& c, const DynArgs& a) {
+  hipLaunchKernelGGL(c.precision == 32 ? k_dyn_contacts<32> : k_dyn_contacts<64>, dim3(nblocks(a.nc, 256)), dim3(256),
+                     0, c.stream, a);
+  WDG_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_dyndt, dim3(nblocks(c.n, 256)), dim3(256), 0, c.stream, a);
+  WDG_LAUNCH_CHECK();
 }
 
 double crit_dt(Ctx& c) {
@@ -826,19 +920,15 @@ double crit_dt(Ctx& c) {
   if (c.n == 0) return INFINITY;
   if (c.con().n == 0) return INFINITY;
   DynArgs a = dyn_args(c);
-  unsigned long long* out = reinterpret_cast<unsigned long long*>(c.red.p);
-  unsigned long long init = (unsigned long long)0x7FF0000000000000ull;  // +inf
-  WDG_HIP(hipMemcpyAsync(out, &init, sizeof(init), hipMemcpyHostToDevice, c.stream));
-  a.out = out;
-  hipLaunchKernelGGL(c.precision == 32 ? k_dyndt<32> : k_dyndt<64>, dim3(nblocks(c.n, 256)), dim3(256), 0, c.stream,
-                     a);
+  const unsigned nb = nblocks(c.n, 256);
+  c.obsPart.ensure(nb);
+  a.out = reinterpret_cast<unsigned long long*>(c.obsPart.p);
+  dyn_launch(c, a);
+  hipLaunchKernelGGL(k_min_words, dim3(1), dim3(1024), 0, c.stream, (int64_t)nb, (const unsigned long long*)a.out,
+                     reinterpret_cast<unsigned long long*>(c.hresDev));
   WDG_LAUNCH_CHECK();
-  unsigned long long hb;
-  WDG_HIP(hipMemcpyAsync(&hb, out, sizeof(hb), hipMemcpyDeviceToHost, c.stream));
   WDG_HIP(hipStreamSynchronize(c.stream));
-  double r;
-  std::memcpy(&r, &hb, 8);
-  return std::sqrt(r);
+  return std::sqrt(c.hres[0]);
 }
 
 // DynDt::critDt_stiffness of each scene of a batched context: the same per-particle values,
@@ -854,9 +944,7 @@ void crit_dt_scenes(Ctx& c, std::vector<double>& out) {
   WDG_HIP(hipMemcpyAsync(d.p, h.data(), h.size() * 8, hipMemcpyHostToDevice, c.stream));
   a.out = d.p;
   a.scene = c.scene.p;
-  hipLaunchKernelGGL(c.precision == 32 ? k_dyndt<32> : k_dyndt<64>, dim3(nblocks(c.n, 256)), dim3(256), 0, c.stream,
-                     a);
-  WDG_LAUNCH_CHECK();
+  dyn_launch(c, a);
   WDG_HIP(hipMemcpyAsync(h.data(), d.p, h.size() * 8, hipMemcpyDeviceToHost, c.stream));
   WDG_HIP(hipStreamSynchronize(c.stream));
   d.release();
@@ -868,27 +956,24 @@ void crit_dt_scenes(Ctx& c, std::vector<double>& out) {
 }
 
 // ------------------------------------------------------------------ observables
-__global__ void k_count_contacts(int64_t n, RealView rv, const uint32_t* __restrict__ adj,
-                                 const uint32_t* __restrict__ adjOff, uint32_t* cnt) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  uint32_t k = 0;
-  for (uint32_t j = adjOff[i]; j < adjOff[i + 1]; j++) k += rv_real(rv, adj[j] & ~ADJ_PA) ? 1u : 0u;
-  cnt[i] = k;
-}
-
-// block partial sums in fixed order (deterministic): [C2, N0, N1, N, Vs]
-__global__ __launch_bounds__(256) void k_obs_partial(int64_t n, const uint32_t* __restrict__ cnt,
+// block partial sums in fixed order (deterministic): [C2, N0, N1, N, Vs]; a particle's real
+// contacts are counted from its per-entry real slots when they are kept
+__global__ __launch_bounds__(256) void k_obs_partial(int64_t n, RealView rv, const uint32_t* __restrict__ adj,
+                                                     const uint32_t* __restrict__ adjOff,
+                                                     const uint32_t* __restrict__ eidx,
                                                      const uint32_t* __restrict__ flags, const double* __restrict__ rad,
                                                      const double* __restrict__ px, const double* __restrict__ py,
                                                      const double* __restrict__ pz, double lo0, double lo1, double lo2,
                                                      double hi0, double hi1, double hi2, double* part) {
-  __shared__ double s[5][256];
-  const int tid = threadIdx.x;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + tid;
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   double v[5] = {0, 0, 0, 0, 0};
   if (i < n) {
-    uint32_t k = cnt[i];
+    uint32_t k = 0;
+    if (adjOff) {
+      const uint32_t j1 = adjOff[i + 1];
+      for (uint32_t j = adjOff[i]; j < j1; j++)
+        k += (eidx ? eidx[j] != NO_STATE : rv_real(rv, adj[j] & ~ADJ_PA)) ? 1u : 0u;
+    }
     v[0] = k;
     v[1] = k == 0;
     v[2] = k == 1;
@@ -900,41 +985,28 @@ __global__ __launch_bounds__(256) void k_obs_partial(int64_t n, const uint32_t* 
       if (in) v[4] = (4 / 3.) * M_PI * (r * r * r);
     }
   }
-  for (int q = 0; q < 5; q++) s[q][tid] = v[q];
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (tid < st)
-      for (int q = 0; q < 5; q++) s[q][tid] += s[q][tid + st];
-    __syncthreads();
-  }
-  if (tid == 0)
-    for (int q = 0; q < 5; q++) part[(int64_t)q * gridDim.x + blockIdx.x] = s[q][0];
+  block_sum_store<5, 256>(v, part + (int64_t)5 * blockIdx.x);
 }
 
 void observables(Ctx& c, const double lo[3], const double hi[3], double out[3]) {
   if (c.forcesPending) flush_forces(c);
   Contacts& C = c.con();
-  c.scount.ensure(c.n + 1);
-  if (C.n > 0 && c.n > 0) {
-    hipLaunchKernelGGL(k_count_contacts, dim3(nblocks(c.n, 256)), dim3(256), 0, c.stream, c.n, c.rview(), C.adj.p,
-                       C.adjOff.p, c.scount.p);
-    WDG_LAUNCH_CHECK();
-  } else {
-    WDG_HIP(hipMemsetAsync(c.scount.p, 0, (c.n + 1) * sizeof(uint32_t), c.stream));
-  }
-  unsigned nb = nblocks(c.n, 256);
-  std::vector<double> part((size_t)5 * nb);
-  DBuf<double> dpart;
-  dpart.ensure(part.size());
-  hipLaunchKernelGGL(k_obs_partial, dim3(nb), dim3(256), 0, c.stream, c.n, c.scount.p, c.flags.p, c.radius.p,
-                     c.pos[0].p, c.pos[1].p, c.pos[2].p, lo[0], lo[1], lo[2], hi[0], hi[1], hi[2], dpart.p);
-  WDG_LAUNCH_CHECK();
-  WDG_HIP(hipMemcpyAsync(part.data(), dpart.p, part.size() * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-  WDG_HIP(hipStreamSynchronize(c.stream));
-  dpart.release();
   double S[5] = {0, 0, 0, 0, 0};
-  for (int q = 0; q < 5; q++)
-    for (unsigned b = 0; b < nb; b++) S[q] += part[(size_t)q * nb + b];
+  if (c.n > 0) {
+    const unsigned nb = nblocks(c.n, 256);
+    c.obsPart.ensure((size_t)5 * nb);
+    const bool any = C.n > 0;
+    hipLaunchKernelGGL(k_obs_partial, dim3(nb), dim3(256), 0, c.stream, c.n, c.rview(), (const uint32_t*)C.adj.p,
+                       any ? (const uint32_t*)C.adjOff.p : nullptr,
+                       any && c.eidxValid ? (const uint32_t*)C.eidx.p : nullptr, c.flags.p, c.radius.p, c.pos[0].p,
+                       c.pos[1].p, c.pos[2].p, lo[0], lo[1], lo[2], hi[0], hi[1], hi[2], c.obsPart.p);
+    WDG_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_sum_rows<5>, dim3(1), dim3(1024), 0, c.stream, (int64_t)nb, (const double*)c.obsPart.p,
+                       c.hresDev);
+    WDG_LAUNCH_CHECK();
+    WDG_HIP(hipStreamSynchronize(c.stream));
+    for (int q = 0; q < 5; q++) S[q] = c.hres[q];
+  }
   const double C2 = S[0], N0 = S[1], N1 = S[2], N = S[3], Vs = S[4];
   out[0] = C2 / N;
   out[1] = (C2 - N1) / (N - N0 - N1);
@@ -946,7 +1018,7 @@ void observables(Ctx& c, const double lo[3], const double hi[3], double out[3]) 
 // DemFuncs::stressStiffness, stress part (Funcs.cpp:183-229): per real contact
 // d0 = |posA - shift - posB|, n = ori*e_x, F = ori*force (the gather record's global force),
 // fN = F.n, fT = F - n fN, sigma_ij += d0 (fN n_i n_j + (fT_i n_j + fT_j n_i)/2).
-// Block partial sums in slot order, added on the host in block order.
+// Workgroup partial sums, added by k_sum_rows.
 struct StressArgs {
   int64_t nc;
   const uint32_t *A, *B, *info;
@@ -960,9 +1032,7 @@ struct StressArgs {
 };
 template <int PREC>
 __global__ __launch_bounds__(256) void k_stress(StressArgs a) {
-  __shared__ double sh[9][256];
-  const int tid = threadIdx.x;
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + tid;
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
   if (c < a.nc && rv_real(a.rv, (uint32_t)c)) {
     const uint32_t r = rv_index(a.rv, (uint32_t)c);
@@ -1004,15 +1074,7 @@ __global__ __launch_bounds__(256) void k_stress(StressArgs a) {
     for (int i = 0; i < 3; i++)
       for (int j = 0; j < 3; j++) v[3 * i + j] = d0 * (fN * nn[i] * nn[j] + .5 * (tt[i] * nn[j] + tt[j] * nn[i]));
   }
-  for (int q = 0; q < 9; q++) sh[q][tid] = v[q];
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (tid < st)
-      for (int q = 0; q < 9; q++) sh[q][tid] += sh[q][tid + st];
-    __syncthreads();
-  }
-  if (tid == 0)
-    for (int q = 0; q < 9; q++) a.part[(int64_t)blockIdx.x * 9 + q] = sh[q][0];
+  block_sum_store<9, 256>(v, a.part + (int64_t)9 * blockIdx.x);
 }
 
 void stress(Ctx& c, double volume, double out[9]) {
@@ -1025,8 +1087,7 @@ void stress(Ctx& c, double volume, double out[9]) {
   if (C.n == 0) return;
   Reals& R = c.reals();
   const unsigned nb = nblocks(C.n, 256);
-  DBuf<double> part;
-  part.ensure((size_t)nb * 9);
+  c.obsPart.ensure((size_t)nb * 9);
   StressArgs a{};
   a.nc = C.n; a.A = C.A.p; a.B = C.B.p; a.info = C.info.p; a.dist = C.dist.p; a.rv = c.rview();
   a.N0 = R.hN[0].p; a.N1 = R.hN[1].p; a.N2 = R.hN[2].p; a.Y0 = R.hY[0].p; a.Y1 = R.hY[1].p; a.Y2 = R.hY[2].p;
@@ -1034,16 +1095,14 @@ void stress(Ctx& c, double volume, double out[9]) {
   a.px = c.pos[0].p; a.py = c.pos[1].p; a.pz = c.pos[2].p;
   for (int k = 0; k < 3; k++) a.L[k] = c.field.cell[k];
   a.periodic = c.field.periodic;
-  a.part = part.p;
+  a.part = c.obsPart.p;
   hipLaunchKernelGGL(c.precision == 32 ? k_stress<32> : k_stress<64>, dim3(nb), dim3(256), 0, c.stream, a);
   WDG_LAUNCH_CHECK();
-  std::vector<double> h((size_t)nb * 9);
-  WDG_HIP(hipMemcpyAsync(h.data(), part.p, h.size() * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+  hipLaunchKernelGGL(k_sum_rows<9>, dim3(1), dim3(1024), 0, c.stream, (int64_t)nb, (const double*)c.obsPart.p,
+                     c.hresDev);
+  WDG_LAUNCH_CHECK();
   WDG_HIP(hipStreamSynchronize(c.stream));
-  part.release();
-  for (unsigned b = 0; b < nb; b++)
-    for (int k = 0; k < 9; k++) out[k] += h[(size_t)b * 9 + k];
-  for (int k = 0; k < 9; k++) out[k] /= volume;
+  for (int k = 0; k < 9; k++) out[k] = c.hres[k] / volume;
 }
 
 // sum over integrated nodes of m v.v/2 + w.(I w)/2
@@ -1053,9 +1112,7 @@ __global__ __launch_bounds__(256) void k_ek(int64_t n, const uint32_t* __restric
                                           const double* __restrict__ wy, const double* __restrict__ wz,
                                           const double* __restrict__ ix, const double* __restrict__ iy,
                                           const double* __restrict__ iz, double* part) {
-  __shared__ double sh[256];
-  const int tid = threadIdx.x;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + tid;
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   double e = 0;
   if (i < n && (flags[i] & F_INTEGRATED)) {
     const d3 v = mk3(vx[i], vy[i], vz[i]), w = mk3(wx[i], wy[i], wz[i]);
@@ -1063,38 +1120,29 @@ __global__ __launch_bounds__(256) void k_ek(int64_t n, const uint32_t* __restric
     const double er = 0.5 * dot3(w, mk3(ix[i] * w.x, iy[i] * w.y, iz[i] * w.z));
     e = et + er;
   }
-  sh[tid] = e;
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (tid < st) sh[tid] += sh[tid + st];
-    __syncthreads();
-  }
-  if (tid == 0) part[blockIdx.x] = sh[0];
+  double v[1] = {e};
+  block_sum_store<1, 256>(v, part + blockIdx.x);
 }
 
 double kinetic_energy(Ctx& c) {
   if (c.n == 0) return 0;
   const unsigned nb = nblocks(c.n, 256);
-  DBuf<double> part;
-  part.ensure(nb);
+  c.obsPart.ensure(nb);
   hipLaunchKernelGGL(k_ek, dim3(nb), dim3(256), 0, c.stream, c.n, c.flags.p, c.mass.p, c.vel[0].p, c.vel[1].p,
                      c.vel[2].p, c.angVel[0].p, c.angVel[1].p, c.angVel[2].p, c.inertia[0].p, c.inertia[1].p,
-                     c.inertia[2].p, part.p);
+                     c.inertia[2].p, c.obsPart.p);
   WDG_LAUNCH_CHECK();
-  std::vector<double> h(nb);
-  WDG_HIP(hipMemcpyAsync(h.data(), part.p, nb * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+  hipLaunchKernelGGL(k_sum_rows<1>, dim3(1), dim3(1024), 0, c.stream, (int64_t)nb, (const double*)c.obsPart.p,
+                     c.hresDev);
+  WDG_LAUNCH_CHECK();
   WDG_HIP(hipStreamSynchronize(c.stream));
-  part.release();
-  double s = 0;
-  for (double x : h) s += x;
-  return s;
+  return c.hres[0];
 }
 
 // ------------------------------------------------------------------ kinetic energy, no allocation
 // For callers that cannot allocate device memory (code under HIP graph capture, serving loops):
-// k_ek's per-workgroup partials go to a file-scope device array instead of a fresh buffer, and
-// one thread adds them in block order, left to right, as kinetic_energy does on the host, so
-// both give the same bits. Every GPU holds its own copy of the array until the process ends;
+// k_ek's per-workgroup partials go to a file-scope device array instead of the context's buffer, and
+// are added as kinetic_energy adds them (k_sum_rows), so both give the same bits. Every GPU holds its own copy of the array until the process ends;
 // its address on each device is looked up once, with that device current, at context creation.
 // All calls on one GPU share the array: calls that overlap on one GPU race. The partials are
 // written in full before they are read, so nothing needs clearing.
@@ -1113,13 +1161,6 @@ void scratch_setup(int device) {
   g_scratch[device] = static_cast<double*>(p);
 }
 
-__global__ void k_sum_in_order(const double* __restrict__ part, int64_t nb, double* out) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  double s = 0;
-  for (int64_t b = 0; b < nb; b++) s += part[b];
-  *out = s;
-}
-
 void kinetic_energy_noalloc(Ctx& c, double* dOut) {
   const int64_t nb = nblocks(c.n, 256);
   if (nb > EK_SCRATCH_MAX)
@@ -1133,7 +1174,7 @@ void kinetic_energy_noalloc(Ctx& c, double* dOut) {
                        c.inertia[1].p, c.inertia[2].p, part);
     WDG_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(k_sum_in_order, dim3(1), dim3(64), 0, c.stream, part, nb, dOut);
+  hipLaunchKernelGGL(k_sum_rows<1>, dim3(1), dim3(1024), 0, c.stream, nb, (const double*)part, dOut);
   WDG_LAUNCH_CHECK();
 }
 

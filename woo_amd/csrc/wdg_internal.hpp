@@ -82,6 +82,7 @@ __host__ __device__ inline int unpack_cd(uint64_t v, int k) {
 // [DIRTY_PP + 0/1] dirty flags set by alternate leapfrog launches (each launch clears the other)
 constexpr int DIRTY_PP = 12;
 constexpr int HOST_DIRTY = 40, HOST_ERR = 41;  // words of the pinned host mirror only
+constexpr int HOST_RES = 64, HOST_WORDS = 128;  // its words from HOST_RES on hold doubles
 
 // device error bits
 enum : uint32_t {
@@ -388,6 +389,8 @@ struct Ctx {
   DBuf<double> energy;
   DBuf<double> enPart;
   DBuf<double> red;       // reductions
+  DBuf<double> obsPart;   // per-workgroup partial results of the observables
+  DBuf<double> dynRec;    // DynDt: the stiffness record of each real contact
   DBuf<double> xfer;      // user-id-ordered staging for upload/download
   DBuf<uint32_t> dflags;  // [0] dirty, [1] error bits, [2..] scratch counters
   uint32_t* hflags = nullptr;  // pinned host mirror
@@ -395,6 +398,7 @@ struct Ctx {
   // waits for the stream but copies nothing: [HOST_DIRTY] the number of the last leapfrog that left a
   // particle outside its Verlet skin, [HOST_ERR] the error bits as that launch found them.
   uint32_t* hflagsDev = nullptr;
+  double *hres = nullptr, *hresDev = nullptr;  // pinned results of the reductions (in the same block)
   uint32_t lfNumber = 0;    // leapfrog launches that wrote them
   bool hostWords = false;   // they describe the last leapfrog
 
