@@ -123,7 +123,6 @@ struct RestoreArgs {
   const uint32_t* rec;
   const double* data;
   RealView rv;
-  const uint64_t* dist;  // packed cellDist per slot (periodic cells; else null)
   double *N0, *N1, *N2, *Y0, *Y1, *Y2, *F0, *F1, *F2, *uN, *gp;
   // material epochs (while more than one table is kept): each record's (else all take epoch)
   uint8_t* hE;
@@ -144,13 +143,12 @@ __global__ void k_restore(RestoreArgs a) {
   a.Y0[k] = T1.x; a.Y1[k] = T1.y; a.Y2[k] = T1.z;
   a.F0[k] = d[9]; a.F1[k] = d[10]; a.F2[k] = d[11];
   a.uN[k] = d[12];
-  // the gather record as the force pass writes it: global force on pA, contact point, cellDist
+  // the gather record as the force pass writes it: global force on pA, contact point
   const d3 G = quat_rot(quat_from_cols(T0, T1, cross3(T0, T1)), mk3(d[9], d[10], d[11]));
   double2* g2 = reinterpret_cast<double2*>(a.gp + (int64_t)GP * k);
   g2[0] = make_double2(G.x, G.y);
   g2[1] = make_double2(G.z, d[6]);
   g2[2] = make_double2(d[7], d[8]);
-  g2[3] = make_double2(__longlong_as_double((long long)(a.dist ? a.dist[s] : 0ull)), 0.);
 }
 
 // Contact history of a checkpoint (the save half is wdg_contact_list(which=1)): a full
@@ -217,7 +215,6 @@ void restore_contacts(Ctx& c, int64_t n, const int32_t* ids, const int32_t* cell
   Reals& R = c.reals();
   RestoreArgs a{};
   a.nc = nc; a.rec = drec.p; a.data = ddata.p; a.rv = c.rview();
-  a.dist = c.field.periodic ? C.dist.p : nullptr;
   a.N0 = R.hN[0].p; a.N1 = R.hN[1].p; a.N2 = R.hN[2].p;
   a.Y0 = R.hY[0].p; a.Y1 = R.hY[1].p; a.Y2 = R.hY[2].p;
   a.F0 = R.hF[0].p; a.F1 = R.hF[1].p; a.F2 = R.hF[2].p; a.uN = R.huN.p; a.gp = R.gp.p;
@@ -334,7 +331,6 @@ void snapshot_contacts_load(Ctx& c, int slot) {
     Reals& R = c.reals();
     RestoreArgs a{};
     a.nc = nc; a.rec = c.snapMatch.p; a.data = c.snapRec[slot].p; a.rv = c.rview();
-    a.dist = per ? C.dist.p : nullptr;
     a.N0 = R.hN[0].p; a.N1 = R.hN[1].p; a.N2 = R.hN[2].p;
     a.Y0 = R.hY[0].p; a.Y1 = R.hY[1].p; a.Y2 = R.hY[2].p;
     a.F0 = R.hF[0].p; a.F1 = R.hF[1].p; a.F2 = R.hF[2].p; a.uN = R.huN.p; a.gp = R.gp.p;

@@ -14,8 +14,8 @@
 //     old index and the new state written at its new index. Both follow slot
 //     order, so state reads and writes stream through HBM.
 // The state of a real contact is L6Geom.trsf columns 0 and 1 (column 2 is
-// always col0 x col1), local force, uN, and the 64-byte gather record (global
-// force on pA, contact point, cellDist) that the force gather reads.
+// always col0 x col1), local force, uN, and the 48-byte gather record (global
+// force on pA, contact point) that the force gather reads.
 #include "wdg_internal.hpp"
 #include "wdg_math.hpp"
 #include "wdg_math32.hpp"
@@ -32,7 +32,6 @@ struct ContactArgs {
   double *N0, *N1, *N2, *Y0, *Y1, *Y2, *F0, *F1, *F2, *uN, *gp;
   unsigned long long* nbits;
   uint32_t *ntpre, *ngcnt;
-  uint32_t* act;
   uint32_t* sidx;  // state index of each real slot of the new set
   const uint32_t* osidx;  // the same for the old set, when its filter made it (else null)
   uint4* desc;           // per new state index: info, pA, pB, old state index (or NO_STATE)
@@ -194,8 +193,8 @@ struct SlotD {
 // is given) the slot of every state index, the state index of every real slot and the
 // force pass's record. running = real slots of the group so far.
 __device__ __forceinline__ void group_pass(int64_t c, bool keep, int64_t base, uint32_t& running,
-                                           unsigned long long* bits, uint32_t* tpre, uint32_t* act,
-                                           uint32_t* sidx, const SlotD& d = SlotD{}, uint4* desc = nullptr,
+                                           unsigned long long* bits, uint32_t* tpre, uint32_t* sidx,
+                                           const SlotD& d = SlotD{}, uint4* desc = nullptr,
                                            uint64_t* descDist = nullptr) {
   __shared__ uint32_t wc[GROUP_BS / 64];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -212,10 +211,9 @@ __device__ __forceinline__ void group_pass(int64_t c, bool keep, int64_t base, u
     tot += x;
   }
   if (lane == 0 && (wv & 3) == 0) tpre[c >> 8] = running + wpre;
-  if (keep && act) {
+  if (keep && sidx) {
     const unsigned long long lt = lane ? (~0ull >> (64 - lane)) : 0ull;
     const uint32_t st = state_index((uint32_t)(base / GROUP), running + wpre + (uint32_t)__popcll(b & lt));
-    act[st] = (uint32_t)c;
     sidx[c] = st;
     desc[st] = make_uint4(d.info, d.pA, d.pB, d.ko);
     if (descDist) descDist[st] = d.cd;
@@ -321,7 +319,9 @@ __device__ __forceinline__ bool filter_slot(const ContactArgs& a, int64_t c, Slo
 // after it and sets the step's trsfRenorm flag. The leapfrog counts the step when it ran.
 __device__ __forceinline__ bool step_skipped(const ContactArgs& a) {
   if (!a.gs) return false;
-  const bool skip = a.gs[0] != 0u || (a.gs[6] == 0u && (*a.dirtyPrev != 0u || a.dflags[1] != 0u));
+  // (all the words at once, not one after the other)
+  const uint32_t stop = a.gs[0], first = a.gs[6], dirty = *a.dirtyPrev, err = a.dflags[1];
+  const bool skip = (stop != 0u) | ((first == 0u) & ((dirty | err) != 0u));
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (skip) {
       a.gs[0] = 1u;
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(GROUP_BS) void k_cfilter(ContactArgs a) {
   uint32_t running = 0;
 #pragma unroll
   for (int pass = 0; pass < NP; pass++)
-    group_pass(base + pass * GROUP_BS + threadIdx.x, keep[pass], base, running, a.nbits, a.ntpre, a.act, a.sidx,
+    group_pass(base + pass * GROUP_BS + threadIdx.x, keep[pass], base, running, a.nbits, a.ntpre, a.sidx,
                d[pass], a.desc, PERIODIC ? a.descDist : nullptr);
   if (threadIdx.x == 0) a.ngcnt[g] = running;
   if (a.eidx) eidx_tail<NP>(a, base, wk);
@@ -376,7 +376,9 @@ __device__ __forceinline__ void stage_materials(const ContactArgs& a, wdg_materi
   __syncthreads();
 }
 __device__ __forceinline__ wdg_material material(const ContactArgs& a, const wdg_material* smat, uint32_t m) {
-  return m < (uint32_t)MAT_LDS ? smat[m] : a.mats[m];
+  wdg_material r = smat[m < (uint32_t)MAT_LDS ? m : 0u];
+  if (m >= (uint32_t)MAT_LDS) r = a.mats[m];
+  return r;
 }
 
 // Law2_L6Geom_FrictPhys_IdealElPl with rolling and twisting resistance (an internal law code)
@@ -419,24 +421,46 @@ __device__ __forceinline__ void en_clear(const ContactArgs& a, int64_t k) {
   e2[1] = make_double2(0., 0.);
 }
 
-template <bool PERIODIC, int LAW, bool FACETS, bool ENERGY>
+// The state arrays are read and written once per step, at consecutive addresses. Where the sets of
+// before and after the step do not fit the 256 MB last-level cache, they go past it, which so keeps
+// what is read again (particles, the filter's records, gather records): a step of 1M spheres (1.4M
+// contacts) is 3.4% faster; below that the next step finds its state there: past the cache, steps
+// of 20,000 and of 200,000 spheres were 2% slower. The FP32 form's sets are half as large and keep to
+// ordinary accesses (250,000 spheres: 7% slower past the cache).
+constexpr int64_t STREAM_SLOTS = (256ll << 20) / (2 * 10 * 8);
+template <bool STREAM, class T>
+__device__ __forceinline__ T state_load(const T* p) {
+  return STREAM ? __builtin_nontemporal_load(p) : *p;
+}
+template <bool STREAM, class T>
+__device__ __forceinline__ void state_store(T* p, T v) {
+  if (STREAM) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
+template <bool PERIODIC, int LAW, bool FACETS, bool ENERGY, bool STREAM>
 __global__ __launch_bounds__(CF_BS, FACETS ? 3 : 4) void k_cforce(ContactArgs a) {
   __shared__ wdg_material smat[MAT_LDS];
-  if (a.gstop && *a.gstop) return;
-  stage_materials(a, smat);
+  // the words that the step hangs on and the first record are loaded side by side: two waits on
+  // memory before the contact's own loads instead of four
+  const uint32_t stop = a.gstop ? *a.gstop : 0u;
   const int renorm = a.renormPtr ? (int)*a.renormPtr : a.renorm;
   const uint32_t lb = xcd_block(blockIdx.x, gridDim.x);
   const uint32_t nblk = (uint32_t)a.cfBlocks;
   const int64_t g = lb / nblk;
   const uint32_t cnt = a.ngcnt[g];
+  const uint32_t loc0 = (lb % nblk) * CF_BS + threadIdx.x;  // < GROUP: desc has a place for every slot
+  uint4 dk = a.desc[state_index((uint32_t)g, loc0)];
+  if (stop) return;
+  stage_materials(a, smat);
   double en[4] = {0., 0., 0., 0.};
   // the filter has written the entries of every real slot
   if (a.eidx && blockIdx.x == 0 && threadIdx.x == 0) a.dflags[EIDX_FULL] = 0u;
-  for (uint32_t loc = (lb % nblk) * CF_BS + threadIdx.x; loc < cnt; loc += CF_BS * nblk) {
+  for (uint32_t loc = loc0; loc < cnt; loc += CF_BS * nblk) {
     const int64_t k = state_index((uint32_t)g, loc);
     if (ENERGY && a.enC) en_clear(a, k);
     // the filter's record of the slot: type bits, particles in role order, old state index
-    const uint4 dk = a.desc[k];
+    if (loc != loc0) dk = a.desc[k];
     const uint32_t info = dk.x, pA = dk.y, pB = dk.z;
     const bool real = dk.w != NO_STATE;
     const uint32_t ko = real ? dk.w : 0u;
@@ -459,9 +483,9 @@ __global__ __launch_bounds__(CF_BS, FACETS ? 3 : 4) void k_cforce(ContactArgs a)
       matA += ep * (uint32_t)a.nMats;
       matB += ep * (uint32_t)a.nMats;
     }
-    const d3 prevNormalL = mk3(a.oN0[ko], a.oN1[ko], a.oN2[ko]);
-    const d3 prevYL = mk3(a.oY0[ko], a.oY1[ko], a.oY2[ko]);
-    const double oFt0 = a.oF1[ko], oFt1 = a.oF2[ko];
+    const d3 prevNormalL = mk3(state_load<STREAM>(&a.oN0[ko]), state_load<STREAM>(&a.oN1[ko]), state_load<STREAM>(&a.oN2[ko]));
+    const d3 prevYL = mk3(state_load<STREAM>(&a.oY0[ko]), state_load<STREAM>(&a.oY1[ko]), state_load<STREAM>(&a.oY2[ko]));
+    const double oFt0 = state_load<STREAM>(&a.oF1[ko]), oFt1 = state_load<STREAM>(&a.oF2[ko]);
     const double* og = a.ogp + (int64_t)GP * ko;
     const double2 ogc = reinterpret_cast<const double2*>(og)[2];
     const d3 prevContPtL = mk3(og[3], ogc.x, ogc.y);
@@ -661,10 +685,10 @@ __global__ __launch_bounds__(CF_BS, FACETS ? 3 : 4) void k_cforce(ContactArgs a)
         en_add(a, en, k, 0, kn0 * (2 / 5.) * ((q * q) * s) + 0.5 * (Ft0 * Ft0 + Ft1 * Ft1) / kt);
       }
     }
-    a.N0[k] = T0.x; a.N1[k] = T0.y; a.N2[k] = T0.z;
-    a.Y0[k] = T1.x; a.Y1[k] = T1.y; a.Y2[k] = T1.z;
-    a.F0[k] = Fn; a.F1[k] = Ft0; a.F2[k] = Ft1;
-    a.uN[k] = uN;
+    state_store<STREAM>(&a.N0[k], T0.x); state_store<STREAM>(&a.N1[k], T0.y); state_store<STREAM>(&a.N2[k], T0.z);
+    state_store<STREAM>(&a.Y0[k], T1.x); state_store<STREAM>(&a.Y1[k], T1.y); state_store<STREAM>(&a.Y2[k], T1.z);
+    state_store<STREAM>(&a.F0[k], Fn); state_store<STREAM>(&a.F1[k], Ft0); state_store<STREAM>(&a.F2[k], Ft1);
+    state_store<STREAM>(&a.uN[k], uN);
     // Contact::getForceTorqueBranch: F = node.ori * force, node.ori = Quaternion(trsf)
     const q4 q = quat_from_cols(T0, T1, T2);
     const d3 G = quat_rot(q, mk3(Fn, Ft0, Ft1));
@@ -672,7 +696,6 @@ __global__ __launch_bounds__(CF_BS, FACETS ? 3 : 4) void k_cforce(ContactArgs a)
     g2[0] = make_double2(G.x, G.y);
     g2[1] = make_double2(G.z, contPt.x);
     g2[2] = make_double2(contPt.y, contPt.z);
-    g2[3] = make_double2(__longlong_as_double((long long)cd), 0.);
     if (LAW == LAW_IEP_ROLL) {
       // Contact::getForceTorqueBranch: T = node.ori * torque, zero when the torque is zero
       const bool tz = tq.x == 0. && tq.y == 0. && tq.z == 0.;
@@ -776,7 +799,7 @@ __global__ __launch_bounds__(GROUP_BS) void k_cfilter32(ContactArgs a) {
   uint32_t running = 0;
 #pragma unroll
   for (int pass = 0; pass < NP; pass++)
-    group_pass(base + pass * GROUP_BS + threadIdx.x, keep[pass], base, running, a.nbits, a.ntpre, a.act, a.sidx,
+    group_pass(base + pass * GROUP_BS + threadIdx.x, keep[pass], base, running, a.nbits, a.ntpre, a.sidx,
                d[pass], a.desc, PERIODIC ? a.descDist : nullptr);
   if (threadIdx.x == 0) a.ngcnt[g] = running;
   if (a.eidx) eidx_tail<NP>(a, base, wk);
@@ -793,12 +816,13 @@ __global__ __launch_bounds__(CF_BS, 4) void k_cforce32(ContactArgs a) {
         *N2 = reinterpret_cast<float*>(a.N2), *Y0 = reinterpret_cast<float*>(a.Y0), *Y1 = reinterpret_cast<float*>(a.Y1),
         *Y2 = reinterpret_cast<float*>(a.Y2), *F0 = reinterpret_cast<float*>(a.F0), *F1 = reinterpret_cast<float*>(a.F1),
         *F2 = reinterpret_cast<float*>(a.F2), *UN = reinterpret_cast<float*>(a.uN), *gp = reinterpret_cast<float*>(a.gp);
-  if (a.gstop && *a.gstop) return;
+  const uint32_t stop = a.gstop ? *a.gstop : 0u;
   const int renorm = a.renormPtr ? (int)*a.renormPtr : a.renorm;
   const uint32_t lb = xcd_block(blockIdx.x, gridDim.x);
   const uint32_t nblk = (uint32_t)a.cfBlocks;
   const int64_t g = lb / nblk;
   const uint32_t cnt = a.ngcnt[g];
+  if (stop) return;
   // energy terms from the float law's values, evaluated and summed in FP64
   double en[4] = {0., 0., 0., 0.};
   if (a.eidx && blockIdx.x == 0 && threadIdx.x == 0) a.dflags[EIDX_FULL] = 0u;
@@ -1032,7 +1056,6 @@ static ContactArgs contact_args(Ctx& c, int from, int to) {
   a.nbits = N.bits.p;
   a.ntpre = N.tpre.p;
   a.ngcnt = N.gcnt.p;
-  a.act = c.act.p;
   a.sidx = N.sidx.p;
   a.osidx = O.sidxValid ? O.sidx.p : nullptr;
   a.desc = c.desc.p;
@@ -1210,7 +1233,7 @@ void eidx_clear(Ctx& c) {
   WDG_LAUNCH_CHECK();
 }
 
-template <bool E>
+template <bool E, bool S>
 static void launch_cforce(Ctx& c, const ContactArgs& a, dim3 grid, bool f32, bool hertz, bool roll, bool per,
                           bool fac) {
   const dim3 block(CF_BS);
@@ -1226,17 +1249,17 @@ static void launch_cforce(Ctx& c, const ContactArgs& a, dim3 grid, bool f32, boo
     }
   } else {
     if (hertz) {
-      if (per) hipLaunchKernelGGL((k_cforce<true, WDG_LAW_HERTZDMT, false, E>), grid, block, 0, c.stream, a);
-      else if (fac) hipLaunchKernelGGL((k_cforce<false, WDG_LAW_HERTZDMT, true, E>), grid, block, 0, c.stream, a);
-      else hipLaunchKernelGGL((k_cforce<false, WDG_LAW_HERTZDMT, false, E>), grid, block, 0, c.stream, a);
+      if (per) hipLaunchKernelGGL((k_cforce<true, WDG_LAW_HERTZDMT, false, E, S>), grid, block, 0, c.stream, a);
+      else if (fac) hipLaunchKernelGGL((k_cforce<false, WDG_LAW_HERTZDMT, true, E, S>), grid, block, 0, c.stream, a);
+      else hipLaunchKernelGGL((k_cforce<false, WDG_LAW_HERTZDMT, false, E, S>), grid, block, 0, c.stream, a);
     } else if (roll) {
-      if (per) hipLaunchKernelGGL((k_cforce<true, LAW_IEP_ROLL, false, E>), grid, block, 0, c.stream, a);
-      else if (fac) hipLaunchKernelGGL((k_cforce<false, LAW_IEP_ROLL, true, E>), grid, block, 0, c.stream, a);
-      else hipLaunchKernelGGL((k_cforce<false, LAW_IEP_ROLL, false, E>), grid, block, 0, c.stream, a);
+      if (per) hipLaunchKernelGGL((k_cforce<true, LAW_IEP_ROLL, false, E, S>), grid, block, 0, c.stream, a);
+      else if (fac) hipLaunchKernelGGL((k_cforce<false, LAW_IEP_ROLL, true, E, S>), grid, block, 0, c.stream, a);
+      else hipLaunchKernelGGL((k_cforce<false, LAW_IEP_ROLL, false, E, S>), grid, block, 0, c.stream, a);
     } else {
-      if (per) hipLaunchKernelGGL((k_cforce<true, WDG_LAW_IDEALELPL, false, E>), grid, block, 0, c.stream, a);
-      else if (fac) hipLaunchKernelGGL((k_cforce<false, WDG_LAW_IDEALELPL, true, E>), grid, block, 0, c.stream, a);
-      else hipLaunchKernelGGL((k_cforce<false, WDG_LAW_IDEALELPL, false, E>), grid, block, 0, c.stream, a);
+      if (per) hipLaunchKernelGGL((k_cforce<true, WDG_LAW_IDEALELPL, false, E, S>), grid, block, 0, c.stream, a);
+      else if (fac) hipLaunchKernelGGL((k_cforce<false, WDG_LAW_IDEALELPL, true, E, S>), grid, block, 0, c.stream, a);
+      else hipLaunchKernelGGL((k_cforce<false, WDG_LAW_IDEALELPL, false, E, S>), grid, block, 0, c.stream, a);
     }
   }
   WDG_LAUNCH_CHECK();
@@ -1279,7 +1302,6 @@ void contact_loop(Ctx& c, const wdg_contact_params* p) {
   c.R[to].ensure(C.n);
   if (roll) c.R[to].ensureRoll(C.n);
   const int64_t ng = ngroups(C.n);
-  c.act.ensure(ng * GROUP);
   c.desc.ensure(ng * GROUP);
   if (c.field.periodic) c.descDist.ensure(ng * GROUP);
   ContactArgs a = contact_args(c, from, to);
@@ -1329,16 +1351,17 @@ void contact_loop(Ctx& c, const wdg_contact_params* p) {
     // per contact, summed per scene once the new real set is current (below)
     energy_scenes_prepare(c, C.n);
     a.enC = c.enC.p;
-    launch_cforce<true>(c, a, gforce, c.precision == 32, hertz, roll, per, fac);
+    launch_cforce<true, false>(c, a, gforce, c.precision == 32, hertz, roll, per, fac);
   } else if (c.trackEnergy) {
     c.enPart.ensure((size_t)4 * gforce.x);
     a.enPart = c.enPart.p;
-    launch_cforce<true>(c, a, gforce, c.precision == 32, hertz, roll, per, fac);
+    launch_cforce<true, false>(c, a, gforce, c.precision == 32, hertz, roll, per, fac);
     // EnergyTracker: elast is resettable (this step's sum replaces it), the dissipations accumulate
     static const int tgt[4] = {WDG_EN_ELAST, WDG_EN_PLAST, WDG_EN_VISCN, WDG_EN_VISCT};
     energy_add(c, gforce.x, 4, tgt, 1);
   } else {
-    launch_cforce<false>(c, a, gforce, c.precision == 32, hertz, roll, per, fac);
+    if (C.n > STREAM_SLOTS) launch_cforce<false, true>(c, a, gforce, c.precision == 32, hertz, roll, per, fac);
+    else launch_cforce<false, false>(c, a, gforce, c.precision == 32, hertz, roll, per, fac);
   }
   // ContactLoop.evalStress (ContactLoop.cpp:123): the stress of this loop's real contacts, in
   // periodic cells (gradV is zero, so there is no gradV work to add)
@@ -1372,7 +1395,7 @@ __global__ __launch_bounds__(GROUP_BS) void k_flag_bits(int64_t nc, const uint32
   uint32_t running = 0;
   for (int pass = 0; pass < GROUP / GROUP_BS; pass++) {
     const int64_t c = base + pass * GROUP_BS + threadIdx.x;
-    group_pass(c, c < nc && flag[c] != 0u, base, running, bits, tpre, nullptr, nullptr);
+    group_pass(c, c < nc && flag[c] != 0u, base, running, bits, tpre, nullptr);
   }
   if (threadIdx.x == 0) gcnt[blockIdx.x] = running;
 }

@@ -109,7 +109,6 @@ static void size_buffers(Ctx& c, const wdg_program* prog) {
     c.R[0].ensureRoll(nc);
     c.R[1].ensureRoll(nc);
   }
-  c.act.ensure(ngroups(nc) * GROUP);
   c.desc.ensure(ngroups(nc) * GROUP);
   if (c.field.periodic) c.descDist.ensure(ngroups(nc) * GROUP);
   if (c.trackEnergy)

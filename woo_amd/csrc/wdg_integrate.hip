@@ -27,6 +27,7 @@ struct GatherArgs {
   RealView rv;
   const double* gp;
   const double* gtq;  // global phys torque per real contact (rolling resistance), else null
+  const uint64_t* descDist;  // packed cellDist per real contact (periodic cells)
   double L[3];
 };
 
@@ -48,14 +49,15 @@ __device__ __forceinline__ void gather_one(const GatherArgs& g, uint32_t e, d3 p
       T = add3(T, cross3(xc, Fc));
       return;
     }
-    const double2* r = reinterpret_cast<const double2*>(g.gp + (int64_t)GP * rv_index(g.rv, slot));
+    const uint32_t q = rv_index(g.rv, slot);
+    const double2* r = reinterpret_cast<const double2*>(g.gp + (int64_t)GP * q);
     const double2 r0 = r[0], r1 = r[1], r2 = r[2];
     const bool isPA = (e & ADJ_PA) != 0u;
     const double sign = isPA ? 1. : -1.;
     const d3 Fc = mul3(mk3(r0.x, r0.y, r1.x), sign);
     d3 shift = mk3(0., 0., 0.);
     if (PERIODIC && !isPA) {
-      const uint64_t cd = (uint64_t)__double_as_longlong(r[3].x);
+      const uint64_t cd = g.descDist[q];
       shift = mk3(g.L[0] * unpack_cd(cd, 0), g.L[1] * unpack_cd(cd, 1), g.L[2] * unpack_cd(cd, 2));
     }
     // Contact::getForceTorqueBranch: xc = contact point - (node pos + periodic shift of pB)
@@ -63,7 +65,7 @@ __device__ __forceinline__ void gather_one(const GatherArgs& g, uint32_t e, d3 p
     F = add3(F, Fc);
     if (g.gtq) {
       // applyForceUninodal: xc x F + T, T the phys torque (rolling resistance) times the sign
-      const double* t = g.gtq + (int64_t)3 * rv_index(g.rv, slot);
+      const double* t = g.gtq + (int64_t)3 * q;
       T = add3(T, add3(cross3(xc, Fc), mul3(mk3(t[0], t[1], t[2]), sign)));
     } else {
       T = add3(T, cross3(xc, Fc));
@@ -88,7 +90,7 @@ __device__ __forceinline__ void gather_record(const GatherArgs& g, uint32_t q, b
     const d3 Fc = mul3(mk3(r0.x, r0.y, r1.x), isPA ? 1. : -1.);
     d3 shift = mk3(0., 0., 0.);
     if (PERIODIC && !isPA) {
-      const uint64_t cd = (uint64_t)__double_as_longlong(r[3].x);
+      const uint64_t cd = g.descDist[q];
       shift = mk3(g.L[0] * unpack_cd(cd, 0), g.L[1] * unpack_cd(cd, 1), g.L[2] * unpack_cd(cd, 2));
     }
     // Contact::getForceTorqueBranch: xc = contact point - (node pos + periodic shift of pB)
@@ -514,7 +516,7 @@ __global__ __launch_bounds__(FN_BS) void k_facet_nodes(GatherArgs g, const doubl
         Fc = mul3(mk3(r0.x, r0.y, r1.x), isPA ? 1. : -1.);
         cp = mk3(r1.y, r2.x, r2.y);
         if (PERIODIC && !isPA) {
-          const uint64_t cd = (uint64_t)__double_as_longlong(r[3].x);
+          const uint64_t cd = g.descDist[q];
           shift = mk3(g.L[0] * unpack_cd(cd, 0), g.L[1] * unpack_cd(cd, 1), g.L[2] * unpack_cd(cd, 2));
         }
         if (g.gtq) {
@@ -559,6 +561,7 @@ static GatherArgs gather_args(Ctx& c) {
   g.sidx = c.reals().sidxValid ? c.reals().sidx.p : nullptr;
   g.eidx = c.eidxValid ? C.eidx.p : nullptr;
   g.nW = c.nW;
+  g.descDist = c.descDist.p;
   if (c.gated) g.gstop = c.gstate.p;
   for (int k = 0; k < 3; k++) g.L[k] = c.field.cell[k];
   return g;

@@ -152,7 +152,7 @@ constexpr int GROUP = 2048;   // slots per group (8 tiles)
 constexpr int GROUP_BS = 1024;  // threads of a group kernel
 inline int64_t ntiles(int64_t nslots) { return (nslots + TILE - 1) / TILE; }
 inline int64_t ngroups(int64_t nslots) { return (nslots + GROUP - 1) / GROUP; }
-constexpr int GP = 8;         // doubles per gather record (FP64 contact form)
+constexpr int GP = 6;         // doubles per gather record (FP64 contact form)
 constexpr int GP32 = 12;      // floats per gather record (FP32 contact form)
 struct Reals {
   DBuf<unsigned long long> bits;  // 64 words per group
@@ -161,7 +161,7 @@ struct Reals {
   DBuf<double> hN[3], hY[3];      // L6Geom.trsf columns 0 and 1
   DBuf<double> hF[3];             // CPhys.force, local frame
   DBuf<double> huN;               // L6Geom.uN
-  // gather record per contact: global force on pA (3), contact point (3), cellDist bits, unused
+  // gather record per contact: global force on pA (3), contact point (3)
   DBuf<double> gp;
   // material table (epoch) each real contact takes its phys from, while more than one is kept
   DBuf<uint8_t> hE;
@@ -357,7 +357,7 @@ struct Ctx {
   DBuf<uint32_t> scanTicket;
   uint32_t scanEpoch = 0, scanTickets = 0;
   DBuf<uint32_t> cellCnt, cellRank;  // spheres per cell, each sphere's place in its cell's count
-  DBuf<uint32_t> act;     // slot of each state index (contact loop), per-slot flags (relaxation)
+  DBuf<uint32_t> act;     // per-slot flags (relaxation)
   DBuf<uint4> desc;       // contact loop: the filter's record of each real slot, by state index
   DBuf<uint64_t> descDist;
   // in-memory snapshots of the kinematic state (pos, vel, angVel, ori; 13 doubles per
