@@ -183,3 +183,76 @@ def test_steps_ahead_equal_engine_calls(n, flat, steps, track):
     assert sa["nSteps"] == sb["nSteps"] and sa["nRefresh"] == sb["nRefresh"]
     if flat:
         assert sa["nCandidates"] > 2 * 2048
+
+
+def _network_graph(rng, N, kind):
+    # both directions of every pair, by receiver; "hub": node 0 exchanges with everyone; "double":
+    # pairs twice, with opposite edges that are not each other's opposite
+    pairs = {(i, (i + d) % N) for i in range(N) for d in (1, 2, 5) if (i + d) % N != i} if N > 1 else set()
+    pairs = {(min(p), max(p)) for p in pairs if rng.random() < .7}
+    if kind == "hub":
+        pairs |= {(0, j) for j in range(1, N)}
+    p = np.array(sorted(pairs), dtype=np.int64).reshape(-1, 2)
+    if kind == "double":
+        p = np.repeat(p, 2, axis=0)
+    n = len(p)
+    recv, send = np.concatenate([p[:, 0], p[:, 1]]), np.concatenate([p[:, 1], p[:, 0]])
+    back = np.concatenate([np.arange(n) + n, np.arange(n)])
+    if kind == "double":  # the second half's opposites are swapped within each pair of edges
+        back[n:] = back[n:] ^ 1
+    o = np.argsort(recv, kind="stable")
+    at = np.empty(2 * n, dtype=np.int64)
+    at[o] = np.arange(2 * n)
+    return (np.concatenate([[0], np.cumsum(np.bincount(recv, minlength=N))]), send[o], at[back[o]],
+            rng.normal(size=(N, 7)), rng.normal(size=(2 * n, 15)), rng.normal(size=(N, 3)))
+
+
+@pytest.mark.parametrize("N,kind", [(1, ""), (2, ""), (16, ""), (17, "hub"), (70, "hub"), (63, "double"), (2100, "")])
+def test_network_at_tile_edges(N, kind):
+    # partly filled wavefronts, nodes without edges and with more than a tile of them, a caller's graph
+    # whose rev is not an involution
+    from oracle.mpnn import Net, layout
+    from tests.test_mpnn_oracle import random_params
+    from woo_amd.surrogate import A0, Graph, Network
+
+    f32 = lambda a: np.asarray(a, dtype=np.float32).astype(np.float64)
+    rng = np.random.default_rng(100 + N)
+    rowOff, send, rev, x, ef, t = _network_graph(rng, N, kind)
+    p, x, ef, t = (f32(q) for q in (random_params(rng), x, ef, t))
+    x[:, 4] = np.where(np.arange(N) % 3 == 0, -1., x[:, 4])
+    net = Network(seed=1)
+    net.set_params(p)
+    g = Graph(rowOff, send, rev, x, ef)
+    out = net.predict(g) / A0
+    ref = Net(p, emulate=True)
+    a_cpu, _ = ref.forward(x, rowOff, send, ef)
+    # activations round to BF16 between the layers: values on a rounding boundary differ by 2^-8
+    assert np.max(np.abs(out - a_cpu)) <= 1e-2 * np.max(np.abs(a_cpu))
+    loss = net.loss_grad(g, t * A0)
+    grad = net.grads().astype(np.float64)
+    loss_cpu, grad_cpu = ref.loss_grad(x, rowOff, send, rev, ef, t)
+    assert abs(loss - loss_cpu) <= 1e-2 * loss_cpu
+    for name, (o, s) in layout()[0].items():
+        a, b = grad[o:o + s], grad_cpu[o:o + s]
+        assert np.linalg.norm(a - b) <= 2e-2 * np.linalg.norm(b), name
+
+
+def test_network_keeps_an_overflow_to_its_neighbours():
+    # a node whose messages overflow changes no output beyond the two rounds of messages
+    from tests.test_mpnn_oracle import random_params
+    from woo_amd.surrogate import Graph, Network
+
+    rng = np.random.default_rng(5)
+    N = 40
+    e = np.array([(i, j) for i in range(N) for j in (i - 1, i + 1) if 0 <= j < N])
+    rowOff = np.concatenate([[0], np.cumsum(np.bincount(e[:, 0], minlength=N))])
+    rev = np.array([np.flatnonzero((e[:, 0] == j) & (e[:, 1] == i))[0] for i, j in e])
+    x, ef = rng.normal(size=(N, 7)), rng.normal(size=(len(e), 15))
+    net = Network(seed=1)
+    net.set_params(np.asarray(random_params(rng), dtype=np.float32))
+    a = net.predict(Graph(rowOff, e[:, 1], rev, x, ef))
+    x[5] = 3e38 * np.sign(x[5])
+    b = net.predict(Graph(rowOff, e[:, 1], rev, x, ef))
+    far = np.abs(np.arange(N) - 5) > 2
+    np.testing.assert_array_equal(a[far], b[far])
+    assert not np.all(np.isfinite(b[~far])) or np.any(np.abs(b[~far]) > 1e30)

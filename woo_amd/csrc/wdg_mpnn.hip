@@ -15,13 +15,19 @@
 // Graph: edges in CSR by receiver (rowOff, recv, send), both directions of every pair, and
 // rev[e] = the opposite edge; every sum over edges follows this order (deterministic).
 //
-// GEMM tiling for 64-wide wavefronts: one wavefront computes a 16-row x 64-column block as
-// four 16x16 MFMA accumulators over K in steps of 32; lane l supplies row (l mod 16), 8
-// consecutive k from 8*(l/16) as one 16-byte load, gathered straight from the node and edge
-// arrays (the concatenated GEMM inputs are never stored). The weight-gradient GEMM reduces
-// over rows: each workgroup stages 32-row chunks of the input and of the output gradient in
-// LDS transposed, so that the MFMA operands are again 16-byte reads, and writes a partial;
-// a second kernel sums the partials in a fixed order.
+// Kernels: a wavefront owns 16 nodes and all the edges they receive. One kernel per layer forms the
+// messages, sums them and updates the nodes (k_layer); nothing per edge is written but, for
+// training, one 64-bit word of relu signs. Because the message GEMM is linear in its three inputs,
+// its backward needs no per-edge gradient either: with S1_i = sum of dY_e over the edges received
+// by i and S2_i over those sent by i (FP32 sums of the same BF16 values), the activation gradients
+// are S1 W_recv^T + S2 W_send^T and the weight gradients h^T S1, h^T S2: GEMMs over nodes, of which
+// there are seven times fewer. S1 and S2 enter the matrix cores as three BF16 terms that add up to
+// the FP32 value exactly.
+//
+// MFMA operands for 64-wide wavefronts (16x16x32): lane l supplies row (l mod 16) and 8 values of k
+// from group l/16. Which 8 k they are is free as long as both operands agree, so the result of one
+// product (rows 4*(l/16) + q) is fed to the next from registers, without a transpose through LDS:
+// messages to the segmented sum, the sum to the update, the update to the decoder.
 #include <algorithm>
 #include <cstring>
 #include <vector>
@@ -38,6 +44,8 @@ constexpr int H = 64;     // hidden width
 constexpr int KX = 32;    // node input columns (NIN used)
 constexpr int KE = 32;    // edge input columns (NEI used)
 constexpr int NIN = 7, NEI = 15;
+constexpr int XP = 8, EP = 16;  // stored columns of the node and edge inputs (the others are zero)
+constexpr int ONE = 15;         // free operand row of the input GEMMs: ones, for the bias gradient
 constexpr int KM = 2 * H + KE;  // message GEMM inner dimension (160)
 constexpr int KU = 2 * H;       // update GEMM inner dimension (128)
 constexpr int NOUT = 3;
@@ -126,396 +134,776 @@ struct PLayout {
   }
 };
 
-// ------------------------------------------------------------------ GEMM input rows
-enum { A_PLAIN = 0, A_EDGE = 1, A_UPD = 2 };
-struct ARows {
-  const bf16* x;      // A_PLAIN: [M x K] row-major
-  const bf16* h;      // A_EDGE / A_UPD: node activations [N x H]
-  const bf16* ef;     // A_EDGE: edge inputs [E x KE]
-  const bf16* agg;    // A_UPD: aggregated messages [N x H]
-  const int32_t *recv, *send;  // A_EDGE
-  int K;
-};
-// 8 consecutive inputs of row r starting at column k (k multiple of 8)
-template <int MODE>
-__device__ __forceinline__ uint4 load8(const ARows& a, int64_t r, int k) {
-  const bf16* p;
-  if (MODE == A_PLAIN) p = a.x + r * a.K + k;
-  else if (MODE == A_EDGE) {
-    if (k < H) p = a.h + (int64_t)a.recv[r] * H + k;
-    else if (k < 2 * H) p = a.h + (int64_t)a.send[r] * H + (k - H);
-    else p = a.ef + r * KE + (k - 2 * H);
-  } else {
-    if (k < H) p = a.h + r * H + k;
-    else p = a.agg + r * H + (k - H);
-  }
-  return *reinterpret_cast<const uint4*>(p);
-}
 __device__ __forceinline__ bf16x8 as_bf8(uint4 v) {
   bf16x8 r;
   memcpy(&r, &v, 16);
   return r;
 }
+__device__ __forceinline__ uint32_t pack2(bf16 lo, bf16 hi) { return (uint32_t)lo | ((uint32_t)hi << 16); }
+// two values rounded to nearest even in one instruction, the first in the low half
+__device__ __forceinline__ uint32_t cvt2(float lo, float hi) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  const b2 r = __builtin_convertvector((f2){lo, hi}, b2);
+  uint32_t u;
+  memcpy(&u, &r, 4);
+  return u;
+}
+__device__ __forceinline__ floatx4 mfma(uint4 a, uint4 b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(a), as_bf8(b), c, 0, 0, 0);
+}
+__device__ __forceinline__ uint4 row8(const bf16* p) { return *reinterpret_cast<const uint4*>(p); }
+// a relu's output is positive (it is never negative; -0 counts as zero)
+__device__ __forceinline__ bool on(uint32_t b) { return (b & 0x7FFFu) != 0u; }
+constexpr uint4 ZERO4 = {0u, 0u, 0u, 0u};
 
-// ------------------------------------------------------------------ forward GEMM
-// Y = relu(A W + b) over M rows, 64 columns. Out: y (BF16, M x 64). With RESID (update
-// layer): u = relu(.) to y, h_new = round(h + u) to hOut.
-// The workgroup stages the BF16 weight image in LDS once; each wavefront then walks 16-row
-// tiles of A (all K/32 row loads of a tile issued before its MFMAs), and writes each output
-// tile through its own LDS tile as 16-byte row stores.
-template <int MODE>
-constexpr int k_of() { return MODE == A_PLAIN ? KX : (MODE == A_EDGE ? KM : KU); }
-template <int MODE, bool RESID>
-__global__ __launch_bounds__(256) void k_mm_fwd(ARows a, int64_t M, const bf16* __restrict__ Wt,
-                                                 const float* __restrict__ bias, bf16* y, bf16* hOut) {
-  constexpr int K = k_of<MODE>(), KS = K / 32, WP = K + 8;  // padded LDS rows (bank spread)
-  __shared__ bf16 Ws[H * WP];
-  __shared__ bf16 tile[4][16][H + 8];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  // weight image [64 x K] into LDS, 16 bytes per thread and step
-  for (int i = threadIdx.x; i < H * K / 8; i += blockDim.x) {
-    const int col = i / (K / 8), k8 = (i % (K / 8)) * 8;
-    *reinterpret_cast<uint4*>(&Ws[col * WP + k8]) = *reinterpret_cast<const uint4*>(Wt + (int64_t)col * K + k8);
+// ------------------------------------------------------------------ encoder
+// h0 = relu(X W + b): the weights as the first operand, so that a lane ends with four consecutive
+// features of one node (8-byte stores)
+__global__ __launch_bounds__(256) void k_enc(int64_t N, const bf16* __restrict__ X, const bf16* __restrict__ Wt,
+                                              const float* __restrict__ bias, bf16* __restrict__ h) {
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int64_t i = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 16 + r;
+  uint4 x = row8(X + min(i, N - 1) * XP);
+  if (g != 0) x = ZERO4;  // columns 8 .. 31 are zero
+#pragma unroll
+  for (int cb = 0; cb < 4; cb++) {
+    const floatx4 b = *reinterpret_cast<const floatx4*>(bias + cb * 16 + 4 * g);
+    const floatx4 v = mfma(row8(Wt + (cb * 16 + r) * KX + 8 * g), x, b);
+    if (i < N)
+      *reinterpret_cast<uint2*>(h + i * H + cb * 16 + 4 * g) =
+          make_uint2(cvt2(fmaxf(v[0], 0.f), fmaxf(v[1], 0.f)), cvt2(fmaxf(v[2], 0.f), fmaxf(v[3], 0.f)));
   }
+}
+
+// ------------------------------------------------------------------ one layer, forward
+// messages m_e = relu([h_recv, h_send, F] Wm + bm), their sums, u = relu([h, agg] Wu + bu) and
+// h + u, for the 16 nodes of each wavefront; LAST: also the decoder and the contact flags.
+// 32 edges at a time: the message product leaves lane l with edges 4*(l/16) + q (of both halves)
+// of feature l mod 16, which is the operand of the segmented sum: a product with the 0/1 matrix
+// of edges and receivers, exact but for the order of an FP32 sum (the 0/1 operand comes from the
+// row offsets). A message that is not finite spreads over the wavefront's nodes there (0 * inf):
+// where a sum is not finite, the wavefront's edges are gone through again and summed one by one.
+// Bound by the chain of a chunk (end points, rows, 40 + 4 products, 20 LDS reads of weights) at three
+// wavefronts per SIMD: 120,000 nodes and 840,000 edges take 60 us a layer; the message product, the
+// sum and the update as kernels of their own took 67 + 23 + 15. Four wavefronts per SIMD spill
+// (78 us). Both weight images (39 KB, rows padded for the banks) are staged once per workgroup,
+// three of which fit a compute unit: 768 workgroups walk the tiles (1,024: 14% slower).
+struct LayerArgs {
+  int64_t N;
+  const int32_t *rowOff, *recv, *send;
+  const bf16 *h, *ef, *x, *Wm, *Wu;
+  const float *bm, *bu, *Wd, *bd;
+  bf16 *hOut, *agg;
+  uint64_t *mMask, *uMask;
+  float* out;
+  uint8_t* flag;
+};
+constexpr int LY_BS = 256;
+constexpr int WMP = KM + 8, WUP = KU + 8;  // padded LDS rows
+template <bool STORE, bool LAST>
+__global__ __launch_bounds__(LY_BS, 3) void k_layer(LayerArgs a) {
+  __shared__ __attribute__((aligned(16))) bf16 Wm[H * WMP];
+  __shared__ __attribute__((aligned(16))) bf16 Wu[H * WUP];
+  __shared__ float Wd[H * NOUT];
+  // (every load in flight before the first store)
+  {
+    constexpr int QM = H * KM / 8 / LY_BS, QU = H * KU / 8 / LY_BS;
+    static_assert(QM * LY_BS * 8 == H * KM && QU * LY_BS * 8 == H * KU, "whole passes over the images");
+    uint4 v[QM + QU];
+#pragma unroll
+    for (int q = 0; q < QM; q++) v[q] = row8(a.Wm + (q * LY_BS + threadIdx.x) * 8);
+#pragma unroll
+    for (int q = 0; q < QU; q++) v[QM + q] = row8(a.Wu + (q * LY_BS + threadIdx.x) * 8);
+#pragma unroll
+    for (int q = 0; q < QM; q++) {
+      const int i = q * LY_BS + threadIdx.x;
+      *reinterpret_cast<uint4*>(&Wm[i / (KM / 8) * WMP + i % (KM / 8) * 8]) = v[q];
+    }
+#pragma unroll
+    for (int q = 0; q < QU; q++) {
+      const int i = q * LY_BS + threadIdx.x;
+      *reinterpret_cast<uint4*>(&Wu[i / (KU / 8) * WUP + i % (KU / 8) * 8]) = v[QM + q];
+    }
+  }
+  if (LAST && threadIdx.x < H * NOUT) Wd[threadIdx.x] = a.Wd[threadIdx.x];
   __syncthreads();
-  const int kq = 8 * (lane >> 4);
-  float bv[4];
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  float bm[4];
 #pragma unroll
-  for (int cb = 0; cb < 4; cb++) bv[cb] = bias[cb * 16 + (lane & 15)];
-  const int64_t ntiles = (M + 15) / 16;
-  for (int64_t t = (int64_t)blockIdx.x * 4 + wv; t < ntiles; t += (int64_t)gridDim.x * 4) {
-    const int64_t r0 = t * 16;
-    const int64_t r = r0 + (lane & 15);
-    const bool live = r < M;
-    uint4 av[KS];
+  for (int cb = 0; cb < 4; cb++) bm[cb] = a.bm[cb * 16 + r];
+  const int64_t nt = (a.N + 15) / 16;
+  for (int64_t t = (int64_t)xcd_block(blockIdx.x, gridDim.x) * (LY_BS / 64) + (threadIdx.x >> 6); t < nt;
+       t += (int64_t)gridDim.x * (LY_BS / 64)) {
+    const bool node = t * 16 + r < a.N;
+    const int64_t i = node ? t * 16 + r : a.N - 1;
+    const int32_t b0 = a.rowOff[node ? i : a.N], b1 = a.rowOff[i + 1];
+    const int32_t e0 = __shfl(b0, 0), e1 = __shfl(b1, 15);
+    floatx4 agg[4];
+    bool touch = false;
+    for (int pass = 0; pass < 2; pass++) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) av[ks] = live ? load8<MODE>(a, r, ks * 32 + kq) : make_uint4(0, 0, 0, 0);
-    floatx4 acc[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+    for (int cb = 0; cb < 4; cb++) agg[cb] = floatx4{0, 0, 0, 0};
+    int32_t rc[2], sd[2];
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      const bf16x8 A = as_bf8(av[ks]);
+    for (int q = 0; q < 2; q++) {
+      const int32_t e = max(min(e0 + 16 * q + r, e1 - 1), 0);
+      rc[q] = e0 < e1 ? a.recv[e] : 0;
+      sd[q] = e0 < e1 ? a.send[e] : 0;
+    }
+    for (int32_t eb = e0; eb < e1; eb += 32) {
+      uint4 z[2][5];
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        // past the last edge: that edge again (it counts for no node below, and no load is
+        // conditional)
+        const int32_t e = min(eb + 16 * q + r, e1 - 1);
+        const int64_t er = rc[q], es = sd[q];
+        const int32_t en = min(eb + 32 + 16 * q + r, e1 - 1);  // the next ends, a chunk ahead
+        rc[q] = a.recv[en];
+        sd[q] = a.send[en];
+        z[q][4] = row8(a.ef + (int64_t)e * EP + 8 * (g & 1));
+        if (g >= 2) z[q][4] = ZERO4;  // columns 16 .. 31 are zero
+        z[q][0] = row8(a.h + er * H + 8 * g);
+        z[q][1] = row8(a.h + er * H + 32 + 8 * g);
+        z[q][2] = row8(a.h + es * H + 8 * g);
+        z[q][3] = row8(a.h + es * H + 32 + 8 * g);
+        if (LAST) {
+          // overlap inputs (column 3, in the lanes of group 0) of this half's edges, against the
+          // lane's node's range of them
+          const uint64_t pos = __ballot(bf2f((bf16)(z[q][4].y >> 16)) > 0.f) & 0xFFFFull;
+          const int lo = min(max(b0 - (eb + 16 * q), 0), 16), hi = min(max(b1 - (eb + 16 * q), 0), 16);
+          touch = touch || ((uint32_t)pos & ((1u << hi) - 1u) & ~((1u << lo) - 1u)) != 0u;
+        }
+      }
+      // (the weights stay in LDS: held in registers over the loop they would be spilled)
+      int wo = r * WMP + 8 * g;
+      asm volatile("" : "+v"(wo));
+      floatx4 acc[2][4];
+#pragma unroll
+      for (int cb = 0; cb < 4; cb++) acc[0][cb] = acc[1][cb] = floatx4{bm[cb], bm[cb], bm[cb], bm[cb]};
+#pragma unroll
+      for (int ks = 0; ks < 5; ks++) {
+        asm volatile("" ::: "memory");  // a step's weights at a time
+#pragma unroll
+        for (int cb = 0; cb < 4; cb++) {
+          const uint4 w = row8(&Wm[cb * 16 * WMP + ks * 32 + wo]);
+          acc[0][cb] = mfma(z[0][ks], w, acc[0][cb]);
+          acc[1][cb] = mfma(z[1][ks], w, acc[1][cb]);
+        }
+      }
+      // relu, rounded once
+      uint4 mv[4];
 #pragma unroll
       for (int cb = 0; cb < 4; cb++) {
-        const int col = cb * 16 + (lane & 15);
-        const bf16x8 B = as_bf8(*reinterpret_cast<const uint4*>(&Ws[col * WP + ks * 32 + kq]));
-        acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, acc[cb], 0, 0, 0);
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = fmaxf(acc[j >> 2][cb][j & 3], 0.f);
+        mv[cb] = make_uint4(cvt2(v[0], v[1]), cvt2(v[2], v[3]), cvt2(v[4], v[5]), cvt2(v[6], v[7]));
+      }
+      if (STORE) {
+        // sign words: bit 16 * cb + feature of edge 4 * (lane / 16) + q
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+          uint64_t word = 0;
+#pragma unroll
+          for (int cb = 0; cb < 4; cb++) {
+            const uint32_t w0 = q ? mv[cb].z : mv[cb].x, w1 = q ? mv[cb].w : mv[cb].y;
+            const uint64_t s0 = __ballot(on(w0)), s1 = __ballot(on(w0 >> 16)), s2 = __ballot(on(w1)),
+                           s3 = __ballot(on(w1 >> 16));
+            const uint64_t sq = (r & 2) ? ((r & 1) ? s3 : s2) : ((r & 1) ? s1 : s0);
+            word |= ((sq >> (16 * (r >> 2))) & 0xFFFFull) << (16 * cb);
+          }
+          const int32_t e = eb + 16 * q + r;
+          if (g == 0 && e < e1) a.mMask[e] = word;
+        }
+      }
+      // the 0/1 operand: node r against edges eb + 16 * (j / 4) + 4 * g + j % 4
+      const int lo = min(max(b0 - eb, 0), 32), hi = min(max(b1 - eb, 0), 32);
+      const uint32_t in = (uint32_t)((1ull << hi) - 1ull) & ~(uint32_t)((1ull << lo) - 1ull);
+      const uint32_t i0 = in >> (4 * g), i1 = i0 >> 16;
+      if (pass == 0) {
+        const uint4 sw = make_uint4((i0 & 1u) * 0x3F80u | (i0 >> 1 & 1u) * 0x3F800000u,
+                                    (i0 >> 2 & 1u) * 0x3F80u | (i0 >> 3 & 1u) * 0x3F800000u,
+                                    (i1 & 1u) * 0x3F80u | (i1 >> 1 & 1u) * 0x3F800000u,
+                                    (i1 >> 2 & 1u) * 0x3F80u | (i1 >> 3 & 1u) * 0x3F800000u);
+#pragma unroll
+        for (int cb = 0; cb < 4; cb++) agg[cb] = mfma(mv[cb], sw, agg[cb]);
+      } else {
+        for (int k = 0; k < 32; k++) {
+          // edge eb + k: group (k % 16) / 4, value 4 * (k / 16) + k % 4 of its lanes
+          const int kg = (k & 15) >> 2, j = 2 * (k >> 4) + ((k & 3) >> 1);
+          const bool mine = (in >> k) & 1u;
+#pragma unroll
+          for (int cb = 0; cb < 4; cb++) {
+            const uint32_t w = j == 0 ? mv[cb].x : (j == 1 ? mv[cb].y : (j == 2 ? mv[cb].z : mv[cb].w));
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+              const uint32_t o = __shfl(w, 16 * kg + 4 * g + q);
+              const float v = bf2f((bf16)((k & 1) ? o >> 16 : o & 0xFFFFu));
+              agg[cb][q] += mine ? v : 0.f;
+            }
+          }
+        }
       }
     }
-    // C layout: row 4*(lane/16)+q, column lane%16 of each block
+    bool fin = true;
+#pragma unroll
+    for (int cb = 0; cb < 4; cb++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) fin = fin && fabsf(agg[cb][q]) <= 3.402823466e38f;
+    if (__all(fin)) break;
+    }
+    // agg: features 16 * cb + 4 * g + q of node r, rounded once
+    uint2 ag[4];
+#pragma unroll
+    for (int cb = 0; cb < 4; cb++) ag[cb] = make_uint2(cvt2(agg[cb][0], agg[cb][1]), cvt2(agg[cb][2], agg[cb][3]));
+    if (STORE && node)
+#pragma unroll
+      for (int cb = 0; cb < 4; cb++) *reinterpret_cast<uint2*>(a.agg + i * H + cb * 16 + 4 * g) = ag[cb];
+    // update: the weights' columns in the order of the operand's features
+    uint4 hz[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) hz[ks] = row8(a.h + i * H + ks * 32 + 8 * g);
+    int uo = r * WUP + 4 * g;
+    asm volatile("" : "+v"(uo));
+    floatx4 up[4];
 #pragma unroll
     for (int cb = 0; cb < 4; cb++) {
-      const int col = cb * 16 + (lane & 15);
+      const bf16* w = &Wu[cb * 16 * WUP + uo];
+      floatx4 u = *reinterpret_cast<const floatx4*>(a.bu + cb * 16 + 4 * g);
 #pragma unroll
-      for (int q = 0; q < 4; q++) tile[wv][4 * (lane >> 4) + q][col] = f2bf(fmaxf(acc[cb][q] + bv[cb], 0.f));
-    }
-    wave_lds_sync();
+      for (int ks = 0; ks < 2; ks++) u = mfma(row8(w + ks * 32 + 4 * g), hz[ks], u);
 #pragma unroll
-    for (int half = 0; half < 2; half++) {
-      const int row = half * 8 + (lane >> 3), c0 = (lane & 7) * 8;
-      const int64_t rr = r0 + row;
-      if (rr >= M) continue;
-      const uint4 v = *reinterpret_cast<const uint4*>(&tile[wv][row][c0]);
-      *reinterpret_cast<uint4*>(y + rr * H + c0) = v;
-      if (RESID) {
-        const uint4 hv = *reinterpret_cast<const uint4*>(a.h + rr * H + c0);
-        const uint32_t uw[4] = {v.x, v.y, v.z, v.w}, hw[4] = {hv.x, hv.y, hv.z, hv.w};
-        uint32_t o[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const bf16 lo = f2bf(bf2f((bf16)(hw[q] & 0xFFFFu)) + bf2f((bf16)(uw[q] & 0xFFFFu)));
-          const bf16 hi = f2bf(bf2f((bf16)(hw[q] >> 16)) + bf2f((bf16)(uw[q] >> 16)));
-          o[q] = (uint32_t)lo | ((uint32_t)hi << 16);
-        }
-        *reinterpret_cast<uint4*>(hOut + rr * H + c0) = make_uint4(o[0], o[1], o[2], o[3]);
+      for (int ks = 0; ks < 2; ks++) {
+        const uint2 w0 = *reinterpret_cast<const uint2*>(w + H + ks * 32),
+                    w1 = *reinterpret_cast<const uint2*>(w + H + ks * 32 + 16);
+        u = mfma(make_uint4(w0.x, w0.y, w1.x, w1.y), make_uint4(ag[2 * ks].x, ag[2 * ks].y, ag[2 * ks + 1].x, ag[2 * ks + 1].y), u);
       }
+      up[cb] = u;
     }
-    // the tile is written again by the next iteration only after every lane has read it
-    wave_lds_sync();
-  }
-}
-// workgroups for a forward GEMM over M rows: enough wavefronts to fill the chip, each walking a
-// few tiles so that the weight staging is amortised
-static unsigned fwd_blocks(int64_t M) {
-  const int64_t tiles = (M + 15) / 16;
-  return (unsigned)std::max<int64_t>(1, std::min<int64_t>((tiles + 3) / 4, 1024));
-}
-
-// ------------------------------------------------------------------ input-gradient GEMM
-// dX[:, c] = sum_k dY[:, k] W[c, k] for output columns c < KOUT (W row-major [K x 64], BF16);
-// dY BF16 [M x 64]; dX FP32 [M x KOUT]
-template <int KOUT>
-__global__ __launch_bounds__(256) void k_mm_dx(const bf16* __restrict__ dY, int64_t M, const bf16* __restrict__ W,
-                                                float* dX) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int64_t r0 = ((int64_t)blockIdx.x * 4 + wv) * 16;
-  if (r0 >= M) return;
-  const int64_t r = r0 + (lane & 15);
-  const bool live = r < M;
-  const int kq = 8 * (lane >> 4);
-  constexpr int NB = KOUT / 16;
-  floatx4 acc[NB];
+    uint64_t um = 0;
+    float o[NOUT] = {0.f, 0.f, 0.f};
 #pragma unroll
-  for (int cb = 0; cb < NB; cb++) acc[cb] = floatx4{0, 0, 0, 0};
+    for (int cb = 0; cb < 4; cb++) {
+      const int f0 = cb * 16 + 4 * g;
+      const uint2 hw = *reinterpret_cast<const uint2*>(a.h + i * H + f0);
+      const bf16 hh[4] = {(bf16)(hw.x & 0xFFFFu), (bf16)(hw.x >> 16), (bf16)(hw.y & 0xFFFFu), (bf16)(hw.y >> 16)};
+      bf16 hn[4];
 #pragma unroll
-  for (int k0 = 0; k0 < H; k0 += 32) {
-    const uint4 av = live ? *reinterpret_cast<const uint4*>(dY + r * H + k0 + kq) : make_uint4(0, 0, 0, 0);
-    const bf16x8 A = as_bf8(av);
+      for (int q = 0; q < 4; q++) {
+        const bf16 u = f2bf(fmaxf(up[cb][q], 0.f));
+        um |= (uint64_t)(on(u) ? 1u : 0u) << (f0 + q);
+        hn[q] = f2bf(bf2f(hh[q]) + bf2f(u));
+        if (LAST)
 #pragma unroll
-    for (int cb = 0; cb < NB; cb++) {
-      const int col = cb * 16 + (lane & 15);
-      const bf16x8 B = as_bf8(*reinterpret_cast<const uint4*>(W + (int64_t)col * H + k0 + kq));
-      acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, acc[cb], 0, 0, 0);
+          for (int c = 0; c < NOUT; c++) o[c] += bf2f(hn[q]) * Wd[(f0 + q) * NOUT + c];
+      }
+      if (node && (STORE || !LAST))
+        *reinterpret_cast<uint2*>(a.hOut + i * H + f0) = make_uint2(pack2(hn[0], hn[1]), pack2(hn[2], hn[3]));
     }
-  }
+    if (STORE) {
+      um |= (uint64_t)__shfl_xor((unsigned long long)um, 16);
+      um |= (uint64_t)__shfl_xor((unsigned long long)um, 32);
+      if (node && g == 0) a.uMask[i] = um;
+    }
+    if (LAST) {
 #pragma unroll
-  for (int cb = 0; cb < NB; cb++) {
-    const int col = cb * 16 + (lane & 15);
+      for (int c = 0; c < NOUT; c++) {
+        o[c] += __shfl_xor(o[c], 16);
+        o[c] += __shfl_xor(o[c], 32);
+      }
+      // a node is in contact when its floor overlap input or the overlap input of one of its edges
+      // is positive. Nodes not in contact move in free flight (the network's output is not used for
+      // them), so they carry no loss.
+      if (node && g == 0) {
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int64_t rr = r0 + 4 * (lane >> 4) + q;
-      if (rr < M) dX[rr * KOUT + col] = acc[cb][q];
+        for (int c = 0; c < NOUT; c++) a.out[i * NOUT + c] = a.bd[c] + o[c];
+        a.flag[i] = touch || bf2f(a.x[i * XP + 4]) > 0.f ? 1 : 0;
+      }
     }
   }
 }
 
-// ------------------------------------------------------------------ weight-gradient GEMM
-// partial[blk][c][o] = sum over the workgroup's rows m of A[m][c] dY[m][o]; partialB[blk][o]
-// = sum of dY[m][o] (bias gradient). Rows in chunks of 32, staged transposed in LDS.
-constexpr int DW_CHUNKS = 8;  // 32-row chunks per workgroup
-template <int MODE, int KP>
-__global__ __launch_bounds__(256) void k_mm_dw(ARows a, int64_t M, const bf16* __restrict__ dY, float* partial,
-                                                float* partialB) {
-  __shared__ __attribute__((aligned(16))) bf16 At[KP][32 + 8];
-  __shared__ __attribute__((aligned(16))) bf16 Dt[H][32 + 8];
-  __shared__ float bsum[4][H];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  constexpr int TILES = (KP / 16) * (H / 16);
-  constexpr int TPW = (TILES + 3) / 4;  // output tiles per wavefront
-  floatx4 acc[TPW];
+// ------------------------------------------------------------------ loss and decoder, backward
+// loss = mean over nodes of |a - t|^2, dA = 2 (a - t) / N, dh = dA W^T, partials of dW (H x 3) and
+// db (3): DEC_ROWS nodes per workgroup, a feature per lane, DEC_ROWS / 4 nodes per wavefront
+// (25,000 nodes: 9 us; a reduction of the workgroup per feature took 68)
+constexpr int DEC_ROWS = 64, DECW = (H + 1) * NOUT;
+__global__ __launch_bounds__(256) void k_loss_dec(int64_t N, const float* __restrict__ a, const float* __restrict__ t,
+                                                   const uint8_t* __restrict__ flag, const bf16* __restrict__ h,
+                                                   const float* __restrict__ W, float* __restrict__ dh,
+                                                   float* __restrict__ part, float* __restrict__ partLoss) {
+  __shared__ float G[DEC_ROWS][NOUT + 1];
+  __shared__ float sm[4][H][NOUT];
+  const int64_t i0 = (int64_t)blockIdx.x * DEC_ROWS;
+  const int k = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  if (wv == 0) {
+    const int64_t i = i0 + k;
+    float l = 0.f;
 #pragma unroll
-  for (int t = 0; t < TPW; t++) acc[t] = floatx4{0, 0, 0, 0};
-  float bacc = 0.f;  // bias partial of column lane, rows of this wavefront's share
-  const int64_t rowBase = (int64_t)blockIdx.x * DW_CHUNKS * 32;
-  for (int ch = 0; ch < DW_CHUNKS; ch++) {
-    const int64_t m0 = rowBase + ch * 32;
-    if (m0 >= M) break;
-    // stage: 32 rows x KP inputs and 32 rows x 64 gradients, transposed
-    for (int idx = threadIdx.x; idx < 32 * (KP / 8); idx += 256) {
-      const int rr = idx / (KP / 8), k8 = (idx % (KP / 8)) * 8;
-      const int64_t m = m0 + rr;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (m < M) v = load8<MODE>(a, m, k8);
-      bf16 e[8];
-      memcpy(e, &v, 16);
-#pragma unroll
-      for (int q = 0; q < 8; q++) At[k8 + q][rr] = e[q];
+    for (int c = 0; c < NOUT; c++) {
+      const float x = a[min(i, N - 1) * NOUT + c] - t[min(i, N - 1) * NOUT + c];
+      const float d = i < N && flag[min(i, N - 1)] ? x : 0.f;
+      l += d * d;
+      G[k][c] = 2.f * d / (float)N;
     }
-    for (int idx = threadIdx.x; idx < 32 * (H / 8); idx += 256) {
-      const int rr = idx / (H / 8), k8 = (idx % (H / 8)) * 8;
-      const int64_t m = m0 + rr;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (m < M) v = *reinterpret_cast<const uint4*>(dY + m * H + k8);
-      bf16 e[8];
-      memcpy(e, &v, 16);
-#pragma unroll
-      for (int q = 0; q < 8; q++) Dt[k8 + q][rr] = e[q];
-    }
-    __syncthreads();
-    // bias: wavefront wv adds rows 8*wv .. 8*wv+7 of column lane
-#pragma unroll
-    for (int q = 0; q < 8; q++) bacc += bf2f(Dt[lane][8 * wv + q]);
-#pragma unroll
-    for (int t = 0; t < TPW; t++) {
-      const int tile = wv * TPW + t;
-      if (tile < TILES) {
-        const int cb = tile / (H / 16), ob = tile % (H / 16);
-        const int kq = 8 * (lane >> 4);
-        const bf16x8 A = as_bf8(*reinterpret_cast<const uint4*>(&At[cb * 16 + (lane & 15)][kq]));
-        const bf16x8 B = as_bf8(*reinterpret_cast<const uint4*>(&Dt[ob * 16 + (lane & 15)][kq]));
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, acc[t], 0, 0, 0);
-      }
-    }
-    __syncthreads();
+    for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
+    if (k == 0) partLoss[blockIdx.x] = l;
   }
-  float* P = partial + (int64_t)blockIdx.x * KP * H;
-#pragma unroll
-  for (int t = 0; t < TPW; t++) {
-    const int tile = wv * TPW + t;
-    if (tile < TILES) {
-      const int cb = tile / (H / 16), ob = tile % (H / 16);
-#pragma unroll
-      for (int q = 0; q < 4; q++) P[(cb * 16 + 4 * (lane >> 4) + q) * H + ob * 16 + (lane & 15)] = acc[t][q];
-    }
-  }
-  bsum[wv][lane] = bacc;
+  const float w[NOUT] = {W[k * NOUT], W[k * NOUT + 1], W[k * NOUT + 2]};
   __syncthreads();
-  if (threadIdx.x < H)
-    partialB[(int64_t)blockIdx.x * H + threadIdx.x] =
-        ((bsum[0][threadIdx.x] + bsum[1][threadIdx.x]) + bsum[2][threadIdx.x]) + bsum[3][threadIdx.x];
-}
-// grad[i] = sum over blocks of partial[blk][i], in block order
-__global__ void k_sum_partials(const float* __restrict__ partial, int64_t nblk, int64_t n, float* grad) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float s = 0.f;
-  for (int64_t b = 0; b < nblk; b++) s += partial[b * n + i];
-  grad[i] = s;
-}
-// first level of a two-level sum for many blocks: segment y of len blocks, in block order
-__global__ void k_sum_seg(const float* __restrict__ partial, int64_t nblk, int64_t n, int64_t len, float* seg) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int64_t b0 = (int64_t)blockIdx.y * len, b1 = b0 + len < nblk ? b0 + len : nblk;
-  float s = 0.f;
-  for (int64_t b = b0; b < b1; b++) s += partial[b * n + i];
-  seg[(int64_t)blockIdx.y * n + i] = s;
+  float s[NOUT] = {0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int q = 0; q < DEC_ROWS / 4; q++) {
+    const int row = wv * (DEC_ROWS / 4) + q;
+    const int64_t i = i0 + row;
+    if (i >= N) break;
+    const float g[NOUT] = {G[row][0], G[row][1], G[row][2]};
+    const float x = bf2f(h[i * H + k]);
+    dh[i * H + k] = (g[0] * w[0] + g[1] * w[1]) + g[2] * w[2];
+#pragma unroll
+    for (int c = 0; c < NOUT; c++) s[c] += x * g[c];
+  }
+#pragma unroll
+  for (int c = 0; c < NOUT; c++) sm[wv][k][c] = s[c];
+  __syncthreads();
+  float* P = part + (int64_t)blockIdx.x * DECW;
+  if (threadIdx.x < H * NOUT) {
+    const int kk = threadIdx.x / NOUT, c = threadIdx.x % NOUT;
+    P[threadIdx.x] = ((sm[0][kk][c] + sm[1][kk][c]) + sm[2][kk][c]) + sm[3][kk][c];
+  } else if (threadIdx.x < DECW) {
+    const int c = threadIdx.x - H * NOUT;
+    float b = 0.f;
+    for (int q = 0; q < DEC_ROWS; q++) b += G[q][c];
+    P[threadIdx.x] = b;
+  }
 }
 
-// ------------------------------------------------------------------ graph sums
-// agg_i = sum of m_e over edges received by i, in edge order (eight threads per node, eight
-// features each, 16-byte loads and stores)
-__global__ __launch_bounds__(256) void k_agg(int64_t N, const int32_t* __restrict__ rowOff,
-                                              const bf16* __restrict__ m, bf16* agg) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t i = t >> 3;
-  const int f0 = (int)(t & 7) * 8;
-  if (i >= N) return;
-  float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  const int32_t e1 = rowOff[i + 1];
-  for (int32_t e = rowOff[i]; e < e1; e++) {
-    const uint4 v = *reinterpret_cast<const uint4*>(m + (int64_t)e * H + f0);
+// ------------------------------------------------------------------ update, backward
+// dUb = BF16(dh * (u > 0)); [dhp | dagg] = [dh | 0] + dUb Wu^T: dhp FP32, dagg BF16 (g, the gradient
+// of every message of the node before its relu mask)
+__global__ __launch_bounds__(256) void k_bwd_update(int64_t N, const float* __restrict__ dh,
+                                                     const uint64_t* __restrict__ uMask, const bf16* __restrict__ Wr,
+                                                     bf16* __restrict__ dUb, float* __restrict__ dhp,
+                                                     bf16* __restrict__ gOut) {
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t * 16 >= N) return;
+  const bool node = t * 16 + r < N;
+  const int64_t i = node ? t * 16 + r : N - 1;
+  const uint64_t um = uMask[i];
+  uint4 d[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ks++) {
+    const int f0 = ks * 32 + 8 * g;
+    const float4 x = *reinterpret_cast<const float4*>(dh + i * H + f0), y = *reinterpret_cast<const float4*>(dh + i * H + f0 + 4);
+    const uint32_t m = (uint32_t)(um >> f0);
+    const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+    bf16 b[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) b[q] = f2bf((m >> q) & 1u ? v[q] : 0.f);
+    d[ks] = make_uint4(pack2(b[0], b[1]), pack2(b[2], b[3]), pack2(b[4], b[5]), pack2(b[6], b[7]));
+    if (node) *reinterpret_cast<uint4*>(dUb + i * H + f0) = d[ks];
+  }
+#pragma unroll
+  for (int cb = 0; cb < 8; cb++) {
+    floatx4 acc = floatx4{0, 0, 0, 0};
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) acc = mfma(row8(Wr + (cb * 16 + r) * H + ks * 32 + 8 * g), d[ks], acc);
+    if (cb < 4) {
+      const int64_t o = i * H + cb * 16 + 4 * g;
+      const float4 x = *reinterpret_cast<const float4*>(dh + o);
+      if (node) *reinterpret_cast<float4*>(dhp + o) = make_float4(x.x + acc[0], x.y + acc[1], x.z + acc[2], x.w + acc[3]);
+    } else if (node) {
+      *reinterpret_cast<uint2*>(gOut + i * H + (cb - 4) * 16 + 4 * g) =
+          make_uint2(pack2(f2bf(acc[0]), f2bf(acc[1])), pack2(f2bf(acc[2]), f2bf(acc[3])));
+    }
+  }
+}
+
+// ------------------------------------------------------------------ messages, backward
+// an FP32 value as three BF16 terms of 8 bits each, by truncation: their sum is the value itself
+// (a value that is not finite is its first term)
+// (two values at a time, each term of both packed in one word)
+__device__ __forceinline__ uint32_t top16(float& x) {
+  uint32_t u;
+  memcpy(&u, &x, 4);
+  const bool fin = (u & 0x7F800000u) != 0x7F800000u;
+  const uint32_t b = fin ? u >> 16 : (uint32_t)f2bf(x);
+  x = fin ? x - bf2f((bf16)b) : 0.f;
+  return b;
+}
+__device__ __forceinline__ void split3_8(const float (&x)[8], uint4 (&o)[3]) {
+  float y[8];
+#pragma unroll
+  for (int q = 0; q < 8; q++) y[q] = x[q];
+#pragma unroll
+  for (int p = 0; p < 3; p++) {
+    uint32_t b[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) b[q] = top16(y[q]);
+    o[p] = make_uint4(b[0] | b[1] << 16, b[2] | b[3] << 16, b[4] | b[5] << 16, b[6] | b[7] << 16);
+  }
+}
+// s += g masked by 8 bits
+__device__ __forceinline__ void add_masked(float (&s)[8], uint4 v, uint32_t m) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    s[2 * q] += (m >> (2 * q)) & 1u ? bf2f((bf16)(w[q] & 0xFFFFu)) : 0.f;
+    s[2 * q + 1] += (m >> (2 * q + 1)) & 1u ? bf2f((bf16)(w[q] >> 16)) : 0.f;
+  }
+}
+// S1 and S2 of the wavefront's 16 nodes (four lanes per node, 16 features each), and
+// dh = dhp + S1 Wrecv^T + S2 Wsend^T. OPPOSITE: rev[e] is the opposite edge throughout, so the edges
+// that a node sends are the opposites of those it receives; else the edges by sender give S2.
+struct MsgArgs {
+  int64_t N;
+  const int32_t *rowOff, *recv, *send, *rev, *sOff, *sEdge;
+  const uint64_t* mask;
+  const bf16 *g, *Wm;
+  const float* dhp;
+  float *dh, *S1, *S2;
+};
+template <bool OPPOSITE>
+__global__ __launch_bounds__(256) void k_bwd_message(MsgArgs a) {
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t * 16 >= a.N) return;
+  const bool node = t * 16 + r < a.N;
+  const int64_t i = node ? t * 16 + r : a.N - 1;
+  float s1[2][8], s2[2][8];
+#pragma unroll
+  for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+    for (int q = 0; q < 8; q++) s1[ks][q] = s2[ks][q] = 0.f;
+  const uint4 gi[2] = {row8(a.g + i * H + 8 * g), row8(a.g + i * H + 32 + 8 * g)};
+  const int32_t e0 = a.rowOff[i], e1 = a.rowOff[i + 1];
+  // 16 edges at a time: lane g of a node fetches the words of four of them, all in flight together
+  // (two waits on memory per batch, the second one also for the neighbours' rows)
+  for (int32_t eb = e0; eb < e1; eb += 16) {
+    int32_t nb[4];
+    uint64_t m1[4], m2[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int32_t e = min(eb + 4 * k + g, e1 - 1);
+      const int32_t o = a.rev[e];
+      nb[k] = OPPOSITE ? a.send[e] : a.recv[o];
+      m1[k] = a.mask[e];
+      m2[k] = a.mask[o];
+      if (eb + 4 * k + g >= e1) m1[k] = m2[k] = 0;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if (eb + 4 * k >= e1) break;
+      uint4 v[4][2];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int64_t j = __shfl(nb[k], r + 16 * q);
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) v[q][ks] = row8(a.g + j * H + ks * 32 + 8 * g);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const uint64_t x1 = (uint64_t)__shfl((unsigned long long)m1[k], r + 16 * q),
+                       x2 = (uint64_t)__shfl((unsigned long long)m2[k], r + 16 * q);
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+          add_masked(s1[ks], gi[ks], (uint32_t)(x1 >> (ks * 32 + 8 * g)));
+          add_masked(s2[ks], v[q][ks], (uint32_t)(x2 >> (ks * 32 + 8 * g)));
+        }
+      }
+    }
+  }
+  uint4 p1[2][3], p2[2][3];
+#pragma unroll
+  for (int ks = 0; ks < 2; ks++) {
+    split3_8(s1[ks], p1[ks]);
+    split3_8(s2[ks], p2[ks]);
+  }
+#pragma unroll
+  for (int cb = 0; cb < 4; cb++) {
+    floatx4 acc = floatx4{0, 0, 0, 0};
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+      const uint4 w1 = row8(a.Wm + (cb * 16 + r) * H + ks * 32 + 8 * g),
+                  w2 = row8(a.Wm + (H + cb * 16 + r) * H + ks * 32 + 8 * g);
+#pragma unroll
+      for (int p = 2; p >= 0; p--) {
+        acc = mfma(w1, p1[ks][p], acc);
+        acc = mfma(w2, p2[ks][p], acc);
+      }
+    }
+    const int64_t o = i * H + cb * 16 + 4 * g;
+    const float4 x = *reinterpret_cast<const float4*>(a.dhp + o);
+    if (node)
+      *reinterpret_cast<float4*>(a.dh + o) = make_float4(x.x + acc[0], x.y + acc[1], x.z + acc[2], x.w + acc[3]);
+  }
+  if (!node) return;
+  if (!OPPOSITE) {
+    // the weight gradient takes the edges that the node sends
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+      for (int q = 0; q < 8; q++) s2[ks][q] = 0.f;
+    for (int32_t k = a.sOff[i]; k < a.sOff[i + 1]; k++) {
+      const int32_t e = a.sEdge[k];
+      const int64_t j = a.recv[e];
+      const uint64_t m = a.mask[e];
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++)
+        add_masked(s2[ks], row8(a.g + j * H + ks * 32 + 8 * g), (uint32_t)(m >> (ks * 32 + 8 * g)));
+    }
+  }
+#pragma unroll
+  for (int ks = 0; ks < 2; ks++) {
+    const int64_t o = i * H + ks * 32 + 8 * g;
+    *reinterpret_cast<float4*>(a.S1 + o) = make_float4(s1[ks][0], s1[ks][1], s1[ks][2], s1[ks][3]);
+    *reinterpret_cast<float4*>(a.S1 + o + 4) = make_float4(s1[ks][4], s1[ks][5], s1[ks][6], s1[ks][7]);
+    *reinterpret_cast<float4*>(a.S2 + o) = make_float4(s2[ks][0], s2[ks][1], s2[ks][2], s2[ks][3]);
+    *reinterpret_cast<float4*>(a.S2 + o + 4) = make_float4(s2[ks][4], s2[ks][5], s2[ks][6], s2[ks][7]);
+  }
+}
+
+// ------------------------------------------------------------------ weight gradients over nodes
+// One partial per workgroup: [h, agg]^T dUb (KU x H), the column sums of dUb (H), h^T S1 and h^T S2
+// (2H x H). Chunks of 32 nodes are staged in LDS transposed, so that the operands are 16-byte
+// reads; wavefront w forms output features 16 w .. 16 w + 15 (16 accumulators). A workgroup per
+// compute unit at most: more would write and read more partials (66 KB each) than they save.
+constexpr int DWN = KU * H + H + 2 * H * H;
+__global__ __launch_bounds__(256) void k_dw_node(int64_t N, const bf16* __restrict__ h, const bf16* __restrict__ agg,
+                                                  const bf16* __restrict__ dUb, const float* __restrict__ S1,
+                                                  const float* __restrict__ S2, float* __restrict__ part) {
+  __shared__ __attribute__((aligned(16))) bf16 At[KU][32 + 8];
+  __shared__ __attribute__((aligned(16))) bf16 Dt[7][H][32 + 8];  // dUb, the terms of S1, those of S2
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  floatx4 au[8], am[8];
+#pragma unroll
+  for (int cb = 0; cb < 8; cb++) au[cb] = am[cb] = floatx4{0, 0, 0, 0};
+  float bias = 0.f;
+  const int64_t nch = (N + 31) / 32;
+  const int rr = threadIdx.x & 31, c8 = (threadIdx.x >> 5) * 8;
+  auto put = [&](bf16 (*T)[32 + 8], uint4 v) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-      s[2 * q] += bf2f((bf16)(w[q] & 0xFFFFu));
-      s[2 * q + 1] += bf2f((bf16)(w[q] >> 16));
+      T[c8 + 2 * q][rr] = (bf16)(w[q] & 0xFFFFu);
+      T[c8 + 2 * q + 1][rr] = (bf16)(w[q] >> 16);
     }
-  }
-  uint32_t o[4];
+  };
+  // a chunk's rows (zero past the last), loaded while the products of the chunk before run
+  uint4 vh, va, vd;
+  float x1[8], x2[8];
+  auto fetch = [&](int64_t ch) {
+    const bool live = ch * 32 + rr < N;
+    const int64_t o = (live ? ch * 32 + rr : N - 1) * H + c8;
+    vh = row8(h + o);
+    va = row8(agg + o);
+    vd = row8(dUb + o);
 #pragma unroll
-  for (int q = 0; q < 4; q++) o[q] = (uint32_t)f2bf(s[2 * q]) | ((uint32_t)f2bf(s[2 * q + 1]) << 16);
-  *reinterpret_cast<uint4*>(agg + i * H + f0) = make_uint4(o[0], o[1], o[2], o[3]);
-}
-// dY_m,e = dagg_recv(e) * (m_e > 0), BF16
-__global__ void k_edge_dy(int64_t E, const int32_t* __restrict__ recv, const float* __restrict__ dU,
-                          const bf16* __restrict__ m, bf16* dYm) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= E * H) return;
-  const int64_t e = t / H;
-  const int f = (int)(t % H);
-  const float g = dU[(int64_t)recv[e] * KU + H + f];  // the agg part of the update input gradient
-  dYm[t] = f2bf(bf2f(m[t]) > 0.f ? g : 0.f);
-}
-// dh_i = dhOut_i + dU_i[:H] + sum over edges e received by i of dZ_e[:H] + dZ_rev(e)[H:2H]
-__global__ __launch_bounds__(256) void k_node_grad(int64_t N, const int32_t* __restrict__ rowOff,
-                                                    const int32_t* __restrict__ rev, const float* __restrict__ dhOut,
-                                                    const float* __restrict__ dU, const float* __restrict__ dZ,
-                                                    float* dh) {
-  const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int f = threadIdx.x & 63;
-  if (i >= N) return;
-  float s = dhOut[i * H + f] + dU[i * KU + f];
-  for (int32_t e = rowOff[i]; e < rowOff[i + 1]; e++) {
-    s += dZ[(int64_t)e * KU + f];
-    s += dZ[(int64_t)rev[e] * KU + H + f];
+    for (int q = 0; q < 8; q += 4) {
+      const float4 y1 = *reinterpret_cast<const float4*>(S1 + o + q), y2 = *reinterpret_cast<const float4*>(S2 + o + q);
+      x1[q] = y1.x; x1[q + 1] = y1.y; x1[q + 2] = y1.z; x1[q + 3] = y1.w;
+      x2[q] = y2.x; x2[q + 1] = y2.y; x2[q + 2] = y2.z; x2[q + 3] = y2.w;
+    }
+    if (!live) {
+      vh = va = vd = ZERO4;
+#pragma unroll
+      for (int q = 0; q < 8; q++) x1[q] = x2[q] = 0.f;
+    }
+  };
+  if (blockIdx.x < nch) fetch(blockIdx.x);
+  for (int64_t ch = blockIdx.x; ch < nch; ch += gridDim.x) {
+    put(At, vh);
+    put(At + H, va);
+    put(Dt[0], vd);
+    uint4 t3[3];
+    split3_8(x1, t3);
+#pragma unroll
+    for (int p = 0; p < 3; p++) put(Dt[1 + p], t3[p]);
+    split3_8(x2, t3);
+#pragma unroll
+    for (int p = 0; p < 3; p++) put(Dt[4 + p], t3[p]);
+    __syncthreads();
+    if (ch + gridDim.x < nch) fetch(ch + gridDim.x);
+    uint4 d[7];
+#pragma unroll
+    for (int p = 0; p < 7; p++) d[p] = row8(&Dt[p][wv * 16 + r][8 * g]);
+    {
+      const uint32_t w[4] = {d[0].x, d[0].y, d[0].z, d[0].w};
+#pragma unroll
+      for (int q = 0; q < 4; q++) bias += bf2f((bf16)(w[q] & 0xFFFFu)) + bf2f((bf16)(w[q] >> 16));
+    }
+#pragma unroll
+    for (int cb = 0; cb < 8; cb++) {
+      const uint4 x = row8(&At[cb * 16 + r][8 * g]);
+      au[cb] = mfma(x, d[0], au[cb]);
+      if (cb < 4) {
+#pragma unroll
+        for (int p = 2; p >= 0; p--) {
+          am[cb] = mfma(x, d[1 + p], am[cb]);
+          am[4 + cb] = mfma(x, d[4 + p], am[4 + cb]);
+        }
+      }
+    }
+    __syncthreads();
   }
-  dh[i * H + f] = s;
-}
-// dY = g * (act > 0), BF16 (backward of a relu whose output is act)
-__global__ void k_relu_bwd(int64_t n, const float* __restrict__ g, const bf16* __restrict__ act, bf16* dY) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) dY[t] = f2bf(bf2f(act[t]) > 0.f ? g[t] : 0.f);
+  float* P = part + (int64_t)blockIdx.x * DWN;
+  float* Pm = P + KU * H + H;
+#pragma unroll
+  for (int cb = 0; cb < 8; cb++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int o = (cb * 16 + 4 * g + q) * H + wv * 16 + r;
+      P[o] = au[cb][q];
+      Pm[o] = am[cb][q];  // rows 0 .. 63: S1, 64 .. 127: S2
+    }
+  bias += __shfl_xor(bias, 16);
+  bias += __shfl_xor(bias, 32);
+  if (g == 0) P[KU * H + wv * 16 + r] = bias;
 }
 
-// ------------------------------------------------------------------ decoder and loss
-// a_i = h_i W_dec + b_dec (FP32), summed over k in order; one thread per node, the row read
-// as eight 16-byte loads, the weights from LDS
-__global__ __launch_bounds__(256) void k_dec(int64_t N, const bf16* __restrict__ h, const float* __restrict__ W,
-                                              const float* __restrict__ b, float* out) {
-  __shared__ float Ws[H * NOUT];
-  for (int q = threadIdx.x; q < H * NOUT; q += blockDim.x) Ws[q] = W[q];
-  __syncthreads();
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  uint4 hv[H / 8];
+// ------------------------------------------------------------------ weight gradients over input rows
+// in^T D over M rows of inputs, row ONE of the operand set to one (its output row is the bias
+// gradient). EDGE: edge inputs, D_e = mask_e applied to g of the receiver; else node inputs,
+// D_i = BF16(dh_i * (h0_i > 0)). Each wavefront walks chunks of 32 rows; one partial per workgroup.
+struct RowArgs {
+  int64_t M;
+  const bf16* in;
+  const int32_t* recv;
+  const uint64_t* mask;
+  const bf16* g;
+  const float* dh;
+  const bf16* h0;
+};
+constexpr int DWR = 16 * H;
+template <bool EDGE>
+__global__ __launch_bounds__(256) void k_dw_rows(RowArgs a, float* __restrict__ part) {
+  __shared__ float sm[4][DWR];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  floatx4 acc[4];
 #pragma unroll
-  for (int c8 = 0; c8 < H / 8; c8++) hv[c8] = *reinterpret_cast<const uint4*>(h + i * H + c8 * 8);
-  float o[NOUT] = {b[0], b[1], b[2]};
+  for (int cb = 0; cb < 4; cb++) acc[cb] = floatx4{0, 0, 0, 0};
+  const int64_t nch = (a.M + 31) / 32;
+  for (int64_t ch = (int64_t)blockIdx.x * 4 + wv; ch < nch; ch += (int64_t)gridDim.x * 4) {
+    const int64_t m0 = ch * 32 + 8 * g;
+    // (rows past the last: the last one again, zeroed after the loads)
+    bf16 x[8], d[4][8];
+    uint64_t w[8];
 #pragma unroll
-  for (int c8 = 0; c8 < H / 8; c8++) {
-    const uint32_t w[4] = {hv[c8].x, hv[c8].y, hv[c8].z, hv[c8].w};
+    for (int j = 0; j < 8; j++) {
+      const int64_t m = min(m0 + j, a.M - 1);
+      x[j] = a.in[m * (EDGE ? EP : XP) + (EDGE ? r : (r & (XP - 1)))];
+      if (EDGE) {
+        w[j] = a.mask[m];
+        const int64_t i = a.recv[m];
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const int k = c8 * 8 + q;
-      const float x = bf2f((bf16)((q & 1) ? (w[q >> 1] >> 16) : (w[q >> 1] & 0xFFFFu)));
+        for (int cb = 0; cb < 4; cb++) d[cb][j] = a.g[i * H + cb * 16 + r];
+      } else {
+        w[j] = 0;
 #pragma unroll
-      for (int c = 0; c < NOUT; c++) o[c] += x * Ws[k * NOUT + c];
+        for (int cb = 0; cb < 4; cb++) {
+          d[cb][j] = f2bf(a.dh[m * H + cb * 16 + r]);
+          w[j] |= (uint64_t)(on(a.h0[m * H + cb * 16 + r]) ? 1u : 0u) << (cb * 16 + r);
+        }
+      }
     }
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const bool live = m0 + j < a.M;
+      if (!live || (!EDGE && r >= XP)) x[j] = 0;
+      if (live && r == ONE) x[j] = (bf16)0x3F80;
+#pragma unroll
+      for (int cb = 0; cb < 4; cb++)
+        if (!live || !((w[j] >> (cb * 16 + r)) & 1ull)) d[cb][j] = 0;
+    }
+    const uint4 xv = make_uint4(pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7]));
+#pragma unroll
+    for (int cb = 0; cb < 4; cb++)
+      acc[cb] = mfma(xv, make_uint4(pack2(d[cb][0], d[cb][1]), pack2(d[cb][2], d[cb][3]), pack2(d[cb][4], d[cb][5]),
+                                    pack2(d[cb][6], d[cb][7])), acc[cb]);
   }
 #pragma unroll
-  for (int c = 0; c < NOUT; c++) out[i * NOUT + c] = o[c];
-}
-// loss = mean over nodes of |a - t|^2; dA = 2 (a - t) / N; per-block partial loss
-// A node is in contact when its floor overlap input or the overlap input of one of its edges
-// is positive. Nodes not in contact move in free flight (the network's output is not used for
-// them), so they carry no loss.
-__global__ __launch_bounds__(256) void k_contact(int64_t N, const int32_t* __restrict__ rowOff,
-                                                  const bf16* __restrict__ X, const bf16* __restrict__ EF,
-                                                  uint8_t* flag) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  bool c = bf2f(X[i * KX + 4]) > 0.f;
-  for (int32_t e = rowOff[i]; e < rowOff[i + 1] && !c; e++) c = bf2f(EF[(int64_t)e * KE + 3]) > 0.f;
-  flag[i] = c ? 1 : 0;
-}
-__global__ __launch_bounds__(256) void k_loss(int64_t N, const float* __restrict__ a, const float* __restrict__ t,
-                                               const uint8_t* __restrict__ flag, float* dA, float* partLoss) {
-  __shared__ float sm[256];
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  float l = 0.f;
-  if (i < N)
-    for (int c = 0; c < NOUT; c++) {
-      const float d = flag[i] ? a[i * NOUT + c] - t[i * NOUT + c] : 0.f;
-      l += d * d;
-      dA[i * NOUT + c] = 2.f * d / (float)N;
-    }
-  sm[threadIdx.x] = l;
+  for (int cb = 0; cb < 4; cb++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) sm[wv][(4 * g + q) * H + cb * 16 + r] = acc[cb][q];
   __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sm[threadIdx.x] += sm[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partLoss[blockIdx.x] = sm[0];
+  for (int q = threadIdx.x; q < DWR; q += 256)
+    part[(int64_t)blockIdx.x * DWR + q] = ((sm[0][q] + sm[1][q]) + sm[2][q]) + sm[3][q];
 }
-// decoder backward: dh_i = dA_i W^T (FP32), per-block partials of dW (H x 3) and db (3)
-__global__ __launch_bounds__(256) void k_dec_bwd(int64_t N, const bf16* __restrict__ h, const float* __restrict__ W,
-                                                  const float* __restrict__ dA, float* dh, float* partW) {
-  __shared__ float sm[256][NOUT + 1];
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool live = i < N;
-  float g[NOUT] = {0, 0, 0};
-  if (live)
-    for (int c = 0; c < NOUT; c++) g[c] = dA[i * NOUT + c];
-  if (live)
-    for (int k = 0; k < H; k++) dh[i * H + k] = (g[0] * W[k * NOUT + 0] + g[1] * W[k * NOUT + 1]) + g[2] * W[k * NOUT + 2];
-  // dW[k][c] = sum_i h[i][k] g[c]: one pass per k over the block
-  for (int k = 0; k < H + 1; k++) {
-    const float x = k < H ? (live ? bf2f(h[i * H + k]) : 0.f) : (live ? 1.f : 0.f);  // k == H: bias
-    for (int c = 0; c < NOUT; c++) sm[threadIdx.x][c] = x * g[c];
+
+// ------------------------------------------------------------------ sums of the partials
+// every region of the gradient in one launch: 64 columns per workgroup, the partials of a column
+// over 16 wavefronts, then those in order. The last workgroup adds the loss up (in FP64).
+// 25,000 nodes, 175,000 edges: 9 us; one thread per column and eleven
+// launches took 257.
+struct SumArgs {
+  struct Region {
+    const float* src;
+    int64_t stride;
+    int nblk, n;
+    float* dst;
+    int blk0;
+  };
+  Region r[14];
+  int n, blocks;
+};
+__global__ __launch_bounds__(1024) void k_sum_partials(SumArgs a, int64_t nLoss, const float* __restrict__ partLoss,
+                                                        double* loss) {
+  if ((int)blockIdx.x == a.blocks) {
+    __shared__ double sd[1024];
+    double l = 0.;
+    for (int64_t b = threadIdx.x; b < nLoss; b += 1024) l += (double)partLoss[b];
+    sd[threadIdx.x] = l;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-      if (threadIdx.x < s)
-        for (int c = 0; c < NOUT; c++) sm[threadIdx.x][c] += sm[threadIdx.x + s][c];
+    for (int st = 512; st > 0; st >>= 1) {
+      if ((int)threadIdx.x < st) sd[threadIdx.x] += sd[threadIdx.x + st];
       __syncthreads();
     }
-    if (threadIdx.x < NOUT) partW[(int64_t)blockIdx.x * (H + 1) * NOUT + k * NOUT + threadIdx.x] = sm[0][threadIdx.x];
-    __syncthreads();
+    if (threadIdx.x == 0) *loss = sd[0];
+    return;
+  }
+  int q = 0;
+  while (q + 1 < a.n && (int)blockIdx.x >= a.r[q + 1].blk0) q++;
+  const SumArgs::Region R = a.r[q];
+  __shared__ float sm[16][64];
+  const int col = ((int)blockIdx.x - R.blk0) * 64 + (threadIdx.x & 63), wv = threadIdx.x >> 6;
+  float s = 0.f;
+  if (col < R.n) {
+#pragma unroll 8
+    for (int b = wv; b < R.nblk; b += 16) s += R.src[(int64_t)b * R.stride + col];
+  }
+  sm[wv][threadIdx.x & 63] = s;
+  __syncthreads();
+  if (wv == 0 && col < R.n) {
+#pragma unroll
+    for (int k = 1; k < 16; k++) s += sm[k][threadIdx.x];
+    R.dst[col] = s;
   }
 }
 
 // ------------------------------------------------------------------ optimizer and images
+// BF16 images of the weights (K x 64 each): transposed [64 x K] and row-major [K x 64]
+struct ImgArgs {
+  int64_t src[5];
+  int K[5];
+  int64_t t[5], r[5];
+  bf16* img;
+};
+__device__ __forceinline__ void image_write(const ImgArgs& g, int64_t i, float w) {
+#pragma unroll
+  for (int q = 0; q < 5; q++) {
+    const int64_t t = i - g.src[q];
+    if (t >= 0 && t < (int64_t)g.K[q] * H) {
+      const bf16 b = f2bf(w);
+      g.img[g.r[q] + t] = b;
+      g.img[g.t[q] + (t % H) * g.K[q] + t / H] = b;
+    }
+  }
+}
 __global__ void k_adam(int64_t n, float* p, const float* __restrict__ g, float* m, float* v, float lr, float b1,
-                       float b2, float eps, float c1, float c2) {
+                       float b2, float eps, float c1, float c2, ImgArgs im) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const float gi = g[i];
@@ -523,16 +911,13 @@ __global__ void k_adam(int64_t n, float* p, const float* __restrict__ g, float* 
   const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
   m[i] = mi;
   v[i] = vi;
-  p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  const float w = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  p[i] = w;
+  image_write(im, i, w);
 }
-// BF16 images of a K x 64 weight: transposed [64 x K] and row-major [K x 64]
-__global__ void k_images(const float* __restrict__ W, int K, bf16* Wt, bf16* Wr) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= K * H) return;
-  const int k = t / H, o = t % H;
-  const bf16 b = f2bf(W[t]);
-  Wr[t] = b;
-  Wt[o * K + k] = b;
+__global__ void k_images(int64_t n, const float* __restrict__ p, ImgArgs im) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) image_write(im, i, p[i]);
 }
 
 // ------------------------------------------------------------------ state
@@ -547,6 +932,9 @@ struct Mpnn {
   // graph
   int64_t N = 0, E = 0;
   DBuf<int32_t> rowOff, recv, send, rev;
+  // edges by sender, for a caller's graph in which rev is not the opposite edge throughout
+  DBuf<int32_t> sOff, sEdge;
+  bool opposite = true;
   DBuf<bf16> X, EF;
   DBuf<float> T;  // targets
   DBuf<int32_t> deg, slotSide, edgeOfSlot;
@@ -560,19 +948,23 @@ struct Mpnn {
   int64_t uidRefresh = -1, uidN = -1;
   uint64_t uidUploads = 0;
   // activations
-  DBuf<bf16> h[3], m[2], agg[2], u[2];
-  DBuf<float> out, dA, dhA, dhB, dU, dZ, part, partB, partLoss, partSeg;
-  DBuf<bf16> dY, dYe;
+  DBuf<bf16> h[3], agg[2];
+  DBuf<uint64_t> mMask[2], uMask[2];  // relu signs of the messages and of the updates, a bit per feature
+  DBuf<float> out, dhA, dhB, S1, S2, part, partLoss;
+  DBuf<bf16> dUb, g;          // gradients at the relus of the updates, and of the summed messages
+  double *hres = nullptr, *hresDev = nullptr;  // the loss, in pinned host memory
   DBuf<uint8_t> cflag;  // node in contact (else in free flight)
   hipEvent_t done = nullptr;  // orders the network's stream and an engine context's stream
   // graphs kept on the device (training sets): inputs, structure and targets
   struct Kept {
     int64_t N = -1, E = 0;
-    DBuf<int32_t> rowOff, recv, send, rev;
+    DBuf<int32_t> rowOff, recv, send, rev, sOff, sEdge;
+    bool opposite = true;
     DBuf<bf16> X, EF;
     DBuf<float> T;
     void release() {
       rowOff.release(); recv.release(); send.release(); rev.release(); X.release(); EF.release(); T.release();
+      sOff.release(); sEdge.release();
       N = -1;
     }
   };
@@ -601,172 +993,130 @@ static void copy_buf(DBuf<T>& dst, const DBuf<T>& src, size_t n, hipStream_t st)
   if (n) WDG_HIP(hipMemcpyAsync(dst.p, src.p, n * sizeof(T), hipMemcpyDeviceToDevice, st));
 }
 
-static void images(Mpnn& s) {
+static ImgArgs img_args(Mpnn& s) {
+  ImgArgs g{};
   const int Ks[5] = {KX, KM, KU, KM, KU};
   const size_t src[5] = {s.L.encW, s.L.mW[0], s.L.uW[0], s.L.mW[1], s.L.uW[1]};
   size_t o = 0;
   for (int q = 0; q < 5; q++) {
     s.imgT[q] = o; o += (size_t)Ks[q] * H;
     s.imgR[q] = o; o += (size_t)Ks[q] * H;
+    g.src[q] = (int64_t)src[q]; g.K[q] = Ks[q];
+    g.t[q] = (int64_t)s.imgT[q]; g.r[q] = (int64_t)s.imgR[q];
   }
   s.img.ensure(o);
-  for (int q = 0; q < 5; q++) {
-    hipLaunchKernelGGL(k_images, dim3(nblocks((int64_t)Ks[q] * H, 256)), dim3(256), 0, s.stream, s.P.p + src[q], Ks[q],
-                       s.img.p + s.imgT[q], s.img.p + s.imgR[q]);
-    WDG_LAUNCH_CHECK();
-  }
+  g.img = s.img.p;
+  return g;
 }
-
-// sums of per-block partials in a fixed order: directly for few blocks, else over SUM_SEGS
-// segments of consecutive blocks and then over the segments
-constexpr int64_t SUM_SEGS = 64;
-static void sum_partials(Mpnn& s, const float* partial, int64_t nblk, int64_t n, float* out) {
-  if (nblk <= 2 * SUM_SEGS) {
-    hipLaunchKernelGGL(k_sum_partials, dim3(nblocks(n, 256)), dim3(256), 0, s.stream, partial, nblk, n, out);
-    WDG_LAUNCH_CHECK();
-    return;
-  }
-  const int64_t len = (nblk + SUM_SEGS - 1) / SUM_SEGS;
-  hipLaunchKernelGGL(k_sum_seg, dim3(nblocks(n, 256), (unsigned)SUM_SEGS), dim3(256), 0, s.stream, partial, nblk, n,
-                     len, s.partSeg.p);
-  WDG_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_sum_partials, dim3(nblocks(n, 256)), dim3(256), 0, s.stream, (const float*)s.partSeg.p,
-                     SUM_SEGS, n, out);
+static void images(Mpnn& s) {
+  const ImgArgs g = img_args(s);
+  hipLaunchKernelGGL(k_images, dim3(nblocks((int64_t)s.L.total, 256)), dim3(256), 0, s.stream, (int64_t)s.L.total,
+                     (const float*)s.P.p, g);
   WDG_LAUNCH_CHECK();
 }
 
-template <int MODE, int KP>
-static void dw(Mpnn& s, const ARows& a, int64_t M, const bf16* dY, float* gW, float* gB) {
-  const int64_t rowsPer = (int64_t)DW_CHUNKS * 32;
-  const int64_t nblk = std::max<int64_t>((M + rowsPer - 1) / rowsPer, 1);
-  hipLaunchKernelGGL((k_mm_dw<MODE, KP>), dim3((unsigned)nblk), dim3(256), 0, s.stream, a, M, dY, s.part.p, s.partB.p);
-  WDG_LAUNCH_CHECK();
-  sum_partials(s, s.part.p, nblk, (int64_t)KP * H, gW);
-  sum_partials(s, s.partB.p, nblk, (int64_t)H, gB);
-}
-
-static void forward(Mpnn& s) {
+// store: also what the backward pass reads (relu signs, summed messages)
+static void forward(Mpnn& s, bool store) {
   const int64_t N = s.N, E = s.E;
-  for (auto& b : s.h) b.ensure((size_t)std::max<int64_t>(N, 1) * H);
-  for (int l = 0; l < 2; l++) {
-    s.m[l].ensure((size_t)std::max<int64_t>(E, 1) * H);
-    s.agg[l].ensure((size_t)std::max<int64_t>(N, 1) * H);
-    s.u[l].ensure((size_t)std::max<int64_t>(N, 1) * H);
-  }
-  s.out.ensure((size_t)std::max<int64_t>(N, 1) * NOUT);
-  s.cflag.ensure((size_t)std::max<int64_t>(N, 1));
-  if (N == 0) return;
-  hipLaunchKernelGGL(k_contact, dim3(nblocks(N, 256)), dim3(256), 0, s.stream, N, (const int32_t*)s.rowOff.p,
-                     (const bf16*)s.X.p, (const bf16*)s.EF.p, s.cflag.p);
-  WDG_LAUNCH_CHECK();
-  const unsigned gN = fwd_blocks(N), gE = fwd_blocks(E);
-  ARows a{};
-  a.x = s.X.p;
-  a.K = KX;
-  hipLaunchKernelGGL((k_mm_fwd<A_PLAIN, false>), dim3(gN), dim3(256), 0, s.stream, a, N,
-                     (const bf16*)(s.img.p + s.imgT[0]), (const float*)(s.P.p + s.L.encB), s.h[0].p, (bf16*)nullptr);
-  WDG_LAUNCH_CHECK();
-  for (int l = 0; l < 2; l++) {
-    ARows ae{};
-    ae.h = s.h[l].p; ae.ef = s.EF.p; ae.recv = s.recv.p; ae.send = s.send.p; ae.K = KM;
-    if (E > 0) {
-      hipLaunchKernelGGL((k_mm_fwd<A_EDGE, false>), dim3(gE), dim3(256), 0, s.stream, ae, E,
-                         (const bf16*)(s.img.p + s.imgT[1 + 2 * l]), (const float*)(s.P.p + s.L.mB[l]), s.m[l].p,
-                         (bf16*)nullptr);
-      WDG_LAUNCH_CHECK();
+  const size_t n = (size_t)std::max<int64_t>(N, 1);
+  for (auto& b : s.h) b.ensure(n * H);
+  s.out.ensure(n * NOUT);
+  s.cflag.ensure(n);
+  if (store)
+    for (int l = 0; l < 2; l++) {
+      s.agg[l].ensure(n * H);
+      s.uMask[l].ensure(n);
+      s.mMask[l].ensure((size_t)std::max<int64_t>(E, 1));
     }
-    hipLaunchKernelGGL(k_agg, dim3(nblocks(N * 8, 256)), dim3(256), 0, s.stream, N, (const int32_t*)s.rowOff.p,
-                       (const bf16*)s.m[l].p, s.agg[l].p);
-    WDG_LAUNCH_CHECK();
-    ARows au{};
-    au.h = s.h[l].p; au.agg = s.agg[l].p; au.K = KU;
-    hipLaunchKernelGGL((k_mm_fwd<A_UPD, true>), dim3(gN), dim3(256), 0, s.stream, au, N,
-                       (const bf16*)(s.img.p + s.imgT[2 + 2 * l]), (const float*)(s.P.p + s.L.uB[l]), s.u[l].p,
-                       s.h[l + 1].p);
+  if (N == 0) return;
+  const int64_t nt = (N + 15) / 16;
+  hipLaunchKernelGGL(k_enc, dim3(nblocks(nt, 4)), dim3(256), 0, s.stream, N, (const bf16*)s.X.p,
+                     (const bf16*)(s.img.p + s.imgT[0]), (const float*)(s.P.p + s.L.encB), s.h[0].p);
+  WDG_LAUNCH_CHECK();
+  for (int l = 0; l < 2; l++) {
+    LayerArgs a{};
+    a.N = N;
+    a.rowOff = s.rowOff.p; a.recv = s.recv.p; a.send = s.send.p;
+    a.h = s.h[l].p; a.ef = s.EF.p; a.x = s.X.p;
+    a.Wm = s.img.p + s.imgT[1 + 2 * l]; a.Wu = s.img.p + s.imgT[2 + 2 * l];
+    a.bm = s.P.p + s.L.mB[l]; a.bu = s.P.p + s.L.uB[l];
+    a.Wd = s.P.p + s.L.decW; a.bd = s.P.p + s.L.decB;
+    a.hOut = s.h[l + 1].p; a.agg = s.agg[l].p; a.mMask = s.mMask[l].p; a.uMask = s.uMask[l].p;
+    a.out = s.out.p; a.flag = s.cflag.p;
+    auto* k = store ? (l ? k_layer<true, true> : k_layer<true, false>) : (l ? k_layer<false, true> : k_layer<false, false>);
+    hipLaunchKernelGGL(k, dim3((unsigned)std::min<int64_t>(nblocks(nt, LY_BS / 64), 768)), dim3(LY_BS), 0, s.stream, a);
     WDG_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(k_dec, dim3(nblocks(N, 256)), dim3(256), 0, s.stream, N, (const bf16*)s.h[2].p,
-                     (const float*)(s.P.p + s.L.decW), (const float*)(s.P.p + s.L.decB), s.out.p);
-  WDG_LAUNCH_CHECK();
 }
 
 // gradients of the loss (mean squared error against s.T) into s.G; returns the loss
 static double backward(Mpnn& s) {
   const int64_t N = s.N, E = s.E;
-  const int64_t nbN = nblocks(N, 256);
-  s.dA.ensure((size_t)N * NOUT);
-  s.partLoss.ensure((size_t)nbN);
-  s.dhA.ensure((size_t)N * H);
-  s.dhB.ensure((size_t)N * H);
-  s.dU.ensure((size_t)N * KU);
-  s.dZ.ensure((size_t)std::max<int64_t>(E, 1) * KU);
-  s.dY.ensure((size_t)N * H);
-  s.dYe.ensure((size_t)std::max<int64_t>(E, 1) * H);
-  // one partial buffer, sized for the largest user (no reallocation while kernels run)
-  {
-    const int64_t rowsPer = (int64_t)DW_CHUNKS * 32;
-    const int64_t bE = std::max<int64_t>((E + rowsPer - 1) / rowsPer, 1), bN = std::max<int64_t>((N + rowsPer - 1) / rowsPer, 1);
-    const size_t need = std::max({(size_t)bE * KM * H, (size_t)bN * KU * H, (size_t)nbN * (H + 1) * NOUT});
-    s.part.ensure(need);
-    s.partB.ensure((size_t)std::max(bE, bN) * H);
-    s.partSeg.ensure((size_t)SUM_SEGS * KM * H);
-  }
-  WDG_HIP(hipMemsetAsync(s.G.p, 0, s.L.total * sizeof(float), s.stream));
-  hipLaunchKernelGGL(k_loss, dim3((unsigned)nbN), dim3(256), 0, s.stream, N, (const float*)s.out.p,
-                     (const float*)s.T.p, (const uint8_t*)s.cflag.p, s.dA.p, s.partLoss.p);
+  const int64_t nt = (N + 15) / 16;
+  const size_t n = (size_t)N;
+  s.dhA.ensure(n * H); s.dhB.ensure(n * H);
+  s.S1.ensure(n * H); s.S2.ensure(n * H);
+  s.dUb.ensure(n * H); s.g.ensure(n * H);
+  // workgroups of the weight gradients (each leaves one partial): one per compute unit for the
+  // products over nodes, more for those over edges, whose partials are small
+  const int64_t bN = std::min<int64_t>((N + 31) / 32, 256), bE = std::min<int64_t>((E + 127) / 128, 512),
+                bX = std::min<int64_t>((N + 127) / 128, 512), bD = (N + DEC_ROWS - 1) / DEC_ROWS;
+  const int64_t oN = 0, oE = oN + 2 * bN * DWN, oX = oE + 2 * bE * DWR, oD = oX + bX * DWR;
+  s.part.ensure((size_t)(oD + bD * DECW));
+  s.partLoss.ensure((size_t)bD);
+  SumArgs sum{};
+  auto region = [&](const float* src, int64_t stride, int64_t nblk, int cnt, size_t dst) {
+    SumArgs::Region& r = sum.r[sum.n++];
+    r = {src, stride, (int)nblk, cnt, s.G.p + dst, sum.blocks};
+    sum.blocks += (cnt + 63) / 64;
+  };
+  hipLaunchKernelGGL(k_loss_dec, dim3((unsigned)bD), dim3(256), 0, s.stream, N, (const float*)s.out.p,
+                     (const float*)s.T.p, (const uint8_t*)s.cflag.p, (const bf16*)s.h[2].p,
+                     (const float*)(s.P.p + s.L.decW), s.dhA.p, s.part.p + oD, s.partLoss.p);
   WDG_LAUNCH_CHECK();
-  // decoder
-  hipLaunchKernelGGL(k_dec_bwd, dim3((unsigned)nbN), dim3(256), 0, s.stream, N, (const bf16*)s.h[2].p,
-                     (const float*)(s.P.p + s.L.decW), (const float*)s.dA.p, s.dhA.p, s.part.p);
-  WDG_LAUNCH_CHECK();
-  sum_partials(s, s.part.p, nbN, (int64_t)(H + 1) * NOUT, s.G.p + s.L.decW);  // decW then decB are adjacent
-  float* dh = s.dhA.p;   // gradient of the current layer output
-  float* dh2 = s.dhB.p;
-  const unsigned gN = (unsigned)((N + 63) / 64), gE = (unsigned)((E + 63) / 64);
+  region(s.part.p + oD, DECW, bD, DECW, s.L.decW);  // decW then decB are adjacent
   for (int l = 1; l >= 0; l--) {
-    // update: u = relu([h, agg] Wu + bu), h_out = h + u
-    hipLaunchKernelGGL(k_relu_bwd, dim3(nblocks(N * H, 256)), dim3(256), 0, s.stream, N * H, (const float*)dh,
-                       (const bf16*)s.u[l].p, s.dY.p);
+    hipLaunchKernelGGL(k_bwd_update, dim3(nblocks(nt, 4)), dim3(256), 0, s.stream, N, (const float*)s.dhA.p,
+                       (const uint64_t*)s.uMask[l].p, (const bf16*)(s.img.p + s.imgR[2 + 2 * l]), s.dUb.p, s.dhB.p,
+                       s.g.p);
     WDG_LAUNCH_CHECK();
-    ARows au{};
-    au.h = s.h[l].p; au.agg = s.agg[l].p; au.K = KU;
-    dw<A_UPD, KU>(s, au, N, s.dY.p, s.G.p + s.L.uW[l], s.G.p + s.L.uB[l]);
-    hipLaunchKernelGGL((k_mm_dx<KU>), dim3(gN), dim3(256), 0, s.stream, (const bf16*)s.dY.p, N,
-                       (const bf16*)(s.img.p + s.imgR[2 + 2 * l]), s.dU.p);
+    MsgArgs a{};
+    a.N = N;
+    a.rowOff = s.rowOff.p; a.recv = s.recv.p; a.send = s.send.p; a.rev = s.rev.p;
+    a.sOff = s.sOff.p; a.sEdge = s.sEdge.p;
+    a.mask = s.mMask[l].p; a.g = s.g.p; a.Wm = s.img.p + s.imgR[1 + 2 * l];
+    a.dhp = s.dhB.p; a.dh = s.dhA.p; a.S1 = s.S1.p; a.S2 = s.S2.p;
+    hipLaunchKernelGGL(s.opposite ? k_bwd_message<true> : k_bwd_message<false>, dim3(nblocks(nt, 4)), dim3(256), 0,
+                       s.stream, a);
     WDG_LAUNCH_CHECK();
-    // messages
+    float *pN = s.part.p + oN + l * bN * DWN, *pE = s.part.p + oE + l * bE * DWR;
+    hipLaunchKernelGGL(k_dw_node, dim3((unsigned)bN), dim3(256), 0, s.stream, N, (const bf16*)s.h[l].p,
+                       (const bf16*)s.agg[l].p, (const bf16*)s.dUb.p, (const float*)s.S1.p, (const float*)s.S2.p, pN);
+    WDG_LAUNCH_CHECK();
     if (E > 0) {
-      hipLaunchKernelGGL(k_edge_dy, dim3(nblocks(E * H, 256)), dim3(256), 0, s.stream, E, (const int32_t*)s.recv.p,
-                         (const float*)s.dU.p, (const bf16*)s.m[l].p, s.dYe.p);
-      WDG_LAUNCH_CHECK();
-      ARows ae{};
-      ae.h = s.h[l].p; ae.ef = s.EF.p; ae.recv = s.recv.p; ae.send = s.send.p; ae.K = KM;
-      dw<A_EDGE, KM>(s, ae, E, s.dYe.p, s.G.p + s.L.mW[l], s.G.p + s.L.mB[l]);
-      // only the node-activation columns of the message input need a gradient
-      hipLaunchKernelGGL((k_mm_dx<KU>), dim3(gE), dim3(256), 0, s.stream, (const bf16*)s.dYe.p, E,
-                         (const bf16*)(s.img.p + s.imgR[1 + 2 * l]), s.dZ.p);
+      RowArgs r{};
+      r.M = E; r.in = s.EF.p; r.recv = s.recv.p; r.mask = s.mMask[l].p; r.g = s.g.p;
+      hipLaunchKernelGGL(k_dw_rows<true>, dim3((unsigned)bE), dim3(256), 0, s.stream, r, pE);
       WDG_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(k_node_grad, dim3((unsigned)((N + 3) / 4)), dim3(256), 0, s.stream, N,
-                       (const int32_t*)s.rowOff.p, (const int32_t*)s.rev.p, (const float*)dh, (const float*)s.dU.p,
-                       (const float*)s.dZ.p, dh2);
-    WDG_LAUNCH_CHECK();
-    std::swap(dh, dh2);
+    region(pN, DWN, bN, KU * H + H, s.L.uW[l]);  // uW then uB are adjacent
+    region(pN + KU * H + H, DWN, bN, 2 * H * H, s.L.mW[l]);
+    region(pE, DWR, E > 0 ? bE : 0, NEI * H, s.L.mW[l] + 2 * H * H);
+    region(nullptr, 0, 0, (KE - NEI) * H, s.L.mW[l] + (size_t)(2 * H + NEI) * H);
+    region(pE + ONE * H, DWR, E > 0 ? bE : 0, H, s.L.mB[l]);
   }
-  // encoder
-  hipLaunchKernelGGL(k_relu_bwd, dim3(nblocks(N * H, 256)), dim3(256), 0, s.stream, N * H, (const float*)dh,
-                     (const bf16*)s.h[0].p, s.dY.p);
+  RowArgs r{};
+  r.M = N; r.in = s.X.p; r.dh = s.dhA.p; r.h0 = s.h[0].p;
+  hipLaunchKernelGGL(k_dw_rows<false>, dim3((unsigned)bX), dim3(256), 0, s.stream, r, s.part.p + oX);
   WDG_LAUNCH_CHECK();
-  ARows ax{};
-  ax.x = s.X.p;
-  ax.K = KX;
-  dw<A_PLAIN, KX>(s, ax, N, s.dY.p, s.G.p + s.L.encW, s.G.p + s.L.encB);
-  std::vector<float> pl((size_t)nbN);
-  WDG_HIP(hipMemcpyAsync(pl.data(), s.partLoss.p, nbN * sizeof(float), hipMemcpyDeviceToHost, s.stream));
+  region(s.part.p + oX, DWR, bX, NIN * H, s.L.encW);
+  region(nullptr, 0, 0, (KX - NIN) * H, s.L.encW + (size_t)NIN * H);
+  region(s.part.p + oX + ONE * H, DWR, bX, H, s.L.encB);
+  hipLaunchKernelGGL(k_sum_partials, dim3((unsigned)sum.blocks + 1), dim3(1024), 0, s.stream, sum, bD,
+                     (const float*)s.partLoss.p, s.hresDev);
+  WDG_LAUNCH_CHECK();
   WDG_HIP(hipStreamSynchronize(s.stream));
-  double loss = 0;
-  for (float x : pl) loss += x;
-  return loss / (double)N;
+  return *s.hres / (double)N;
 }
 
 // ------------------------------------------------------------------ graph from an engine context
@@ -837,17 +1187,17 @@ __global__ __launch_bounds__(256) void k_mg_inputs(GraphArgs g, int64_t E) {
   if (q < E) {
     const int64_t i = g.nW + g.recv[q], j = g.nW + g.send[q];
     g.rev[q] = g.edgeOfSlot[g.slotSide[q] ^ 1];
-    float f[KE];
-    for (int c = NEI; c < KE; c++) f[c] = 0.f;
+    float f[EP];
+    for (int c = NEI; c < EP; c++) f[c] = 0.f;
     edge_inputs(g.px[i], g.py[i], g.pz[i], g.px[j], g.py[j], g.pz[j], g.vx[i], g.vy[i], g.vz[i], g.vx[j], g.vy[j],
                 g.vz[j], g.rad[i], g.rad[j], f);
-    store_row<KE>(g.EF + q * KE, f);
+    store_row<EP>(g.EF + q * EP, f);
   } else if (q < E + g.nSph) {
     const int64_t t = q - E, s = g.nW + t;
-    float x[KX];
-    for (int c = NIN; c < KX; c++) x[c] = 0.f;
+    float x[XP];
+    for (int c = NIN; c < XP; c++) x[c] = 0.f;
     node_inputs(g.vx[s], g.vy[s], g.vz[s], g.rad[s], g.pz[s] - g.floorZ, x);
-    store_row<KX>(g.X + t * KX, x);
+    store_row<XP>(g.X + t * XP, x);
   }
 }
 // coarse step: v += a dT, x += v dT for the spheres; a is the network's output (in units of
@@ -932,6 +1282,8 @@ int wdg_mpnn_create(int device, uint64_t seed, wdg_mpnn** out) {
     WDG_HIP(hipSetDevice(device));
     WDG_HIP(hipStreamCreate(&s.stream));
     WDG_HIP(hipEventCreateWithFlags(&s.done, hipEventDisableTiming));
+    WDG_HIP(hipHostMalloc((void**)&s.hres, sizeof(double), hipHostMallocDefault));
+    WDG_HIP(hipHostGetDevicePointer((void**)&s.hresDev, s.hres, 0));
     const size_t n = s.L.total;
     s.P.ensure(n); s.G.ensure(n); s.Am.ensure(n); s.Av.ensure(n);
     // Glorot-uniform weights over the used input rows, zero biases and padding rows (the
@@ -975,12 +1327,13 @@ int wdg_mpnn_create(int device, uint64_t seed, wdg_mpnn** out) {
 int wdg_mpnn_destroy(wdg_mpnn* m) {
   if (!m) return WDG_OK;
   Mpnn& s = m->s;
-  DBuf<float>* fb[] = {&s.P, &s.G, &s.Am, &s.Av, &s.T, &s.out, &s.dA, &s.dhA, &s.dhB, &s.dU, &s.dZ, &s.part, &s.partB,
-                       &s.partLoss, &s.partSeg};
+  DBuf<float>* fb[] = {&s.P, &s.G, &s.Am, &s.Av, &s.T, &s.out, &s.dhA, &s.dhB, &s.S1, &s.S2, &s.part, &s.partLoss};
   for (auto* b : fb) b->release();
-  DBuf<bf16>* bb[] = {&s.img, &s.X, &s.EF, &s.h[0], &s.h[1], &s.h[2], &s.m[0], &s.m[1], &s.agg[0], &s.agg[1],
-                      &s.u[0], &s.u[1], &s.dY, &s.dYe};
+  DBuf<bf16>* bb[] = {&s.img, &s.X, &s.EF, &s.h[0], &s.h[1], &s.h[2], &s.agg[0], &s.agg[1],
+                      &s.dUb, &s.g};
   for (auto* b : bb) b->release();
+  for (int l = 0; l < 2; l++) { s.mMask[l].release(); s.uMask[l].release(); }
+  s.sOff.release(); s.sEdge.release();
   s.cflag.release();
   s.rowOff.release(); s.recv.release(); s.send.release(); s.rev.release();
   s.deg.release(); s.slotSide.release(); s.edgeOfSlot.release(); s.degScan.release(); s.nodeUid.release();
@@ -988,6 +1341,7 @@ int wdg_mpnn_destroy(wdg_mpnn* m) {
   if (s.stream) (void)hipStreamSynchronize(s.stream);
   if (s.done) (void)hipEventDestroy(s.done);
   if (s.stream) (void)hipStreamDestroy(s.stream);
+  if (s.hres) (void)hipHostFree(s.hres);
   delete m;
   return WDG_OK;
 }
@@ -1026,17 +1380,30 @@ int wdg_mpnn_set_graph(wdg_mpnn* m, int64_t N, int64_t E, const float* x, const 
   return mguard([&] {
     Mpnn& s = m->s;
     if (rowOff[0] != 0 || rowOff[N] != E) throw Error(WDG_E_ARG, "rowOff must run from 0 to E");
-    std::vector<bf16> X((size_t)std::max<int64_t>(N, 1) * KX, 0), F((size_t)std::max<int64_t>(E, 1) * KE, 0);
+    std::vector<bf16> X((size_t)std::max<int64_t>(N, 1) * XP, 0), F((size_t)std::max<int64_t>(E, 1) * EP, 0);
     std::vector<int32_t> recv((size_t)std::max<int64_t>(E, 1));
     for (int64_t i = 0; i < N; i++) {
       if (rowOff[i + 1] < rowOff[i]) throw Error(WDG_E_ARG, "rowOff must not decrease");
-      for (int c = 0; c < NIN; c++) X[i * KX + c] = f2bf(x[i * NIN + c]);
+      for (int c = 0; c < NIN; c++) X[i * XP + c] = f2bf(x[i * NIN + c]);
       for (int32_t e = rowOff[i]; e < rowOff[i + 1]; e++) recv[e] = (int32_t)i;
     }
     for (int64_t e = 0; e < E; e++) {
       if (send[e] < 0 || send[e] >= N || rev[e] < 0 || rev[e] >= E) throw Error(WDG_E_ARG, "edge index out of range");
-      for (int c = 0; c < NEI; c++) F[e * KE + c] = f2bf(ef[e * NEI + c]);
+      for (int c = 0; c < NEI; c++) F[e * EP + c] = f2bf(ef[e * NEI + c]);
     }
+    bool opposite = true;
+    for (int64_t e = 0; e < E && opposite; e++)
+      opposite = rev[rev[e]] == e && send[rev[e]] == recv[e] && recv[rev[e]] == send[e];
+    std::vector<int32_t> sOff, sEdge;
+    if (!opposite) {
+      sOff.assign((size_t)N + 1, 0);
+      for (int64_t e = 0; e < E; e++) sOff[send[e] + 1]++;
+      for (int64_t i = 0; i < N; i++) sOff[i + 1] += sOff[i];
+      std::vector<int32_t> at(sOff.begin(), sOff.end() - 1);
+      sEdge.resize((size_t)E);
+      for (int64_t e = 0; e < E; e++) sEdge[at[send[e]]++] = (int32_t)e;
+    }
+    s.opposite = opposite;
     s.N = N;
     s.E = E;
     s.outRow.clear();
@@ -1052,6 +1419,11 @@ int wdg_mpnn_set_graph(wdg_mpnn* m, int64_t N, int64_t E, const float* x, const 
       WDG_HIP(hipMemcpy(s.send.p, send, E * 4, hipMemcpyHostToDevice));
       WDG_HIP(hipMemcpy(s.rev.p, rev, E * 4, hipMemcpyHostToDevice));
     }
+    if (!opposite) {
+      s.sOff.ensure(sOff.size()); s.sEdge.ensure(sEdge.size());
+      WDG_HIP(hipMemcpy(s.sOff.p, sOff.data(), sOff.size() * 4, hipMemcpyHostToDevice));
+      WDG_HIP(hipMemcpy(s.sEdge.p, sEdge.data(), sEdge.size() * 4, hipMemcpyHostToDevice));
+    }
     if (t) WDG_HIP(hipMemcpy(s.T.p, t, (size_t)N * NOUT * 4, hipMemcpyHostToDevice));
   });
 }
@@ -1061,7 +1433,7 @@ int wdg_mpnn_forward(wdg_mpnn* m, float* out) {
   if (!m) return WDG_E_ARG;
   return mguard([&] {
     Mpnn& s = m->s;
-    forward(s);
+    forward(s, false);
     if (out) out_rows(s);
     if (out && s.N > 0) {
       std::vector<float> o((size_t)s.N * NOUT);
@@ -1113,8 +1485,8 @@ int wdg_mpnn_get_graph(wdg_mpnn* m, int64_t* N, int64_t* E, int32_t* rowOff, int
       for (int64_t r = 0; r < rows; r++)
         for (int c2 = 0; c2 < used; c2++) out[r * used + c2] = bf2f(h[(size_t)r * K + c2]);
     };
-    if (x) widen(s.X, s.N, KX, NIN, x);
-    if (ef) widen(s.EF, s.E, KE, NEI, ef);
+    if (x) widen(s.X, s.N, XP, NIN, x);
+    if (ef) widen(s.EF, s.E, EP, NEI, ef);
     if (nodeRow) {
       out_rows(s);
       for (int64_t q = 0; q < s.N; q++) nodeRow[q] = s.outRow.empty() ? q : s.outRow[q];
@@ -1133,8 +1505,13 @@ int wdg_mpnn_keep_graph(wdg_mpnn* m, int32_t slot) {
     copy_buf(k.recv, s.recv, (size_t)s.E, s.stream);
     copy_buf(k.send, s.send, (size_t)s.E, s.stream);
     copy_buf(k.rev, s.rev, (size_t)s.E, s.stream);
-    copy_buf(k.X, s.X, (size_t)s.N * KX, s.stream);
-    copy_buf(k.EF, s.EF, (size_t)s.E * KE, s.stream);
+    k.opposite = s.opposite;
+    if (!s.opposite) {
+      copy_buf(k.sOff, s.sOff, (size_t)s.N + 1, s.stream);
+      copy_buf(k.sEdge, s.sEdge, (size_t)s.E, s.stream);
+    }
+    copy_buf(k.X, s.X, (size_t)s.N * XP, s.stream);
+    copy_buf(k.EF, s.EF, (size_t)s.E * EP, s.stream);
     copy_buf(k.T, s.T, (size_t)s.N * NOUT, s.stream);
     k.N = s.N;
     k.E = s.E;
@@ -1155,8 +1532,13 @@ int wdg_mpnn_use_graph(wdg_mpnn* m, int32_t slot) {
     copy_buf(s.recv, k.recv, (size_t)s.E, s.stream);
     copy_buf(s.send, k.send, (size_t)s.E, s.stream);
     copy_buf(s.rev, k.rev, (size_t)s.E, s.stream);
-    copy_buf(s.X, k.X, (size_t)s.N * KX, s.stream);
-    copy_buf(s.EF, k.EF, (size_t)s.E * KE, s.stream);
+    s.opposite = k.opposite;
+    if (!s.opposite) {
+      copy_buf(s.sOff, k.sOff, (size_t)s.N + 1, s.stream);
+      copy_buf(s.sEdge, k.sEdge, (size_t)s.E, s.stream);
+    }
+    copy_buf(s.X, k.X, (size_t)s.N * XP, s.stream);
+    copy_buf(s.EF, k.EF, (size_t)s.E * EP, s.stream);
     copy_buf(s.T, k.T, (size_t)s.N * NOUT, s.stream);
     s.outRow.clear();
     s.fromCtx = nullptr;
@@ -1169,7 +1551,7 @@ int wdg_mpnn_grad(wdg_mpnn* m, double* loss) {
   return mguard([&] {
     Mpnn& s = m->s;
     if (s.N == 0) throw Error(WDG_E_STATE, "empty graph");
-    forward(s);
+    forward(s, true);
     const double l = backward(s);
     if (loss) *loss = l;
   });
@@ -1184,9 +1566,8 @@ int wdg_mpnn_adam(wdg_mpnn* m, double lr, double b1, double b2, double eps) {
     const double c1 = 1 - std::pow(b1, (double)s.adamStep), c2 = 1 - std::pow(b2, (double)s.adamStep);
     hipLaunchKernelGGL(k_adam, dim3(nblocks((int64_t)s.L.total, 256)), dim3(256), 0, s.stream, (int64_t)s.L.total,
                        s.P.p, (const float*)s.G.p, s.Am.p, s.Av.p, (float)lr, (float)b1, (float)b2, (float)eps,
-                       (float)c1, (float)c2);
+                       (float)c1, (float)c2, img_args(s));
     WDG_LAUNCH_CHECK();
-    images(s);
     WDG_HIP(hipStreamSynchronize(s.stream));
   });
 }
@@ -1268,8 +1649,9 @@ int wdg_mpnn_graph_from_ctx(wdg_mpnn* m, wdg_ctx* ctx, double cutoff, double flo
     s.edgeOfSlot.ensure((size_t)std::max<int64_t>(2 * C.n, 2));
     s.recv.ensure((size_t)std::max<int64_t>(E, 1)); s.send.ensure((size_t)std::max<int64_t>(E, 1));
     s.rev.ensure((size_t)std::max<int64_t>(E, 1)); s.slotSide.ensure((size_t)std::max<int64_t>(E, 1));
-    s.X.ensure((size_t)std::max<int64_t>(nSph, 1) * KX);
-    s.EF.ensure((size_t)std::max<int64_t>(E, 1) * KE);
+    s.opposite = true;
+    s.X.ensure((size_t)std::max<int64_t>(nSph, 1) * XP);
+    s.EF.ensure((size_t)std::max<int64_t>(E, 1) * EP);
     s.T.ensure((size_t)std::max<int64_t>(nSph, 1) * NOUT);
     g.recv = s.recv.p; g.send = s.send.p; g.rev = s.rev.p; g.slotSide = s.slotSide.p; g.edgeOfSlot = s.edgeOfSlot.p;
     g.X = s.X.p; g.EF = s.EF.p;
