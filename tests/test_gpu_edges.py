@@ -154,6 +154,28 @@ def test_observables_over_workgroups(n, stepped):
     assert abs(d.crit_dt() / crit - 1) <= 64 * eps
 
 
+@pytest.mark.parametrize("n", [1, 32768, 32769, 43690, 43691])
+def test_fields_to_and_from_the_host(n):
+    # rows through pinned memory and directly, on both sides of the size where the way changes; the
+    # storage order differs from the user's after a refresh
+    from woo_amd._native import SPHERE, Device
+
+    rng = np.random.default_rng(n)
+    d = Device(0)
+    d.set_field(periodic=True, cell=(1., 1., 1.))
+    d.set_materials([dict(kind=0, density=1., young=1., ktDivKn=.2, tanPhi=.5, surfEnergy=0., alpha=0.)])
+    d.upload_particles(shape=np.full(n, SPHERE, np.int32), pos=rng.uniform(0., 1., (n, 3)), radius=np.full(n, 1e-3),
+                       mass=np.ones(n), inertia=np.ones((n, 3)), vel=np.zeros((n, 3)))
+    d.collide(-.05)
+    sent = {}
+    for f, w in (("vel", 3), ("ori", 4), ("mass", 1), ("inertia", 3), ("angVel", 3)):
+        sent[f] = rng.uniform(.5, 1., (n, w) if w > 1 else n)
+        d.set(f, sent[f])
+    d.collide(-.05, forceInit=True)
+    for f, a in sent.items():
+        np.testing.assert_array_equal(d.get(f), a, err_msg=f)
+
+
 @pytest.mark.parametrize("n,flat,steps", [(20, False, 1), (300, False, 7), (300, False, 130), (4900, True, 40)])
 @pytest.mark.parametrize("track", [False, True])
 def test_steps_ahead_equal_engine_calls(n, flat, steps, track):

@@ -392,6 +392,7 @@ struct Ctx {
   DBuf<double> obsPart;   // per-workgroup partial results of the observables
   DBuf<double> dynRec;    // DynDt: the stiffness record of each real contact
   DBuf<double> xfer;      // user-id-ordered staging for upload/download
+  double *hxfer = nullptr, *hxferDev = nullptr;  // the same for small fields, in pinned host memory
   DBuf<uint32_t> dflags;  // [0] dirty, [1] error bits, [2..] scratch counters
   uint32_t* hflags = nullptr;  // pinned host mirror
   // Words of the pinned mirror that the leapfrog writes itself, so that a collider call after it

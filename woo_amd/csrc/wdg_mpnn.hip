@@ -941,6 +941,8 @@ struct Mpnn {
   // graph from an engine context: the host row of each node in the output (spheres in user-id
   // order); empty for graphs given by the caller
   std::vector<int64_t> outRow;
+  DBuf<int64_t> rowDev;  // outRow on the device
+  DBuf<float> ordered;   // outputs, and targets as given, in output order
   Ctx* fromCtx = nullptr;  // the engine context of the current graph (storage order of its nodes)
   DBuf<uint32_t> degScan;
   DBuf<uint32_t> nodeUid;  // user id of each node of a graph from an engine context
@@ -980,11 +982,30 @@ static void out_rows(Mpnn& s) {
   std::vector<uint32_t> uid((size_t)s.N);
   WDG_HIP(hipMemcpyAsync(uid.data(), s.nodeUid.p, s.N * 4, hipMemcpyDeviceToHost, s.stream));
   WDG_HIP(hipStreamSynchronize(s.stream));
-  std::vector<int64_t> idx((size_t)s.N);
-  for (int64_t t = 0; t < s.N; t++) idx[t] = t;
-  std::sort(idx.begin(), idx.end(), [&](int64_t a, int64_t b) { return uid[a] < uid[b]; });
-  s.outRow.assign((size_t)s.N, 0);
-  for (int64_t r = 0; r < s.N; r++) s.outRow[idx[r]] = r;
+  // the rank of each user id among the nodes', by counting (ids are distinct and below the number of
+  // particles)
+  std::vector<int64_t> rank((size_t)*std::max_element(uid.begin(), uid.end()) + 1, 0);
+  for (const uint32_t u : uid) rank[u] = 1;
+  int64_t r = 0;
+  for (int64_t& q : rank) {
+    const int64_t here = q;
+    q = r;
+    r += here;
+  }
+  s.outRow.resize((size_t)s.N);
+  for (int64_t t = 0; t < s.N; t++) s.outRow[t] = rank[uid[t]];
+  s.rowDev.ensure((size_t)s.N);
+  WDG_HIP(hipMemcpyAsync(s.rowDev.p, s.outRow.data(), s.N * sizeof(int64_t), hipMemcpyHostToDevice, s.stream));
+  WDG_HIP(hipStreamSynchronize(s.stream));
+}
+// rows of NOUT floats between node order and output order
+__global__ __launch_bounds__(256) void k_rows(int64_t n, const int64_t* __restrict__ row, const float* __restrict__ in,
+                                               float* __restrict__ out, int toOutput) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n * NOUT) return;
+  const int64_t o = row[t / NOUT] * NOUT + t % NOUT;
+  if (toOutput) out[o] = in[t];
+  else out[t] = in[o];
 }
 
 template <class T>
@@ -1327,13 +1348,13 @@ int wdg_mpnn_create(int device, uint64_t seed, wdg_mpnn** out) {
 int wdg_mpnn_destroy(wdg_mpnn* m) {
   if (!m) return WDG_OK;
   Mpnn& s = m->s;
-  DBuf<float>* fb[] = {&s.P, &s.G, &s.Am, &s.Av, &s.T, &s.out, &s.dhA, &s.dhB, &s.S1, &s.S2, &s.part, &s.partLoss};
+  DBuf<float>* fb[] = {&s.P, &s.G, &s.Am, &s.Av, &s.T, &s.out, &s.dhA, &s.dhB, &s.S1, &s.S2, &s.part, &s.partLoss, &s.ordered};
   for (auto* b : fb) b->release();
   DBuf<bf16>* bb[] = {&s.img, &s.X, &s.EF, &s.h[0], &s.h[1], &s.h[2], &s.agg[0], &s.agg[1],
                       &s.dUb, &s.g};
   for (auto* b : bb) b->release();
   for (int l = 0; l < 2; l++) { s.mMask[l].release(); s.uMask[l].release(); }
-  s.sOff.release(); s.sEdge.release();
+  s.sOff.release(); s.sEdge.release(); s.rowDev.release();
   s.cflag.release();
   s.rowOff.release(); s.recv.release(); s.send.release(); s.rev.release();
   s.deg.release(); s.slotSide.release(); s.edgeOfSlot.release(); s.degScan.release(); s.nodeUid.release();
@@ -1436,13 +1457,16 @@ int wdg_mpnn_forward(wdg_mpnn* m, float* out) {
     forward(s, false);
     if (out) out_rows(s);
     if (out && s.N > 0) {
-      std::vector<float> o((size_t)s.N * NOUT);
-      WDG_HIP(hipMemcpyAsync(o.data(), s.out.p, o.size() * 4, hipMemcpyDeviceToHost, s.stream));
-      WDG_HIP(hipStreamSynchronize(s.stream));
-      for (int64_t t = 0; t < s.N; t++) {
-        const int64_t r = s.outRow.empty() ? t : s.outRow[t];
-        for (int c2 = 0; c2 < NOUT; c2++) out[r * NOUT + c2] = o[t * NOUT + c2];
+      const float* o = s.out.p;
+      if (!s.outRow.empty()) {
+        s.ordered.ensure((size_t)s.N * NOUT);
+        hipLaunchKernelGGL(k_rows, dim3(nblocks(s.N * NOUT, 256)), dim3(256), 0, s.stream, s.N,
+                           (const int64_t*)s.rowDev.p, (const float*)s.out.p, s.ordered.p, 1);
+        WDG_LAUNCH_CHECK();
+        o = s.ordered.p;
       }
+      WDG_HIP(hipMemcpyAsync(out, o, (size_t)s.N * NOUT * 4, hipMemcpyDeviceToHost, s.stream));
+      WDG_HIP(hipStreamSynchronize(s.stream));
     }
     // without an output the pass stays queued: wdg_mpnn_advance orders the engine's stream after it
     if (!s.fromCtx) WDG_HIP(hipStreamSynchronize(s.stream));
@@ -1455,13 +1479,18 @@ int wdg_mpnn_set_targets(wdg_mpnn* m, const float* t) {
   return mguard([&] {
     Mpnn& s = m->s;
     out_rows(s);
-    std::vector<float> T((size_t)std::max<int64_t>(s.N, 1) * NOUT);
-    for (int64_t q = 0; q < s.N; q++) {
-      const int64_t r = s.outRow.empty() ? q : s.outRow[q];
-      for (int c2 = 0; c2 < NOUT; c2++) T[q * NOUT + c2] = t[r * NOUT + c2];
+    const size_t nt = (size_t)s.N * NOUT;
+    s.T.ensure(std::max<size_t>(nt, 1));
+    if (!nt) return;
+    if (s.outRow.empty()) {
+      WDG_HIP(hipMemcpyAsync(s.T.p, t, nt * 4, hipMemcpyHostToDevice, s.stream));
+    } else {
+      s.ordered.ensure(nt);
+      WDG_HIP(hipMemcpyAsync(s.ordered.p, t, nt * 4, hipMemcpyHostToDevice, s.stream));
+      hipLaunchKernelGGL(k_rows, dim3(nblocks(s.N * NOUT, 256)), dim3(256), 0, s.stream, s.N,
+                         (const int64_t*)s.rowDev.p, (const float*)s.ordered.p, s.T.p, 0);
+      WDG_LAUNCH_CHECK();
     }
-    s.T.ensure(T.size());
-    WDG_HIP(hipMemcpyAsync(s.T.p, T.data(), (size_t)s.N * NOUT * 4, hipMemcpyHostToDevice, s.stream));
     WDG_HIP(hipStreamSynchronize(s.stream));
   });
 }

@@ -216,7 +216,7 @@ class Network:
         self.N = g.N
         out = np.empty((g.N, 3), dtype=np.float32)
         _chk(self.L.wdg_mpnn_forward(self.h, _fptr(out)))
-        return out.astype(np.float64) * A0
+        return np.multiply(out, A0, dtype=np.float64)
 
     def step_acc(self, g, gravity=(0., 0., -G)):
         """the accelerations the learned step applies: the network's for spheres in contact,
@@ -245,7 +245,7 @@ class Network:
         """forward pass on the current graph; accelerations (m/s^2) when out"""
         o = np.empty((self.N, 3), dtype=np.float32) if out else None
         _chk(self.L.wdg_mpnn_forward(self.h, _fptr(o)))
-        return None if o is None else o.astype(np.float64) * A0
+        return None if o is None else np.multiply(o, A0, dtype=np.float64)
 
     def advance(self, dev, dT):
         """the context's spheres over the coarse step dT with the last forward pass"""
