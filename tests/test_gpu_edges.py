@@ -100,6 +100,44 @@ def test_pairs_over_lanes_per_sphere(n):
     np.testing.assert_array_equal(np.sort(got, axis=1), want[np.lexsort((want[:, 1], want[:, 0]))])
 
 
+@pytest.mark.parametrize("n", [60, 700, 41000, 100001])
+def test_forces_where_pairs_outnumber_the_staging(n):
+    # a sphere with more pairs than are staged: its slots are generated again in place, in whatever
+    # order, and every sphere still sums its own contacts
+    from scipy.spatial import cKDTree
+
+    from woo_amd._native import SPHERE, Device
+
+    rng = np.random.default_rng(n)
+    m = int(np.ceil(n ** (1 / 3.)))
+    pos = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n] * 2.3e-3
+    pos = pos + rng.uniform(-1e-4, 1e-4, pos.shape)
+    pos[:45] = pos[n // 2] + rng.uniform(-.6e-3, .6e-3, (45, 3))  # 44 neighbours each
+    r = rng.uniform(.95e-3, 1.05e-3, n)
+    d = Device(0)
+    d.set_field(periodic=False)
+    E = 1e6
+    d.set_materials([dict(kind=0, density=1., young=E, ktDivKn=.2, tanPhi=.5, surfEnergy=0., alpha=0.)])
+    d.upload_particles(shape=np.full(n, SPHERE, np.int32), pos=pos, radius=r, mass=np.ones(n), inertia=np.ones((n, 3)),
+                       vel=np.zeros((n, 3)))
+    d.collide(-.05)
+    d.contact_loop(0, 1e-9)
+    got = d.get("force")
+    i, j = cKDTree(pos).query_pairs(2.2e-3, output_type="ndarray").T
+    x = pos[j] - pos[i]
+    dist = np.linalg.norm(x, axis=1)
+    k = dist < r[i] + r[j]
+    i, j, x, dist = i[k], j[k], x[k], dist[k]
+    A = np.pi * np.minimum(r[i], r[j]) ** 2
+    F = (1 / (1 / (E * A / r[i]) + 1 / (E * A / r[j])) * (dist - r[i] - r[j]) / dist)[:, None] * x
+    want, size = np.zeros((n, 3)), np.zeros((n, 3))
+    for s, e in ((1., i), (-1., j)):
+        np.add.at(want, e, s * F)
+        np.add.at(size, e, np.abs(F))
+    # a few dozen roundings per term, the overlap's cancellation in uN included
+    assert np.all(np.abs(got - want) <= 1e-12 * (size + size.max()))
+
+
 @pytest.mark.parametrize("n", [2, 255, 257, 5000, 262145 + 300])
 @pytest.mark.parametrize("stepped", [False, True])
 def test_observables_over_workgroups(n, stepped):

@@ -1861,10 +1861,12 @@ static void refresh(Ctx& c) {
     nPairs = c.hflags[4];
     overflow = c.hflags[7] > (uint32_t)PS;
     if (overflow) c.pairStage = (int)std::min<uint32_t>(96u, (c.hflags[7] + 7u) / 8u * 8u);
-    nbFits = c.hflags[8] <= (uint32_t)NS;
+    // (pairs generated again in place: the passes that stage and that do not work off their queues in
+    // different rounds, so the staged neighbours do not tell the slots' order then)
+    nbFits = !overflow && c.hflags[8] <= (uint32_t)NS;
     // a sphere with more neighbours than staged sends the adjacency to the general path; the
     // next refreshes stage more (up to 128)
-    if (!nbFits) c.nbStage = (int)std::min<uint32_t>(128u, (c.hflags[8] + 7u) / 8u * 8u);
+    if (c.hflags[8] > (uint32_t)NS) c.nbStage = (int)std::min<uint32_t>(128u, (c.hflags[8] + 7u) / 8u * 8u);
   }
   Contacts& O = c.con();
   const int64_t nOld = O.n;
