@@ -192,6 +192,38 @@ def test_observables_over_workgroups(n, stepped):
     assert abs(d.crit_dt() / crit - 1) <= 64 * eps
 
 
+@pytest.mark.parametrize("n", [1, 2, 511, 4095, 4096, 4097, 9000])
+def test_long_lists_of_a_floor(n):
+    # a floor's list sorted by one workgroup up to 4,096 entries, by the radix sort above; the force on
+    # the floor is summed in that order whichever way it was sorted, and is that of the engine's
+    # unsorted contacts up to rounding
+    from woo_amd._native import SPHERE, WALL, Device
+
+    rng = np.random.default_rng(n)
+    m = int(np.ceil(n ** .5))
+    r = 1e-3
+    xy = (np.stack(np.meshgrid(np.arange(m), np.arange(m), indexing="ij"), -1).reshape(-1, 2)[:n] + .5) * 2.3e-3
+    z = rng.uniform(.97, .99, n) * r
+    pos = np.column_stack([xy, z])[rng.permutation(n)]
+    wall = np.zeros((1, 3))
+    d = Device(0)
+    d.set_field(periodic=False)
+    E = 1e6
+    d.set_materials([dict(kind=0, density=1., young=E, ktDivKn=.2, tanPhi=.5, surfEnergy=0., alpha=0.)])
+    d.upload_particles(shape=np.array([WALL] + [SPHERE] * n, np.int32), pos=np.vstack([wall, pos]),
+                       radius=np.r_[0., np.full(n, r)], mass=np.ones(n + 1), inertia=np.ones((n + 1, 3)),
+                       vel=np.zeros((n + 1, 3)), wallAxis=np.r_[2, np.zeros(n)].astype(np.int32))
+    out = []
+    for _ in range(2):
+        d.force_reset()
+        d.collide(-.05, forceInit=True)
+        d.contact_loop(0, 1e-9)
+        out.append(d.get("force"))
+    np.testing.assert_array_equal(out[0], out[1])
+    F = E * np.pi * r * (pos[:, 2] - r) / 2.  # two equal lengths in series
+    assert abs(out[0][0, 2] - F.sum()) <= 1e-12 * np.abs(F).sum() * (r / np.abs(pos[:, 2] - r).min())
+
+
 @pytest.mark.parametrize("n", [1, 32768, 32769, 43690, 43691])
 def test_fields_to_and_from_the_host(n):
     # rows through pinned memory and directly, on both sides of the size where the way changes; the

@@ -176,10 +176,11 @@ static inline double ord_to_double(unsigned long long b) {
   return d;
 }
 
-// bounding box of the spheres: a grid-stride loop of few workgroups, each reducing in
-// registers, across its wavefronts in LDS, and then with one atomic per bound (device-wide
-// atomics on one line serialise across the XCDs, so they are kept to a few thousand)
-constexpr int BBOX_BLOCKS = 512;
+// bounding box of the spheres: a grid-stride loop of few workgroups, each reducing in registers and
+// across its wavefronts in LDS to six words; k_bbox_all takes those of all workgroups, to pinned
+// memory: 4 + 2 us at 60,000 spheres (8 us with an atomic of every workgroup on one line, and two
+// copies to set it up and read it back)
+constexpr int BBOX_BLOCKS = 256;
 __global__ __launch_bounds__(256) void k_bbox(int64_t s0, int64_t n, const double* __restrict__ px,
                                               const double* __restrict__ py, const double* __restrict__ pz,
                                               unsigned long long* out) {
@@ -212,9 +213,23 @@ __global__ __launch_bounds__(256) void k_bbox(int64_t s0, int64_t n, const doubl
     const int k = threadIdx.x;
     unsigned long long v = sm[0][k];
     for (int w = 1; w < 4; w++) v = k < 3 ? (sm[w][k] < v ? sm[w][k] : v) : (sm[w][k] > v ? sm[w][k] : v);
-    if (k < 3) atomicMin(&out[k], v);
-    else atomicMax(&out[k], v);
+    out[6 * (int64_t)blockIdx.x + k] = v;
   }
+}
+// one wavefront per bound; the result in pinned host memory
+__global__ __launch_bounds__(384) void k_bbox_all(int nb, const unsigned long long* __restrict__ part,
+                                                  unsigned long long* out) {
+  const int k = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  unsigned long long v = k < 3 ? ~0ull : 0ull;
+  for (int b = lane; b < nb; b += 64) {
+    const unsigned long long x = part[6 * b + k];
+    v = k < 3 ? (x < v ? x : v) : (x > v ? x : v);
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    const unsigned long long x = __shfl_xor(v, off);
+    v = k < 3 ? (x < v ? x : v) : (x > v ? x : v);
+  }
+  if (lane == 0) out[k] = v;
 }
 
 // bucket of cell (c0, c1, c2) in hashed mode: the coordinates packed into 63 bits and mixed
@@ -930,7 +945,10 @@ static void launch_pairs(Ctx& c, const PairArgs& a) {
 }
 
 // largest of the per-workgroup maxima of k_pairs, one workgroup
-__global__ __launch_bounds__(1024) void k_block_max(int64_t nb, const uint32_t* __restrict__ bmax, uint32_t* out) {
+// (and the number of pairs, dflags[4]: all three to the host's pinned words 4, 7 and 8; the merge's
+// counter of extra slots is cleared on the way)
+__global__ __launch_bounds__(1024) void k_block_max(int64_t nb, const uint32_t* __restrict__ bmax, uint32_t* dflags,
+                                                     uint32_t* host) {
   __shared__ uint32_t sm[2][16];
   uint32_t m0 = 0, m1 = 0;
   for (int64_t i = threadIdx.x; i < nb; i += blockDim.x) {
@@ -949,8 +967,10 @@ __global__ __launch_bounds__(1024) void k_block_max(int64_t nb, const uint32_t* 
   if (threadIdx.x < 2) {
     uint32_t m = 0;
     for (int w = 0; w < (int)(blockDim.x >> 6); w++) m = max(m, sm[threadIdx.x][w]);
-    out[threadIdx.x] = m;
+    host[7 + threadIdx.x] = m;
   }
+  if (threadIdx.x == 2) host[4] = dflags[4];
+  if (threadIdx.x == 3) dflags[6] = 0u;
 }
 
 // staged pairs -> slot list. The 64 spheres of a wavefront write one contiguous range of slots:
@@ -1155,8 +1175,9 @@ __global__ __launch_bounds__(256) void k_wall_fill(int64_t nc, int64_t nW, const
                                                    const uint32_t* __restrict__ B, const uint32_t* __restrict__ info,
                                                    const uint32_t* __restrict__ uid,
                                                    const uint32_t* __restrict__ adjOff, uint32_t* cursor,
-                                                   uint64_t* ent) {
+                                                   uint64_t* ent, int64_t n) {
   __shared__ uint32_t cnt[WD_LDS];
+  if (adjOff[n] != (uint32_t)(2 * nc)) return;
   const bool inLds = nW <= WD_LDS;
   if (inLds)
     for (int64_t k = threadIdx.x; k < nW; k += blockDim.x) cnt[k] = 0u;
@@ -1180,6 +1201,70 @@ __global__ __launch_bounds__(256) void k_wall_fill(int64_t nc, int64_t nW, const
   const bool swap = (info[t] & CI_SWAP) != 0u;
   const uint32_t pos = (inLds ? cnt[lo] : 0u) + loc;
   ent[adjOff[lo] + pos] = ((uint64_t)uid[hi] << 32) | (uint32_t)t | (swap ? 0u : ADJ_PA);
+}
+
+// Each boundary body's entries sorted by the other particle's user id, in LDS by one workgroup
+// (bitonic): lists up to WS_CAP entries; RW_LONGEST tells the host of longer ones. Instead of marks,
+// scans, a gather, two to four radix passes and a scatter over all of them, with a wait for their
+// number: 4 us for the walls of 2,000 spheres, 7 us for a floor under 60,000, against some 60.
+constexpr int WS_BS = 512;
+constexpr uint32_t WS_CAP = 4096;
+__global__ __launch_bounds__(WS_BS) void k_wall_sort(const uint32_t* __restrict__ adjOff, int64_t n, uint32_t want,
+                                                     const uint64_t* __restrict__ ent, uint32_t* __restrict__ adj) {
+  __shared__ uint64_t key[WS_CAP];
+  const uint32_t k0 = adjOff[blockIdx.x], m = adjOff[blockIdx.x + 1] - k0;
+  if (adjOff[n] != want || m == 0u || m > WS_CAP) return;
+  uint32_t P = 2u;
+  while (P < m) P <<= 1;
+  for (uint32_t t = threadIdx.x; t < P; t += WS_BS) key[t] = t < m ? ent[k0 + t] : ~0ull;
+  __syncthreads();
+  for (uint32_t size = 2u; size <= P; size <<= 1)
+    for (uint32_t step = size >> 1; step > 0u; step >>= 1) {
+      for (uint32_t t = threadIdx.x; t < (P >> 1); t += WS_BS) {
+        const uint32_t a = 2u * t - (t & (step - 1u)), b = a + step;
+        const bool up = (a & size) == 0u;
+        const uint64_t x = key[a], y = key[b];
+        if ((x > y) == up) {
+          key[a] = y;
+          key[b] = x;
+        }
+      }
+      __syncthreads();
+    }
+  for (uint32_t t = threadIdx.x; t < m; t += WS_BS) adj[k0 + t] = (uint32_t)key[t];
+}
+
+// what the host needs of a finished refresh, to its pinned words; the displacement flag is cleared.
+// staged: lists longer than k_wall_sort takes are not sorted yet (WALL_LONG stops k_ent_pos).
+enum { RW_ENTRIES, RW_LONGEST, RW_GATHERED, RW_EXTRA, RW_ERR };
+__global__ __launch_bounds__(256) void k_refresh_words(int64_t n, int64_t nW, int64_t nG,
+                                                       const uint32_t* __restrict__ gbody,
+                                                       const uint32_t* __restrict__ adjOff, int merged, int staged,
+                                                       uint32_t* dflags, uint32_t* host) {
+  __shared__ uint32_t wm[4][2];
+  uint32_t all = 0u, ga = 0u;
+  for (int64_t b = threadIdx.x; b < nW; b += 256) all = max(all, adjOff[b + 1] - adjOff[b]);
+  for (int64_t q = threadIdx.x; q < nG; q += 256) ga = max(ga, adjOff[gbody[q] + 1] - adjOff[gbody[q]]);
+  for (int off = 32; off > 0; off >>= 1) {
+    all = max(all, (uint32_t)__shfl_xor(all, off));
+    ga = max(ga, (uint32_t)__shfl_xor(ga, off));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    wm[threadIdx.x >> 6][0] = all;
+    wm[threadIdx.x >> 6][1] = ga;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    all = max(max(wm[0][0], wm[1][0]), max(wm[2][0], wm[3][0]));
+    ga = max(max(wm[0][1], wm[1][1]), max(wm[2][1], wm[3][1]));
+    host[RW_ENTRIES] = adjOff[n];
+    host[RW_LONGEST] = all;
+    host[RW_GATHERED] = ga;
+    host[RW_EXTRA] = merged ? dflags[6] : 0u;
+    host[RW_ERR] = dflags[1];
+    dflags[WALL_LONG] = staged && all > WS_CAP ? 1u : 0u;
+    dflags[0] = 0u;
+  }
 }
 
 // each particle's entries sorted by the other particle's user id (the order of
@@ -1250,6 +1335,7 @@ struct AdjArgs {
   uint64_t* ent;
   uint32_t* adj;
   uint32_t* dflags;
+  uint32_t want;  // entries that the lists must hold
 };
 // Storage indices: boundary bodies [0, nW), spheres from nW; sphere t is storage nW + t and its
 // generated pairs are off[t] .. off[t] + count[t]. Sphere p generated the pair with j when j is
@@ -1300,6 +1386,7 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) void k_adj_sym(AdjArgs a) {
   // the wavefront's first sphere
   const int64_t tw = ((int64_t)xcd_block(blockIdx.x, gridDim.x) * ADJ_WAVES + w) * 64;
   if (tw >= a.nSph) return;  // whole wavefront; no workgroup barrier below
+  if (a.adjOff[a.nW + a.nSph] != a.want) return;
   const int64_t t = tw + lane;
   const bool live = t < a.nSph;
   const uint32_t m = live ? a.deg[t] : 0u, k0 = live ? a.adjOff[a.nW + t] : 0u;
@@ -1390,10 +1477,11 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) void k_adj_sym(AdjArgs a) {
 
 // the inverse of the adjacency: per slot the positions of its pA entry and its pB entry; every
 // entry starts at NO_STATE, and the next filter writes those of every real slot
-__global__ void k_ent_pos(int64_t nEnt, const uint32_t* __restrict__ adj, uint32_t* entPos, uint32_t* eidx,
-                          uint32_t* full) {
+__global__ void k_ent_pos(int64_t nEnt, const uint32_t* __restrict__ adj, const uint32_t* __restrict__ total,
+                          uint32_t* entPos, uint32_t* eidx, uint32_t* dflags) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e == 0) *full = 1u;
+  if (*total != (uint32_t)nEnt || dflags[WALL_LONG] != 0u) return;
+  if (e == 0) dflags[EIDX_FULL] = 1u;
   if (e >= nEnt) return;
   const uint32_t v = adj[e];
   entPos[2 * (int64_t)(v & ~ADJ_PA) + ((v & ADJ_PA) ? 0 : 1)] = (uint32_t)e;
@@ -1612,15 +1700,18 @@ static void refresh(Ctx& c) {
       g.org[k] = 0;
     }
   } else if (nSph > 0) {
-    unsigned long long init[6] = {~0ull, ~0ull, ~0ull, 0, 0, 0};
-    unsigned long long* dbb = reinterpret_cast<unsigned long long*>(c.red.p);
-    WDG_HIP(hipMemcpyAsync(dbb, init, sizeof(init), hipMemcpyHostToDevice, c.stream));
-    hipLaunchKernelGGL(k_bbox, dim3((unsigned)std::min<int64_t>(nblocks(nSph, 256), BBOX_BLOCKS)), dim3(256), 0,
-                       c.stream, nW, n, c.pos[0].p, c.pos[1].p, c.pos[2].p, dbb);
+    const int nbb = (int)std::min<int64_t>(nblocks(nSph, 256), BBOX_BLOCKS);
+    c.obsPart.ensure((size_t)6 * BBOX_BLOCKS);
+    unsigned long long* dbb = reinterpret_cast<unsigned long long*>(c.obsPart.p);
+    hipLaunchKernelGGL(k_bbox, dim3((unsigned)nbb), dim3(256), 0, c.stream, nW, n, c.pos[0].p, c.pos[1].p, c.pos[2].p,
+                       dbb);
     WDG_LAUNCH_CHECK();
-    unsigned long long hb[6];
-    WDG_HIP(hipMemcpyAsync(hb, dbb, sizeof(hb), hipMemcpyDeviceToHost, c.stream));
+    hipLaunchKernelGGL(k_bbox_all, dim3(1), dim3(384), 0, c.stream, nbb, (const unsigned long long*)dbb,
+                       reinterpret_cast<unsigned long long*>(c.hresDev));
+    WDG_LAUNCH_CHECK();
     WDG_HIP(hipStreamSynchronize(c.stream));
+    unsigned long long hb[6];
+    std::memcpy(hb, c.hres, sizeof(hb));
     double lo[3], hi[3];
     for (int k = 0; k < 3; k++) {
       lo[k] = ord_to_double(hb[k]);
@@ -1852,11 +1943,10 @@ static void refresh(Ctx& c) {
     c.pairMax.ensure(2 * npb);
     pa.bmax = c.pairMax.p;
     launch_pairs<OUT_STAGE, MODE_NEAR>(c, pa);
-    hipLaunchKernelGGL(k_block_max, dim3(1), dim3(1024), 0, c.stream, npb, (const uint32_t*)c.pairMax.p,
-                       c.dflags.p + 7);
-    WDG_LAUNCH_CHECK();
     scan_exclusive(c, c.scount.p, c.soff.p, nSph, c.dflags.p + 4);
-    WDG_HIP(hipMemcpyAsync(c.hflags, c.dflags.p, 9 * sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream));
+    hipLaunchKernelGGL(k_block_max, dim3(1), dim3(1024), 0, c.stream, npb, (const uint32_t*)c.pairMax.p, c.dflags.p,
+                       c.hflagsDev);
+    WDG_LAUNCH_CHECK();
     WDG_HIP(hipStreamSynchronize(c.stream));
     nPairs = c.hflags[4];
     overflow = c.hflags[7] > (uint32_t)PS;
@@ -1887,9 +1977,8 @@ static void refresh(Ctx& c) {
     WDG_LAUNCH_CHECK();
   }
   // 3. merge with the old real contacts (history)
-  int64_t nExtra = 0;
-  if (nOld > 0 && nSph > 0) {
-    WDG_HIP(hipMemsetAsync(c.dflags.p + 6, 0, sizeof(uint32_t), c.stream));
+  const bool merged = nOld > 0 && nSph > 0;
+  if (merged) {
     MergeArgs ma{};
     ma.nOld = nOld; ma.nW = nW; ma.nPairs = nPairs; ma.ov = c.rview();
     ma.oA = O.A.p; ma.oB = O.B.p; ma.oInfo = O.info.p; ma.oDist = O.dist.p; ma.invPerm = c.invPerm.p;
@@ -1898,101 +1987,122 @@ static void refresh(Ctx& c) {
     ma.nExtra = c.dflags.p + 6;
     hipLaunchKernelGGL(k_merge, dim3(nblocks(nOld, 256)), dim3(256), 0, c.stream, ma);
     WDG_LAUNCH_CHECK();
-    nExtra = read_u32(c, c.dflags.p + 6);
   }
-  const int64_t nNew = nPairs + nExtra;
-  N.n = nNew;
-  // real set of the new list: the carried contacts, with their state moved to the new indices
   const int rNew = 1 - c.rcur;
-  reals_from_flags(c, N.carry.p, nNew, rNew);
-  if (nNew > 0) {
-    Reals &RO = c.R[c.rcur], &RN = c.R[rNew];
-    CarryArgs ya{};
-    ya.n = nNew; ya.carry = N.carry.p; ya.ov = c.rview(c.rcur); ya.nv = c.rview(rNew);
-    DBuf<double>* so[10] = {&RO.hN[0], &RO.hN[1], &RO.hN[2], &RO.hY[0], &RO.hY[1],
-                            &RO.hY[2], &RO.hF[0], &RO.hF[1], &RO.hF[2], &RO.huN};
-    DBuf<double>* sn[10] = {&RN.hN[0], &RN.hN[1], &RN.hN[2], &RN.hY[0], &RN.hY[1],
-                            &RN.hY[2], &RN.hF[0], &RN.hF[1], &RN.hF[2], &RN.huN};
-    for (int q = 0; q < 10; q++) { ya.o[q] = so[q]->p; ya.d[q] = sn[q]->p; }
-    ya.ogp = RO.gp.p; ya.gp = RN.gp.p;
-    if (c.matEpochs > 1) { ya.oE = RO.hE.p; ya.nE = RN.hE.p; }
-    if (c.rollActive) {
-      RN.ensureRoll(nNew);
-      ya.ogt = RO.gtq.p;
-      ya.gt = RN.gtq.p;
-    }
-    hipLaunchKernelGGL(c.precision == 32 ? k_carry_state<32> : k_carry_state<64>, dim3(nblocks(nNew, 256)),
-                       dim3(256), 0, c.stream, ya);
-    WDG_LAUNCH_CHECK();
-  }
-  // 4. per-particle adjacency in canonical order (particle storage, other user id)
-  if (nExtra == 0 && nbFits) {
-    // every slot is a near pair that its spheres staged: spheres' lists straight from the staged
-    // neighbours (bodies included); the bodies' lists from the slot list
-    if (nW > 0) {
-      c.adjDeg.ensure(n + 1);
-      WDG_HIP(hipMemsetAsync(c.adjDeg.p, 0, nW * sizeof(uint32_t), c.stream));
-      if (nNew > 0) {
-        hipLaunchKernelGGL(k_wall_deg, dim3(nblocks(nNew, 256)), dim3(256), 0, c.stream, nNew, nW,
-                           (const uint32_t*)N.A.p, c.adjDeg.p);
-        WDG_LAUNCH_CHECK();
-      }
-      if (nSph > 0) {
-        hipLaunchKernelGGL(k_copy_deg, dim3(nblocks(nSph, 256)), dim3(256), 0, c.stream, nSph, nW,
-                           (const uint32_t*)c.sdeg.p, c.adjDeg.p);
-        WDG_LAUNCH_CHECK();
-      }
-      scan_exclusive(c, c.adjDeg.p, N.adjOff.p, n, N.adjOff.p + n);
-    } else {
-      scan_exclusive(c, c.sdeg.p, N.adjOff.p, n, N.adjOff.p + n);
-    }
-    // both ends of every pair listed it: the lists hold two entries per slot
-    const int64_t nEnt = read_u32(c, N.adjOff.p + n);
-    if (nEnt != 2 * nNew)
-      throw Error(WDG_E_STATE, "broadphase: neighbour lists disagree with the pair list (" + std::to_string(nEnt) +
-                                   " entries for " + std::to_string(nNew) + " pairs)");
+  // The rest is launched for a merge without extra slots (the old real contacts are all near, the
+  // rule while the skin holds), and its counts are read in one wait at the end. Where the merge did
+  // append some, the real set and the adjacency are made again with them.
+  int64_t nNew = nPairs;
+  const uint32_t* hw = c.hflags + HOST_REFRESH;
+  for (int64_t nExtra = 0;;) {
+    nNew = nPairs + nExtra;
+    N.n = nNew;
+    // real set of the new list: the carried contacts, with their state moved to the new indices
+    reals_from_flags(c, N.carry.p, nNew, rNew);
     if (nNew > 0) {
-      c.adjEnt.ensure(2 * nNew);
-      AdjArgs aa{};
-      aa.nSph = nSph; aa.nW = nW; aa.nb = c.stNb.p; aa.deg = c.sdeg.p; aa.count = c.scount.p; aa.off = c.soff.p;
-      aa.B = N.B.p; aa.uid = c.uid.p; aa.adjOff = N.adjOff.p; aa.ent = c.adjEnt.p; aa.adj = N.adj.p;
-      aa.dflags = c.dflags.p;
-      hipLaunchKernelGGL(k_adj_sym, dim3(nblocks(nSph, 64 * ADJ_WAVES)), dim3(64 * ADJ_WAVES), 0, c.stream, aa);
-      WDG_LAUNCH_CHECK();
-      if (nW > 0) {
-        WDG_HIP(hipMemsetAsync(c.adjDeg.p, 0, nW * sizeof(uint32_t), c.stream));
-        hipLaunchKernelGGL(k_wall_fill, dim3(nblocks(nNew, 256)), dim3(256), 0, c.stream, nNew, nW,
-                           (const uint32_t*)N.A.p, (const uint32_t*)N.B.p, (const uint32_t*)N.info.p,
-                           (const uint32_t*)c.uid.p, (const uint32_t*)N.adjOff.p, c.adjDeg.p, c.adjEnt.p);
-        WDG_LAUNCH_CHECK();
-        // the bodies' lists are few and long: all by the radix sort
-        sort_lists(c, N, nW, 0);
+      Reals &RO = c.R[c.rcur], &RN = c.R[rNew];
+      CarryArgs ya{};
+      ya.n = nNew; ya.carry = N.carry.p; ya.ov = c.rview(c.rcur); ya.nv = c.rview(rNew);
+      DBuf<double>* so[10] = {&RO.hN[0], &RO.hN[1], &RO.hN[2], &RO.hY[0], &RO.hY[1],
+                              &RO.hY[2], &RO.hF[0], &RO.hF[1], &RO.hF[2], &RO.huN};
+      DBuf<double>* sn[10] = {&RN.hN[0], &RN.hN[1], &RN.hN[2], &RN.hY[0], &RN.hY[1],
+                              &RN.hY[2], &RN.hF[0], &RN.hF[1], &RN.hF[2], &RN.huN};
+      for (int q = 0; q < 10; q++) { ya.o[q] = so[q]->p; ya.d[q] = sn[q]->p; }
+      ya.ogp = RO.gp.p; ya.gp = RN.gp.p;
+      if (c.matEpochs > 1) { ya.oE = RO.hE.p; ya.nE = RN.hE.p; }
+      if (c.rollActive) {
+        RN.ensureRoll(nNew);
+        ya.ogt = RO.gtq.p;
+        ya.gt = RN.gtq.p;
       }
+      hipLaunchKernelGGL(c.precision == 32 ? k_carry_state<32> : k_carry_state<64>, dim3(nblocks(nNew, 256)),
+                         dim3(256), 0, c.stream, ya);
+      WDG_LAUNCH_CHECK();
     }
-  } else {
-    build_adjacency_atomic(c, N, nNew);
-  }
-  if (nNew > 0) {
-    hipLaunchKernelGGL(k_ent_pos, dim3(nblocks(2 * nNew, 256)), dim3(256), 0, c.stream, 2 * nNew,
-                       (const uint32_t*)N.adj.p, N.entPos.p, N.eidx.p, c.dflags.p + EIDX_FULL);
+    // 4. per-particle adjacency in canonical order (particle storage, other user id)
+    const bool staged = nExtra == 0 && nbFits;
+    if (staged) {
+      // every slot is a near pair that its spheres staged: spheres' lists straight from the staged
+      // neighbours (bodies included); the bodies' lists from the slot list
+      if (nW > 0) {
+        c.adjDeg.ensure(n + 1);
+        WDG_HIP(hipMemsetAsync(c.adjDeg.p, 0, nW * sizeof(uint32_t), c.stream));
+        if (nNew > 0) {
+          hipLaunchKernelGGL(k_wall_deg, dim3(nblocks(nNew, 256)), dim3(256), 0, c.stream, nNew, nW,
+                             (const uint32_t*)N.A.p, c.adjDeg.p);
+          WDG_LAUNCH_CHECK();
+        }
+        if (nSph > 0) {
+          hipLaunchKernelGGL(k_copy_deg, dim3(nblocks(nSph, 256)), dim3(256), 0, c.stream, nSph, nW,
+                             (const uint32_t*)c.sdeg.p, c.adjDeg.p);
+          WDG_LAUNCH_CHECK();
+        }
+        scan_exclusive(c, c.adjDeg.p, N.adjOff.p, n, N.adjOff.p + n);
+      } else {
+        scan_exclusive(c, c.sdeg.p, N.adjOff.p, n, N.adjOff.p + n);
+      }
+      // both ends of every pair listed it, so the lists hold two entries per slot: the kernels check
+      // that themselves (and write nothing otherwise), the host at the end
+      if (nNew > 0) {
+        c.adjEnt.ensure(2 * nNew);
+        AdjArgs aa{};
+        aa.nSph = nSph; aa.nW = nW; aa.nb = c.stNb.p; aa.deg = c.sdeg.p; aa.count = c.scount.p; aa.off = c.soff.p;
+        aa.B = N.B.p; aa.uid = c.uid.p; aa.adjOff = N.adjOff.p; aa.ent = c.adjEnt.p; aa.adj = N.adj.p;
+        aa.dflags = c.dflags.p;
+        aa.want = (uint32_t)(2 * nNew);
+        hipLaunchKernelGGL(k_adj_sym, dim3(nblocks(nSph, 64 * ADJ_WAVES)), dim3(64 * ADJ_WAVES), 0, c.stream, aa);
+        WDG_LAUNCH_CHECK();
+        if (nW > 0) {
+          WDG_HIP(hipMemsetAsync(c.adjDeg.p, 0, nW * sizeof(uint32_t), c.stream));
+          hipLaunchKernelGGL(k_wall_fill, dim3(nblocks(nNew, 256)), dim3(256), 0, c.stream, nNew, nW,
+                             (const uint32_t*)N.A.p, (const uint32_t*)N.B.p, (const uint32_t*)N.info.p,
+                             (const uint32_t*)c.uid.p, (const uint32_t*)N.adjOff.p, c.adjDeg.p, c.adjEnt.p, n);
+          WDG_LAUNCH_CHECK();
+          hipLaunchKernelGGL(k_wall_sort, dim3((unsigned)nW), dim3(WS_BS), 0, c.stream, (const uint32_t*)N.adjOff.p, n,
+                             (uint32_t)(2 * nNew), (const uint64_t*)c.adjEnt.p, N.adj.p);
+          WDG_LAUNCH_CHECK();
+        }
+      }
+    } else {
+      build_adjacency_atomic(c, N, nNew);
+    }
+    auto ent_pos = [&]() {
+      if (nNew == 0) return;
+      hipLaunchKernelGGL(k_ent_pos, dim3(nblocks(2 * nNew, 256)), dim3(256), 0, c.stream, 2 * nNew,
+                         (const uint32_t*)N.adj.p, (const uint32_t*)(N.adjOff.p + n), N.entPos.p, N.eidx.p,
+                         c.dflags.p);
+      WDG_LAUNCH_CHECK();
+    };
+    hipLaunchKernelGGL(k_refresh_words, dim3(1), dim3(256), 0, c.stream, n, nW, c.nGBody, (const uint32_t*)c.gbody.p,
+                       (const uint32_t*)N.adjOff.p, merged ? 1 : 0, staged ? 1 : 0, c.dflags.p,
+                       c.hflagsDev + HOST_REFRESH);
     WDG_LAUNCH_CHECK();
-  }
-  if (c.nGBody > 0) {
-    // the boundary-body gather cuts each list into parts of about 2048 entries
-    std::vector<uint32_t> off((size_t)nW + 1);
-    WDG_HIP(hipMemcpyAsync(off.data(), N.adjOff.p, (nW + 1) * sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream));
+    ent_pos();
     WDG_HIP(hipStreamSynchronize(c.stream));
-    uint32_t mx = 0;
-    for (uint32_t b : c.gbodyHost) mx = std::max(mx, off[b + 1] - off[b]);
-    c.bndParts = (int)std::min<uint32_t>(64u, std::max<uint32_t>(1u, (mx + 2047u) / 2048u));
+    if (nExtra == 0 && hw[RW_EXTRA] > 0) {
+      nExtra = hw[RW_EXTRA];
+      continue;
+    }
+    if (hw[RW_ENTRIES] != 2 * (uint64_t)nNew)
+      throw Error(WDG_E_STATE, "broadphase: neighbour lists disagree with the pair list (" +
+                                   std::to_string(hw[RW_ENTRIES]) + " entries for " + std::to_string(nNew) + " pairs)");
+    if (staged && hw[RW_LONGEST] > WS_CAP) {
+      // bodies with longer lists than a workgroup sorts: all by the radix sort
+      sort_lists(c, N, nW, 0);
+      WDG_HIP(hipMemsetAsync(c.dflags.p + WALL_LONG, 0, sizeof(uint32_t), c.stream));
+      ent_pos();
+    }
+    break;
   }
+  // the boundary-body gather cuts each list into parts of about 2048 entries
+  if (c.nGBody > 0)
+    c.bndParts = (int)std::min<uint32_t>(64u, std::max<uint32_t>(1u, (hw[RW_GATHERED] + 2047u) / 2048u));
   c.eidxValid = false;
   c.eidxClean = true;
   c.cur = 1 - c.cur;
   c.rcur = rNew;
   c.boundsValid = true;
-  WDG_HIP(hipMemsetAsync(c.dflags.p, 0, sizeof(uint32_t), c.stream));
-  uint32_t err = read_u32(c, c.dflags.p + 1);
+  const uint32_t err = hw[RW_ERR];
   c.dirtyKnown = true;
   c.dirtyIdx = 0;
   if (err) {

@@ -39,6 +39,7 @@ constexpr uint32_t EIDX_PA = 0x80000000u;
 // dflags word: set when Contacts::eidx was reset, so that the next filter writes the entries of
 // every real slot (else only of the slots whose real state changed); cleared by the force pass
 constexpr int EIDX_FULL = 48;
+constexpr int WALL_LONG = 49;  // refresh: a boundary body's list is too long for k_wall_sort
 
 // ------------------------------------------------------------------ particle flag bits
 // low bits are DemData.flags (Particle.hpp:196-199); high bits are engine-private
@@ -82,6 +83,7 @@ __host__ __device__ inline int unpack_cd(uint64_t v, int k) {
 // [DIRTY_PP + 0/1] dirty flags set by alternate leapfrog launches (each launch clears the other)
 constexpr int DIRTY_PP = 12;
 constexpr int HOST_DIRTY = 40, HOST_ERR = 41;  // words of the pinned host mirror only
+constexpr int HOST_REFRESH = 52;               // likewise, what a refresh leaves for the host
 constexpr int HOST_RES = 64, HOST_WORDS = 128;  // its words from HOST_RES on hold doubles
 
 // device error bits
