@@ -243,116 +243,116 @@ __global__ __launch_bounds__(LY_BS, 3) void k_layer(LayerArgs a) {
     bool touch = false;
     for (int pass = 0; pass < 2; pass++) {
 #pragma unroll
-    for (int cb = 0; cb < 4; cb++) agg[cb] = floatx4{0, 0, 0, 0};
-    int32_t rc[2], sd[2];
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const int32_t e = max(min(e0 + 16 * q + r, e1 - 1), 0);
-      rc[q] = e0 < e1 ? a.recv[e] : 0;
-      sd[q] = e0 < e1 ? a.send[e] : 0;
-    }
-    for (int32_t eb = e0; eb < e1; eb += 32) {
-      uint4 z[2][5];
+      for (int cb = 0; cb < 4; cb++) agg[cb] = floatx4{0, 0, 0, 0};
+      int32_t rc[2], sd[2];
 #pragma unroll
       for (int q = 0; q < 2; q++) {
-        // past the last edge: that edge again (it counts for no node below, and no load is
-        // conditional)
-        const int32_t e = min(eb + 16 * q + r, e1 - 1);
-        const int64_t er = rc[q], es = sd[q];
-        const int32_t en = min(eb + 32 + 16 * q + r, e1 - 1);  // the next ends, a chunk ahead
-        rc[q] = a.recv[en];
-        sd[q] = a.send[en];
-        z[q][4] = row8(a.ef + (int64_t)e * EP + 8 * (g & 1));
-        if (g >= 2) z[q][4] = ZERO4;  // columns 16 .. 31 are zero
-        z[q][0] = row8(a.h + er * H + 8 * g);
-        z[q][1] = row8(a.h + er * H + 32 + 8 * g);
-        z[q][2] = row8(a.h + es * H + 8 * g);
-        z[q][3] = row8(a.h + es * H + 32 + 8 * g);
-        if (LAST) {
-          // overlap inputs (column 3, in the lanes of group 0) of this half's edges, against the
-          // lane's node's range of them
-          const uint64_t pos = __ballot(bf2f((bf16)(z[q][4].y >> 16)) > 0.f) & 0xFFFFull;
-          const int lo = min(max(b0 - (eb + 16 * q), 0), 16), hi = min(max(b1 - (eb + 16 * q), 0), 16);
-          touch = touch || ((uint32_t)pos & ((1u << hi) - 1u) & ~((1u << lo) - 1u)) != 0u;
-        }
+        const int32_t e = max(min(e0 + 16 * q + r, e1 - 1), 0);
+        rc[q] = e0 < e1 ? a.recv[e] : 0;
+        sd[q] = e0 < e1 ? a.send[e] : 0;
       }
-      // (the weights stay in LDS: held in registers over the loop they would be spilled)
-      int wo = r * WMP + 8 * g;
-      asm volatile("" : "+v"(wo));
-      floatx4 acc[2][4];
-#pragma unroll
-      for (int cb = 0; cb < 4; cb++) acc[0][cb] = acc[1][cb] = floatx4{bm[cb], bm[cb], bm[cb], bm[cb]};
-#pragma unroll
-      for (int ks = 0; ks < 5; ks++) {
-        asm volatile("" ::: "memory");  // a step's weights at a time
-#pragma unroll
-        for (int cb = 0; cb < 4; cb++) {
-          const uint4 w = row8(&Wm[cb * 16 * WMP + ks * 32 + wo]);
-          acc[0][cb] = mfma(z[0][ks], w, acc[0][cb]);
-          acc[1][cb] = mfma(z[1][ks], w, acc[1][cb]);
-        }
-      }
-      // relu, rounded once
-      uint4 mv[4];
-#pragma unroll
-      for (int cb = 0; cb < 4; cb++) {
-        float v[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = fmaxf(acc[j >> 2][cb][j & 3], 0.f);
-        mv[cb] = make_uint4(cvt2(v[0], v[1]), cvt2(v[2], v[3]), cvt2(v[4], v[5]), cvt2(v[6], v[7]));
-      }
-      if (STORE) {
-        // sign words: bit 16 * cb + feature of edge 4 * (lane / 16) + q
+      for (int32_t eb = e0; eb < e1; eb += 32) {
+        uint4 z[2][5];
 #pragma unroll
         for (int q = 0; q < 2; q++) {
-          uint64_t word = 0;
-#pragma unroll
-          for (int cb = 0; cb < 4; cb++) {
-            const uint32_t w0 = q ? mv[cb].z : mv[cb].x, w1 = q ? mv[cb].w : mv[cb].y;
-            const uint64_t s0 = __ballot(on(w0)), s1 = __ballot(on(w0 >> 16)), s2 = __ballot(on(w1)),
-                           s3 = __ballot(on(w1 >> 16));
-            const uint64_t sq = (r & 2) ? ((r & 1) ? s3 : s2) : ((r & 1) ? s1 : s0);
-            word |= ((sq >> (16 * (r >> 2))) & 0xFFFFull) << (16 * cb);
+          // past the last edge: that edge again (it counts for no node below, and no load is
+          // conditional)
+          const int32_t e = min(eb + 16 * q + r, e1 - 1);
+          const int64_t er = rc[q], es = sd[q];
+          const int32_t en = min(eb + 32 + 16 * q + r, e1 - 1);  // the next ends, a chunk ahead
+          rc[q] = a.recv[en];
+          sd[q] = a.send[en];
+          z[q][4] = row8(a.ef + (int64_t)e * EP + 8 * (g & 1));
+          if (g >= 2) z[q][4] = ZERO4;  // columns 16 .. 31 are zero
+          z[q][0] = row8(a.h + er * H + 8 * g);
+          z[q][1] = row8(a.h + er * H + 32 + 8 * g);
+          z[q][2] = row8(a.h + es * H + 8 * g);
+          z[q][3] = row8(a.h + es * H + 32 + 8 * g);
+          if (LAST) {
+            // overlap inputs (column 3, in the lanes of group 0) of this half's edges, against the
+            // lane's node's range of them
+            const uint64_t pos = __ballot(bf2f((bf16)(z[q][4].y >> 16)) > 0.f) & 0xFFFFull;
+            const int lo = min(max(b0 - (eb + 16 * q), 0), 16), hi = min(max(b1 - (eb + 16 * q), 0), 16);
+            touch = touch || ((uint32_t)pos & ((1u << hi) - 1u) & ~((1u << lo) - 1u)) != 0u;
           }
-          const int32_t e = eb + 16 * q + r;
-          if (g == 0 && e < e1) a.mMask[e] = word;
         }
-      }
-      // the 0/1 operand: node r against edges eb + 16 * (j / 4) + 4 * g + j % 4
-      const int lo = min(max(b0 - eb, 0), 32), hi = min(max(b1 - eb, 0), 32);
-      const uint32_t in = (uint32_t)((1ull << hi) - 1ull) & ~(uint32_t)((1ull << lo) - 1ull);
-      const uint32_t i0 = in >> (4 * g), i1 = i0 >> 16;
-      if (pass == 0) {
-        const uint4 sw = make_uint4((i0 & 1u) * 0x3F80u | (i0 >> 1 & 1u) * 0x3F800000u,
-                                    (i0 >> 2 & 1u) * 0x3F80u | (i0 >> 3 & 1u) * 0x3F800000u,
-                                    (i1 & 1u) * 0x3F80u | (i1 >> 1 & 1u) * 0x3F800000u,
-                                    (i1 >> 2 & 1u) * 0x3F80u | (i1 >> 3 & 1u) * 0x3F800000u);
+        // (the weights stay in LDS: held in registers over the loop they would be spilled)
+        int wo = r * WMP + 8 * g;
+        asm volatile("" : "+v"(wo));
+        floatx4 acc[2][4];
 #pragma unroll
-        for (int cb = 0; cb < 4; cb++) agg[cb] = mfma(mv[cb], sw, agg[cb]);
-      } else {
-        for (int k = 0; k < 32; k++) {
-          // edge eb + k: group (k % 16) / 4, value 4 * (k / 16) + k % 4 of its lanes
-          const int kg = (k & 15) >> 2, j = 2 * (k >> 4) + ((k & 3) >> 1);
-          const bool mine = (in >> k) & 1u;
+        for (int cb = 0; cb < 4; cb++) acc[0][cb] = acc[1][cb] = floatx4{bm[cb], bm[cb], bm[cb], bm[cb]};
+#pragma unroll
+        for (int ks = 0; ks < 5; ks++) {
+          asm volatile("" ::: "memory");  // a step's weights at a time
 #pragma unroll
           for (int cb = 0; cb < 4; cb++) {
-            const uint32_t w = j == 0 ? mv[cb].x : (j == 1 ? mv[cb].y : (j == 2 ? mv[cb].z : mv[cb].w));
+            const uint4 w = row8(&Wm[cb * 16 * WMP + ks * 32 + wo]);
+            acc[0][cb] = mfma(z[0][ks], w, acc[0][cb]);
+            acc[1][cb] = mfma(z[1][ks], w, acc[1][cb]);
+          }
+        }
+        // relu, rounded once
+        uint4 mv[4];
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-              const uint32_t o = __shfl(w, 16 * kg + 4 * g + q);
-              const float v = bf2f((bf16)((k & 1) ? o >> 16 : o & 0xFFFFu));
-              agg[cb][q] += mine ? v : 0.f;
+        for (int cb = 0; cb < 4; cb++) {
+          float v[8];
+#pragma unroll
+          for (int j = 0; j < 8; j++) v[j] = fmaxf(acc[j >> 2][cb][j & 3], 0.f);
+          mv[cb] = make_uint4(cvt2(v[0], v[1]), cvt2(v[2], v[3]), cvt2(v[4], v[5]), cvt2(v[6], v[7]));
+        }
+        if (STORE) {
+          // sign words: bit 16 * cb + feature of edge 4 * (lane / 16) + q
+#pragma unroll
+          for (int q = 0; q < 2; q++) {
+            uint64_t word = 0;
+#pragma unroll
+            for (int cb = 0; cb < 4; cb++) {
+              const uint32_t w0 = q ? mv[cb].z : mv[cb].x, w1 = q ? mv[cb].w : mv[cb].y;
+              const uint64_t s0 = __ballot(on(w0)), s1 = __ballot(on(w0 >> 16)), s2 = __ballot(on(w1)),
+                             s3 = __ballot(on(w1 >> 16));
+              const uint64_t sq = (r & 2) ? ((r & 1) ? s3 : s2) : ((r & 1) ? s1 : s0);
+              word |= ((sq >> (16 * (r >> 2))) & 0xFFFFull) << (16 * cb);
+            }
+            const int32_t e = eb + 16 * q + r;
+            if (g == 0 && e < e1) a.mMask[e] = word;
+          }
+        }
+        // the 0/1 operand: node r against edges eb + 16 * (j / 4) + 4 * g + j % 4
+        const int lo = min(max(b0 - eb, 0), 32), hi = min(max(b1 - eb, 0), 32);
+        const uint32_t in = (uint32_t)((1ull << hi) - 1ull) & ~(uint32_t)((1ull << lo) - 1ull);
+        const uint32_t i0 = in >> (4 * g), i1 = i0 >> 16;
+        if (pass == 0) {
+          const uint4 sw = make_uint4((i0 & 1u) * 0x3F80u | (i0 >> 1 & 1u) * 0x3F800000u,
+                                      (i0 >> 2 & 1u) * 0x3F80u | (i0 >> 3 & 1u) * 0x3F800000u,
+                                      (i1 & 1u) * 0x3F80u | (i1 >> 1 & 1u) * 0x3F800000u,
+                                      (i1 >> 2 & 1u) * 0x3F80u | (i1 >> 3 & 1u) * 0x3F800000u);
+#pragma unroll
+          for (int cb = 0; cb < 4; cb++) agg[cb] = mfma(mv[cb], sw, agg[cb]);
+        } else {
+          for (int k = 0; k < 32; k++) {
+            // edge eb + k: group (k % 16) / 4, value 4 * (k / 16) + k % 4 of its lanes
+            const int kg = (k & 15) >> 2, j = 2 * (k >> 4) + ((k & 3) >> 1);
+            const bool mine = (in >> k) & 1u;
+#pragma unroll
+            for (int cb = 0; cb < 4; cb++) {
+              const uint32_t w = j == 0 ? mv[cb].x : (j == 1 ? mv[cb].y : (j == 2 ? mv[cb].z : mv[cb].w));
+#pragma unroll
+              for (int q = 0; q < 4; q++) {
+                const uint32_t o = __shfl(w, 16 * kg + 4 * g + q);
+                const float v = bf2f((bf16)((k & 1) ? o >> 16 : o & 0xFFFFu));
+                agg[cb][q] += mine ? v : 0.f;
+              }
             }
           }
         }
       }
-    }
-    bool fin = true;
+      bool fin = true;
 #pragma unroll
-    for (int cb = 0; cb < 4; cb++)
+      for (int cb = 0; cb < 4; cb++)
 #pragma unroll
-      for (int q = 0; q < 4; q++) fin = fin && fabsf(agg[cb][q]) <= 3.402823466e38f;
-    if (__all(fin)) break;
+        for (int q = 0; q < 4; q++) fin = fin && fabsf(agg[cb][q]) <= 3.402823466e38f;
+      if (__all(fin)) break;
     }
     // agg: features 16 * cb + 4 * g + q of node r, rounded once
     uint2 ag[4];
