@@ -348,3 +348,54 @@ def test_network_keeps_an_overflow_to_its_neighbours():
     far = np.abs(np.arange(N) - 5) > 2
     np.testing.assert_array_equal(a[far], b[far])
     assert not np.all(np.isfinite(b[~far])) or np.any(np.abs(b[~far]) > 1e30)
+
+
+# needle triangles whose vertices are collinear up to rounding: near them the signs of the three edge
+# tests are rounding noise, and about a fifth of the positions lie outside all three edges
+NEEDLES = {64: ((-0.11411671584340066, -0.08510797192370884, -0.015578443378596867),
+                (-0.04603145941331931, -0.03433015160313763, -0.00628390397326742)),
+           32: ((-0.09294396638870239, 0.07020442187786102, -0.024254076182842255),
+                (-0.06973002105951309, 0.05266996845602989, -0.018196310847997665))}
+
+
+def needle_scene(bits, n=8000, far=3.5e-3):
+    # a bed of several groups of slots, and spheres that come within reach of a needle after some steps
+    from tests.scenes import deposition
+
+    sc = deposition(n=n, seed=3, r=2e-3, dense=True, vel_sigma=.05)
+    r = sc["radius"][0]
+    v = np.array([(0., 0., 0.), *NEEDLES[bits]])
+    # the normal as this precision computes it: rounding noise, so not at right angles to the edges
+    nn = np.cross(*v[1:].astype(np.float64 if bits == 64 else np.float32)).astype(np.float64)
+    nn /= np.linalg.norm(nn)
+    t = np.arange(.1, .95, 2.2 * r / np.linalg.norm(v[1]))
+    k = len(t)
+    sc["pos"] = np.vstack([sc["pos"], t[:, None] * v[1] + ((1 + far) * r - t * (v[1] @ nn))[:, None] * nn])
+    sc["vel"] = np.vstack([sc["vel"], np.repeat(-1e-3 * r / sc["dt"] * nn[None], k, 0)])
+    for q in ("radius", "mass", "inertia"):
+        sc[q] = np.concatenate([sc[q], np.repeat(sc[q][:1], k, 0)])
+    sc.update(facets=[dict(verts=v)], walls=[], gravity=(0., 0., 0.))
+    return sc
+
+
+@pytest.mark.parametrize("bits", [64, 32])
+@pytest.mark.parametrize("graph", [False, True])
+def test_an_error_ends_a_batch_after_its_step(bits, graph):
+    # the filter itself raises an error (a sphere outside all edges of a needle facet): its step runs to
+    # the end on every workgroup, the next one on none, as when the engines are called one by one
+    from tests.scenes import GpuRunner, contact_kw
+
+    sc = needle_scene(bits)
+    a, b = GpuRunner(sc), GpuRunner(sc)
+    for d in (a.d, b.d):
+        d.set_precision(bits)
+    with pytest.raises(Exception, match="impossible sphere-facet"):
+        a.run(["Collider", "ContactLoop", "Leapfrog"], 32)
+    assert 2 < a.step < 16
+    with pytest.raises(Exception, match="impossible sphere-facet"):
+        b.d.run(["Collider", "ContactLoop", "Leapfrog"], 32, 0, sc["dt"], contact=contact_kw(sc),
+                leapfrog=dict(damping=sc["damping"]), dynDtPeriod=0, graph=graph)
+    assert a.d.stats()["nCandidates"] > 10 * 2048
+    for f in ("pos", "vel", "angVel", "ori", "force", "torque"):
+        np.testing.assert_array_equal(a.d.get(f), b.d.get(f), err_msg=f)
+    np.testing.assert_array_equal(a.d.contacts(data=False)[0], b.d.contacts(data=False)[0])

@@ -314,13 +314,15 @@ __device__ __forceinline__ bool filter_slot(const ContactArgs& a, int64_t c, Slo
 
 // Whether a gated step is skipped, decided by its first kernel: once a step was skipped, or when
 // the step before it (not the host's collider call, before the batch's first step) left a particle
-// outside its Verlet skin or raised an error. Every workgroup comes to the same answer from words
-// that no other of them writes differently; the first one makes it stick for the kernels and steps
-// after it and sets the step's trsfRenorm flag. The leapfrog counts the step when it ran.
+// outside its Verlet skin or raised an error. Every wavefront must come to the same answer, so none
+// of the words may be one that this kernel writes otherwise: the errors are those that the leapfrog
+// of the step before found (gs[7]), not the live word, to which the filter itself adds. The first
+// workgroup makes the answer stick for the kernels and steps after it and sets the step's trsfRenorm
+// flag. The leapfrog counts the step when it ran.
 __device__ __forceinline__ bool step_skipped(const ContactArgs& a) {
   if (!a.gs) return false;
   // (all the words at once, not one after the other)
-  const uint32_t stop = a.gs[0], first = a.gs[6], dirty = *a.dirtyPrev, err = a.dflags[1];
+  const uint32_t stop = a.gs[0], first = a.gs[6], dirty = *a.dirtyPrev, err = a.gs[7];
   const bool skip = (stop != 0u) | ((first == 0u) & ((dirty | err) != 0u));
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (skip) {

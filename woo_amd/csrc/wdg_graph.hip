@@ -31,7 +31,8 @@
 namespace wdg {
 
 // gstate words: [0] stop, [1] steps executed in the batch, [2] renorm flag of the step, [3..4]
-// the batch's first step (int64), [5] trsfRenorm, [6] set until the batch's first step starts.
+// the batch's first step (int64), [5] trsfRenorm, [6] set until the batch's first step starts, [7] the
+// error bits after the last step executed.
 // A batch is several replays launched back to back: once a gate has stopped, every later kernel
 // of the batch returns at once, so the replays after the stop cost only their launches.
 // The gate of a step without slots, which has no filter (step_skipped in wdg_contact.hip and the
@@ -185,8 +186,8 @@ static int batch(Ctx& c, const wdg_program* prog, int K, int n, int64_t step, do
   } else {
     size_buffers(c, prog);
   }
-  uint32_t w[7] = {0u, 0u, 0u, (uint32_t)((uint64_t)step & 0xFFFFFFFFu), (uint32_t)((uint64_t)step >> 32),
-                   (uint32_t)std::max(prog->contact.trsfRenorm, 0), 1u};
+  uint32_t w[8] = {0u, 0u, 0u, (uint32_t)((uint64_t)step & 0xFFFFFFFFu), (uint32_t)((uint64_t)step >> 32),
+                   (uint32_t)std::max(prog->contact.trsfRenorm, 0), 1u, 0u};
   WDG_HIP(hipMemcpyAsync(c.gstate.p, w, sizeof(w), hipMemcpyHostToDevice, c.stream));
   if (K > 0) {
     for (int r = 0; r < n / K; r++) WDG_HIP(hipGraphLaunch(c.graph.exec, c.stream));

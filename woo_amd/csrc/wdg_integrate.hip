@@ -413,6 +413,7 @@ __global__ __launch_bounds__(256) void k_leapfrog(LeapArgs a, GatherArgs g) {
     if (a.gs) {
       a.gs[1] += 1u;
       a.gs[6] = 0u;
+      a.gs[7] = *a.err;  // (nothing raises an error between the contact loop and the next filter)
     }
     if (a.host) a.host[HOST_ERR] = *a.err;
   }
@@ -660,10 +661,10 @@ void leapfrog(Ctx& c, const wdg_leapfrog_params* p) {
   }
   // a gated step is counted here when its filter ran (without slots k_gate counts it)
   if (c.gated && c.con().n > 0) a.gs = c.gstate.p;
+  a.err = c.dflags.p + 1;
   if (!c.gated) {
     a.host = c.hflagsDev;
     a.number = ++c.lfNumber;
-    a.err = c.dflags.p + 1;
   }
   if (track && energy_per_scene(c)) {
     energy_scenes_prepare(c, c.con().n);
