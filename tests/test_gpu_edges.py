@@ -399,3 +399,23 @@ def test_an_error_ends_a_batch_after_its_step(bits, graph):
     for f in ("pos", "vel", "angVel", "ori", "force", "torque"):
         np.testing.assert_array_equal(a.d.get(f), b.d.get(f), err_msg=f)
     np.testing.assert_array_equal(a.d.contacts(data=False)[0], b.d.contacts(data=False)[0])
+
+
+@pytest.mark.parametrize("how", ["collide", "sync", "run"])
+def test_an_error_is_reported_once(how):
+    # whichever call reports a step's error, the collider's next call goes on
+    from tests.scenes import GpuRunner, contact_kw
+
+    sc = needle_scene(64)
+    g = GpuRunner(sc)
+    eng = ["Collider", "ContactLoop", "Leapfrog"]
+    if how == "run":
+        report = lambda: g.d.run(eng, 32, 0, sc["dt"], contact=contact_kw(sc), leapfrog=dict(damping=sc["damping"]),
+                                 dynDtPeriod=0)
+    else:
+        g.run(eng, 5)
+        report = (lambda: g.d.collide(g.vd)) if how == "collide" else g.d.sync
+    with pytest.raises(Exception, match="impossible sphere-facet"):
+        report()
+    g.d.collide(g.vd)
+    g.d.sync()

@@ -1502,13 +1502,16 @@ static void check_device_errors(Ctx& c, uint32_t err) {
     throw Error(WDG_E_GEOM, "snapshot: a saved contact's periodic image differs from the refreshed pair's");
 }
 
-void check_errors(Ctx& c) {
-  uint32_t err = read_u32(c, c.dflags.p + 1);
-  if (err) {
-    WDG_HIP(hipMemsetAsync(c.dflags.p + 1, 0, sizeof(uint32_t), c.stream));
-    check_device_errors(c, err);
-  }
+// error bits that the host has read (nothing is queued on the stream): cleared, in the leapfrog's pinned
+// copy too, so that each is reported once, and raised
+static void take_errors(Ctx& c, uint32_t err) {
+  if (!err) return;
+  WDG_HIP(hipMemsetAsync(c.dflags.p + 1, 0, sizeof(uint32_t), c.stream));
+  c.hflags[HOST_ERR] = 0u;
+  check_device_errors(c, err);
 }
+
+void check_errors(Ctx& c) { take_errors(c, read_u32(c, c.dflags.p + 1)); }
 
 void drop_contacts(Ctx& c) {
   for (auto& s : c.C) {
@@ -2102,13 +2105,9 @@ static void refresh(Ctx& c) {
   c.cur = 1 - c.cur;
   c.rcur = rNew;
   c.boundsValid = true;
-  const uint32_t err = hw[RW_ERR];
   c.dirtyKnown = true;
   c.dirtyIdx = 0;
-  if (err) {
-    WDG_HIP(hipMemsetAsync(c.dflags.p + 1, 0, sizeof(uint32_t), c.stream));
-    check_device_errors(c, err);
-  }
+  take_errors(c, hw[RW_ERR]);
 }
 
 void collide(Ctx& c, const wdg_collide_params* p) {
@@ -2148,11 +2147,7 @@ void collide(Ctx& c, const wdg_collide_params* p) {
                              c.stream));
       WDG_HIP(hipStreamSynchronize(c.stream));
     }
-    if (c.hflags[1]) {
-      uint32_t err = c.hflags[1];
-      WDG_HIP(hipMemsetAsync(c.dflags.p + 1, 0, sizeof(uint32_t), c.stream));
-      check_device_errors(c, err);
-    }
+    take_errors(c, c.hflags[1]);
     if (c.hflags[c.dirtyIdx]) full = true;
   }
   if (full) {
