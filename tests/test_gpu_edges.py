@@ -419,3 +419,25 @@ def test_an_error_is_reported_once(how):
         report()
     g.d.collide(g.vd)
     g.d.sync()
+
+
+@pytest.mark.parametrize("n,periodic", [(20, False), (300, False), (1500, True)])
+def test_steps_in_calls_of_any_length(n, periodic):
+    # calls of a few steps (launched one after the other) and of more (launched ahead) mixed: the same
+    # steps, refreshes and states as one call for all
+    from tests.scenes import build_gpu, contact_kw, deposition, periodic_hertz
+
+    sc = periodic_hertz(n=n, spacing=.95, vel_sigma=2.) if periodic else deposition(n=n, seed=n, dense=True, vel_sigma=.3)
+    kw = dict(contact=contact_kw(sc), leapfrog=dict(damping=sc["damping"]), dynDtPeriod=0)
+    eng = ["Collider", "ContactLoop", "Leapfrog"]
+    a, b = build_gpu(sc), build_gpu(sc)
+    calls = [1, 1, 2, 3, 4, 5, 6, 1, 9, 4, 17, 1, 2]
+    a.run(eng, sum(calls), 0, sc["dt"], **kw)
+    st = 0
+    for k in calls:
+        st, _ = b.run(eng, k, st, sc["dt"], **kw)
+    assert st == sum(calls)
+    for f in ("pos", "vel", "angVel", "ori", "force", "torque"):
+        np.testing.assert_array_equal(a.get(f), b.get(f), err_msg=f)
+    sa, sb = a.stats(), b.stats()
+    assert sa["nSteps"] == sb["nSteps"] and sa["nRefresh"] == sb["nRefresh"] > 1

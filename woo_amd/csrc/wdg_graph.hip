@@ -232,6 +232,8 @@ static int batch(Ctx& c, const wdg_program* prog, int K, int n, int64_t step, do
   return e;
 }
 
+// fewer steps than these are not launched ahead
+constexpr int AHEAD_MIN = 5;
 // K > 0: replays of a K-step graph; 0: steps launched ahead
 static void run_gated(Ctx& c, const wdg_program* prog, int K, int64_t nSteps, int64_t* step, double* dt) {
   c.gstate.ensure(16);
@@ -251,7 +253,12 @@ static void run_gated(Ctx& c, const wdg_program* prog, int K, int64_t nSteps, in
     // (a periodic scene's step 0 is a plain one when tracking energy: its leapfrog adds no terms,
     // and a graph captured there would skip them at every replay)
     // (updatePhys 'once' is one plain step, after which the loop reads 'never')
-    if (!c.forceClean || c.forcesPending || left < std::max(K, 1) || c.n == 0 || c.updatePhys == 2 ||
+    // (the last few steps of a call without a graph are plain ones: their leapfrogs leave the dirty and
+    // error words for the collider, and the call returns without a wait, where a batch copies words both
+    // ways and waits once more. A call of one step took 57 / 72 / 86 us as a batch and takes 33 / 45 / 61 at
+    // 20 / 20,000 / 250,000 spheres; a step of calls of two 44 / 55 / 70 against the same, of four 34 / 46,
+    // of eight 32 / 42 / 58)
+    if (!c.forceClean || c.forcesPending || left < (K > 0 ? K : AHEAD_MIN) || c.n == 0 || c.updatePhys == 2 ||
         !(c.verletDist > 0) || (c.trackEnergy && c.field.periodic && *step == 0)) {
       if (c.trackEnergy && K == 0) energy_step_begin(c);
       plain_step(c, prog, *step, *dt);
