@@ -1331,7 +1331,7 @@ __global__ void k_big_scatter(int64_t m, const uint32_t* __restrict__ val, const
 // Entries are ranked by the other particle's user id (ids within a list are distinct).
 struct AdjArgs {
   int64_t nSph, nW;
-  const uint32_t *nb, *deg, *count, *off, *B, *uid, *adjOff;
+  const uint32_t *nb, *deg, *count, *off, *A, *B, *uid, *adjOff;
   uint64_t* ent;
   uint32_t* adj;
   uint32_t* dflags;
@@ -1349,25 +1349,21 @@ __device__ __forceinline__ bool adj_generated(const AdjArgs& a, uint32_t p, uint
 __device__ __forceinline__ bool adj_is_pa(const AdjArgs& a, uint32_t up, uint32_t j, uint32_t uj) {
   return j >= (uint32_t)a.nW && up < uj;
 }
-// The entry of neighbour j of sphere p (storage): the slot of the pair (the next one p
-// generated, or found among the pairs j generated), keyed by j's user id for the ranking.
-__device__ __forceinline__ uint64_t adj_entry(const AdjArgs& a, uint32_t p, uint32_t up, uint32_t j, uint32_t& gen) {
-  uint32_t slot;
-  if (adj_generated(a, p, j)) {
-    slot = gen++;
-  } else {
-    slot = 0xFFFFFFFFu;
-    const uint32_t g0 = a.off[j - a.nW], g1 = g0 + a.count[j - a.nW];
-    for (uint32_t u = g0; u < g1; u++)
-      if (a.B[u] == p) { slot = u; break; }
-    if (slot == 0xFFFFFFFFu) {
-      // the pair test disagreed between the two spheres: reported, entry kept in bounds
-      atomicOr(&a.dflags[1], ERR_ADJ);
-      slot = 0u;
-    }
-  }
-  const uint32_t uj = a.uid[j];
-  return ((uint64_t)uj << 32) | slot | (adj_is_pa(a, up, j, uj) ? ADJ_PA : 0u);
+// The entry of neighbour j of sphere p (storage): the slot of the pair (p's r-th generated one, or found
+// among the pairs j generated), keyed by j's user id for the ranking. The slots lie in the order in which
+// p staged its pairs, and so its neighbours, as long as one pass made both: a slot with another partner,
+// like a pair found from one side only, is an error (bad), the entry kept in bounds. (The partner is
+// compared last, so that its load is waited for together with the ids'.)
+__device__ __forceinline__ uint64_t adj_entry(const AdjArgs& a, uint32_t p, uint32_t j, uint32_t r, bool& bad) {
+  const bool own = adj_generated(a, p, j);
+  uint32_t slot = own ? a.off[p - a.nW] + r : find_partner(a.B, a.off[j - a.nW], a.count[j - a.nW], p);
+  const bool in = slot < a.want / 2u;
+  if (!in) slot = 0u;
+  const uint32_t partner = own ? (j < (uint32_t)a.nW ? a.A : a.B)[slot] : j;
+  const uint32_t uj = a.uid[j], up = a.uid[p];
+  const uint64_t e = ((uint64_t)uj << 32) | slot | (adj_is_pa(a, up, j, uj) ? ADJ_PA : 0u);
+  bad = bad || !in || partner != j;
+  return e;
 }
 
 // Each sphere's adjacency ranked by the neighbour's user id. The 64 spheres of a wavefront own
@@ -1406,6 +1402,7 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) void k_adj_sym(AdjArgs a) {
   };
   // the wavefront's spheres in runs whose entries fit the LDS arrays; a sphere with more
   // entries than fit takes its list alone in one thread, through HBM (a.ent)
+  bool bad = false;
   int L0 = 0;
   while (L0 < 64) {
     int L1 = L0 + 1;
@@ -1413,9 +1410,13 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) void k_adj_sym(AdjArgs a) {
     const uint32_t E0 = so[w][L0], E1 = so[w][L1];
     if (E1 - E0 > (uint32_t)ADJ_CAP) {
       if (lane == L0) {
-        const uint32_t p = (uint32_t)(a.nW + t), up = a.uid[p];
-        uint32_t gen = a.off[t];
-        for (uint32_t q = 0; q < m; q++) a.ent[k0 + q] = adj_entry(a, p, up, a.nb[(int64_t)q * a.nSph + t], gen);
+        const uint32_t p = (uint32_t)(a.nW + t);
+        uint32_t gen = 0;
+        for (uint32_t q = 0; q < m; q++) {
+          const uint32_t j = a.nb[(int64_t)q * a.nSph + t];
+          a.ent[k0 + q] = adj_entry(a, p, j, gen, bad);
+          gen += adj_generated(a, p, j) ? 1u : 0u;
+        }
         for (uint32_t q = 0; q < m; q++) {
           const uint64_t e = a.ent[k0 + q];
           uint32_t r = 0;
@@ -1440,22 +1441,10 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) void k_adj_sym(AdjArgs a) {
       uint32_t q;
       owner(e, L, q);
       const uint32_t p = (uint32_t)(a.nW + tw + L), j = sj[w][e - E0], b0 = so[w][L] - E0;
-      uint32_t slot;
-      if (adj_generated(a, p, j)) {
-        // p generated its pairs in the order of its neighbours above it, then its bodies
-        uint32_t r = 0;
+      uint32_t r = 0;
+      if (adj_generated(a, p, j))
         for (uint32_t v = 0; v < q; v++) r += adj_generated(a, p, sj[w][b0 + v]) ? 1u : 0u;
-        slot = a.off[tw + L] + r;
-      } else {
-        slot = find_partner(a.B, a.off[j - a.nW], a.count[j - a.nW], p);
-        if (slot == 0xFFFFFFFFu) {
-          // the pair test disagreed between the two spheres: reported, entry kept in bounds
-          atomicOr(&a.dflags[1], ERR_ADJ);
-          slot = 0u;
-        }
-      }
-      const uint32_t uj = a.uid[j], up = a.uid[p];
-      se[w][e - E0] = ((uint64_t)uj << 32) | slot | (adj_is_pa(a, up, j, uj) ? ADJ_PA : 0u);
+      se[w][e - E0] = adj_entry(a, p, j, r, bad);
     }
     wave_lds_sync();
     // rank among the sphere's keys (distinct: one entry per neighbour)
@@ -1473,6 +1462,7 @@ __global__ __launch_bounds__(64 * ADJ_WAVES) void k_adj_sym(AdjArgs a) {
     wave_lds_sync();
     L0 = L1;
   }
+  if (__any(bad) && lane == 0) atomicOr(&a.dflags[1], ERR_ADJ);
 }
 
 // the inverse of the adjacency: per slot the positions of its pA entry and its pB entry; every
@@ -1955,7 +1945,8 @@ static void refresh(Ctx& c) {
     overflow = c.hflags[7] > (uint32_t)PS;
     if (overflow) c.pairStage = (int)std::min<uint32_t>(96u, (c.hflags[7] + 7u) / 8u * 8u);
     // (pairs generated again in place: the passes that stage and that do not work off their queues in
-    // different rounds, so the staged neighbours do not tell the slots' order then)
+    // different rounds, so the staged neighbours do not tell the slots' order then, and k_adj_sym, which
+    // takes a sphere's slots in that order, would give entries of other pairs)
     nbFits = !overflow && c.hflags[8] <= (uint32_t)NS;
     // a sphere with more neighbours than staged sends the adjacency to the general path; the
     // next refreshes stage more (up to 128)
@@ -2050,7 +2041,7 @@ static void refresh(Ctx& c) {
         c.adjEnt.ensure(2 * nNew);
         AdjArgs aa{};
         aa.nSph = nSph; aa.nW = nW; aa.nb = c.stNb.p; aa.deg = c.sdeg.p; aa.count = c.scount.p; aa.off = c.soff.p;
-        aa.B = N.B.p; aa.uid = c.uid.p; aa.adjOff = N.adjOff.p; aa.ent = c.adjEnt.p; aa.adj = N.adj.p;
+        aa.A = N.A.p; aa.B = N.B.p; aa.uid = c.uid.p; aa.adjOff = N.adjOff.p; aa.ent = c.adjEnt.p; aa.adj = N.adj.p;
         aa.dflags = c.dflags.p;
         aa.want = (uint32_t)(2 * nNew);
         hipLaunchKernelGGL(k_adj_sym, dim3(nblocks(nSph, 64 * ADJ_WAVES)), dim3(64 * ADJ_WAVES), 0, c.stream, aa);
@@ -2086,9 +2077,11 @@ static void refresh(Ctx& c) {
       nExtra = hw[RW_EXTRA];
       continue;
     }
-    if (hw[RW_ENTRIES] != 2 * (uint64_t)nNew)
+    if (hw[RW_ENTRIES] != 2 * (uint64_t)nNew) {
+      drop_contacts(c);  // (the particles have moved in storage: the old list is of no use either)
       throw Error(WDG_E_STATE, "broadphase: neighbour lists disagree with the pair list (" +
                                    std::to_string(hw[RW_ENTRIES]) + " entries for " + std::to_string(nNew) + " pairs)");
+    }
     if (staged && hw[RW_LONGEST] > WS_CAP) {
       // bodies with longer lists than a workgroup sorts: all by the radix sort
       sort_lists(c, N, nW, 0);
@@ -2107,6 +2100,9 @@ static void refresh(Ctx& c) {
   c.boundsValid = true;
   c.dirtyKnown = true;
   c.dirtyIdx = 0;
+  // entries with wrong slots leave places of the slots' entries (entPos) unwritten, through which a
+  // filter would store: nothing steps over such a list
+  if (hw[RW_ERR] & ERR_ADJ) drop_contacts(c);
   take_errors(c, hw[RW_ERR]);
 }
 
