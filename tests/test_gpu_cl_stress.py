@@ -45,3 +45,33 @@ def test_contact_loop_stress_is_zero_in_aperiodic_scenes():
     assert d.stats()["nReal"] > 0
     assert not d.contact_loop_stress().any()
     d.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_contact_loop_stress_while_the_slot_list_grows(graph):
+    # spread spheres (one group of slots), then moved into a dense block (more groups than the partial
+    # sums held): the gated steps allocate nothing, and the stress is that of the engines called one by one
+    from tests.scenes import GpuRunner
+
+    sc = periodic_hertz(n=6000, rmin=3.9e-3, spacing=1.2, seed=36, vel_sigma=.1)
+    sc["pos"][1] = sc["pos"][0] + (7.7e-3, 0., 0.)  # one contact
+    m = int(np.ceil(6000 ** (1 / 3.)))
+    dense = (np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[:6000] + .5) * 7.75e-3
+    a, d = GpuRunner(sc), build_gpu(sc)
+    kw = dict(contact=contact_kw(sc), leapfrog=dict(damping=sc["damping"]), dynDtPeriod=0, graph=graph)
+    step = 0
+    for dev in (a.d, d):
+        dev.set_eval_stress(True)
+    for k in range(2):
+        a.run(ENG, 24)
+        step, _ = d.run(ENG, 24, step, sc["dt"], **kw)
+        s = d.contact_loop_stress()
+        assert s.any()
+        np.testing.assert_array_equal(s, a.d.contact_loop_stress())
+        np.testing.assert_array_equal(d.get("pos"), a.d.get("pos"))
+        if k == 0:
+            assert 0 < d.stats()["nCandidates"] <= 2048
+            for dev in (a.d, d):
+                dev.set("pos", dense)
+    assert d.stats()["nCandidates"] > 7 * 2048
+    d.close()

@@ -115,6 +115,10 @@ static void size_buffers(Ctx& c, const wdg_program* prog) {
   if (c.trackEnergy)
     c.enPart.ensure(std::max<size_t>((size_t)4 * ngroups(nc) * c.tune.cfBlocks, (size_t)3 * nblocks(c.n, 256)));
   if (energy_per_scene(c)) energy_scenes_prepare(c, nc);
+  if (c.evalStress && c.field.periodic) {
+    c.clPart.ensure((size_t)9 * ngroups(nc));
+    c.clStress.ensure(9);
+  }
 }
 
 static void capture(Ctx& c, const wdg_program* prog, int K, int64_t step, double dt) {
