@@ -76,3 +76,30 @@ def test_check_state_is_dem_redo_of_last_coarse_step():
         np.testing.assert_array_equal(d1.get(f), d0.get(f), err_msg=f)
     # the learned state differs from plain DEM (so the checks compared something)
     assert max(st["errors"]) > 0.
+
+
+def test_a_forward_pass_waits_for_the_step_before():
+    # a learned step queued behind other work of the engine moves the spheres by its own forward pass,
+    # also when the network passes another graph before the step has run
+    from woo_amd.surrogate import COARSE
+
+    out = []
+    for wait in (False, True):
+        d, net, arr, rad, dt, step = _setup()
+        net.graph_from(d, force=True)
+        net.keep(0)
+        d.set("vel", 3. * d.get("vel"))
+        net.graph_from(d)
+        a = net.forward()
+        for k in range(40):  # some milliseconds of the engine's stream, none of which waits
+            d.kinetic_energy() if wait else None
+            d.contact_loop(step + k, 1e-12, physKind=1, lawKind=1, poisson=.25, en=.6)
+        net.advance(d, COARSE * dt)
+        if wait:
+            d.sync()
+        net.use(0)
+        b = net.forward()
+        out.append((d.get("pos"), d.get("vel")))
+    assert np.max(np.abs(a - b)) > 1e-3 * np.max(np.abs(a))
+    for x, y in zip(*out):
+        np.testing.assert_array_equal(x, y)

@@ -1734,6 +1734,9 @@ int wdg_mpnn_advance(wdg_mpnn* m, wdg_ctx* ctx, double dT) {
                          c.field.gravity[1], c.field.gravity[2], c.pos[0].p, c.pos[1].p, c.pos[2].p, c.vel[0].p, c.vel[1].p,
                          c.vel[2].p, (const uint32_t*)c.flags.p);
       WDG_LAUNCH_CHECK();
+      // the next forward pass, of whichever graph, writes the outputs that this step reads
+      WDG_HIP(hipEventRecord(s.done, c.stream));
+      WDG_HIP(hipStreamWaitEvent(s.stream, s.done, 0));
     }
     c.dirtyKnown = false;
   });
