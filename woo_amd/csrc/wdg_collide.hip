@@ -920,11 +920,13 @@ __global__ __launch_bounds__(256) void k_pairs(PairArgs a) {
   }
 }
 
-// Lanes per sphere: as many as fill the chip's 1,024 SIMDs with a few wavefronts. Measured (us):
-// all pairs of 300 spheres 73 / 46 / 34 / 24 with 1 / 2 / 4 / 8 lanes, 2,000 in cells 46 / 30 / 19 /
-// 15, 20,000: 56 / 35 / 23 / 18, 150,000: 94 / 92 / 85 / 92, 186,000 sparse in 64 scenes 36 / 46 /
-// 59 / 80, 1M: 309 / 328 / 377 / 481 (the passes over queues and cells that more lanes repeat then
-// cost more than the latency they hide).
+// Lanes per sphere: as many as fill the chip's 1,024 SIMDs with a few wavefronts. Measured (us, with 1 / 2
+// / 4 / 8 lanes): all pairs of 300 spheres 73 / 46 / 34 / 24, 2,000 in cells 46 / 30 / 19 / 15, 20,000: 56 /
+// 35 / 23 / 18, 150,000 dense: 94 / 92 / 85 / 92, 186,000 sparse in 64 scenes 36 / 46 / 59 / 80, 1M: 309 /
+// 328 / 377 / 481 (the passes over queues and cells that more lanes repeat then cost more than the
+// latency they hide, the more so the fewer candidates a sphere has). The density is not known before the
+// pass, so one lane from 100,000 on: that gives up a tenth in a dense scene and four lanes would cost a
+// sparse one two thirds.
 static int pair_lanes(int64_t nSph) { return nSph <= 40000 ? 8 : (nSph <= 100000 ? 4 : 1); }
 template <int OUT, int MODE, int G>
 static void launch_pairs_g(Ctx& c, const PairArgs& a) {

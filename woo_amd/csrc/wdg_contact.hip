@@ -423,13 +423,16 @@ __device__ __forceinline__ void en_clear(const ContactArgs& a, int64_t k) {
   e2[1] = make_double2(0., 0.);
 }
 
-// The state arrays are read and written once per step, at consecutive addresses. Where the sets of
-// before and after the step do not fit the 256 MB last-level cache, they go past it, which so keeps
-// what is read again (particles, the filter's records, gather records): a step of 1M spheres (1.4M
-// contacts) is 3.4% faster; below that the next step finds its state there: past the cache, steps
-// of 20,000 and of 200,000 spheres were 2% slower. The FP32 form's sets are half as large and keep to
-// ordinary accesses (250,000 spheres: 7% slower past the cache).
-constexpr int64_t STREAM_SLOTS = (256ll << 20) / (2 * 10 * 8);
+// The state arrays are read and written once per step, at consecutive addresses. Where the step's whole
+// working set (slots, records, particles, state) is beyond the 256 MB last-level cache they go past it,
+// which so keeps more of what is read again; below, the next step finds the state there. The line is
+// therefore one on slots, which the working set follows, and not on the real contacts that have state.
+// Us a step, through the cache / past it, graph replay without refreshes: 0.67M slots (0.27M real
+// contacts) 69.5 / 74.5, 1.01M (0.14M) 115 / 114, 1.33M (0.52M) 139 / 131, 1.51M (0.26M) 116 / 113, 2.35M
+// (0.41M) 184 / 179, 2.68M (1.06M) 276 / 266, a drum's 2.35M (0.97M) 253 / 243. The FP32 form's sets are
+// half as large and keep to ordinary accesses (250,000 spheres: 7% slower past the cache); so do the
+// variants that track energy, which were not measured.
+constexpr int64_t STREAM_SLOTS = 1 << 20;
 template <bool STREAM, class T>
 __device__ __forceinline__ T state_load(const T* p) {
   return STREAM ? __builtin_nontemporal_load(p) : *p;
