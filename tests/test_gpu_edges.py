@@ -275,6 +275,68 @@ def test_steps_ahead_equal_engine_calls(n, flat, steps, track):
     assert sa["nSteps"] == sb["nSteps"] and sa["nRefresh"] == sb["nRefresh"]
     if flat:
         assert sa["nCandidates"] > 2 * 2048
+    if track:  # every term, by the same sums of the same steps; skipped steps add nothing
+        ea, eb = a.d.energy(), b.d.energy()
+        assert ea == eb and ea["kinetic"] > 0 and (steps == 1 or ea["plast"] > 0)
+
+
+@pytest.mark.parametrize("track", [False, True])
+def test_steps_ahead_with_facet_nodes(track):
+    # the list with IntraForce: the forces on the facets' nodes are those of the last step that ran
+    from tests.scenes import GpuRunner, contact_kw, drum
+
+    sc = drum(n=1500, vel_sigma=.3)
+    a, b = GpuRunner(sc), GpuRunner(sc)
+    eng = ["Collider", "ContactLoop", "IntraForce", "Leapfrog"]
+    ids = np.arange(len(sc["walls"]), len(sc["walls"]) + len(sc["facets"]))
+    for g in (a, b):
+        g.d.set_energy_tracking(track)
+    st = 0
+    for steps in (1, 7, 60):
+        a.run(eng, steps)
+        st, _ = b.d.run(eng, steps, st, sc["dt"], contact=contact_kw(sc), leapfrog=dict(damping=sc["damping"]),
+                        dynDtPeriod=0)
+        na, nb = np.array(a.d.facet_nodes(ids)), np.array(b.d.facet_nodes(ids))
+        assert np.any(na)
+        np.testing.assert_array_equal(na, nb)
+        for f in ("pos", "vel", "angVel", "force", "torque"):
+            np.testing.assert_array_equal(a.d.get(f), b.d.get(f), err_msg=f)
+    assert a.d.stats()["nRefresh"] == b.d.stats()["nRefresh"] > 2
+    if track:
+        assert a.d.energy() == b.d.energy()
+
+
+@pytest.mark.parametrize("n,walls", [(300, False), (5000, False), (5000, True)])
+def test_contacts_pulled_out_of_reach(n, walls):
+    # real contacts that are no near pairs at a refresh are appended behind the new pairs, and the real set
+    # and the adjacency made again with them: they persist (noBreak) and pull as in the oracle
+    from tests.scenes import build_gpu, build_oracle, contact_kw, deposition
+
+    sc = deposition(n=n, seed=n, dense=True, vel_sigma=.02)
+    sc["walls"] = [w for w in sc["walls"] if walls and (w["axis"], w["sense"]) != (0, -1)]
+    sc["gravity"] = (0., 0., 0.)
+    eng = ["Collider", "ContactLoop", "Leapfrog"]
+    o, d = build_oracle(sc, noBreak=1), build_gpu(sc)
+    kw = dict(contact=dict(contact_kw(sc), noBreak=1), leapfrog=dict(damping=sc["damping"]), dynDtPeriod=0)
+    st, _ = d.run(eng, 6, 0, sc["dt"], **kw)
+    o.run(eng, 6)
+    ids = d.contacts(real_only=True, data=False)[0]
+    pos = d.get("pos")
+    right = np.arange(len(pos)) < n  # spheres come before walls
+    right &= pos[:, 0] > sc["box"] / 2
+    pos[right, 0] += 3 * sc["radius"][0]
+    d.set("pos", pos)
+    o.set("pos", pos)
+    far = np.sum(right[ids[:, 0]] != right[ids[:, 1]])
+    assert far > n ** (2 / 3.) / 2
+    d.collide(-.05)
+    np.testing.assert_array_equal(d.contacts(real_only=True, data=False)[0], ids)
+    for steps in (1, 20):
+        st, _ = d.run(eng, steps, st, sc["dt"], **kw)
+        o.run(eng, steps)
+        np.testing.assert_array_equal(d.contacts(real_only=True, data=False)[0], o.contacts(real_only=True, data=False)[0])
+        for f in ("pos", "vel", "angVel", "ori"):
+            np.testing.assert_array_equal(d.get(f), o.get(f), err_msg=f)
 
 
 def _network_graph(rng, N, kind):
