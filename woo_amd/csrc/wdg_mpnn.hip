@@ -957,6 +957,10 @@ struct Mpnn {
   double *hres = nullptr, *hresDev = nullptr;  // the loss, in pinned host memory
   DBuf<uint8_t> cflag;  // node in contact (else in free flight)
   hipEvent_t done = nullptr;  // orders the network's stream and an engine context's stream
+  // the last learned step, which reads out and cflag on the stream of this context: a forward pass that
+  // follows it without a new graph from there (which orders the streams) waits for it
+  hipEvent_t moved = nullptr;
+  const Ctx* movedCtx = nullptr;
   // graphs kept on the device (training sets): inputs, structure and targets
   struct Kept {
     int64_t N = -1, E = 0;
@@ -1050,6 +1054,8 @@ static void forward(Mpnn& s, bool store) {
       s.mMask[l].ensure((size_t)std::max<int64_t>(E, 1));
     }
   if (N == 0) return;
+  if (s.movedCtx) WDG_HIP(hipStreamWaitEvent(s.stream, s.moved, 0));
+  s.movedCtx = nullptr;
   const int64_t nt = (N + 15) / 16;
   hipLaunchKernelGGL(k_enc, dim3(nblocks(nt, 4)), dim3(256), 0, s.stream, N, (const bf16*)s.X.p,
                      (const bf16*)(s.img.p + s.imgT[0]), (const float*)(s.P.p + s.L.encB), s.h[0].p);
@@ -1303,6 +1309,7 @@ int wdg_mpnn_create(int device, uint64_t seed, wdg_mpnn** out) {
     WDG_HIP(hipSetDevice(device));
     WDG_HIP(hipStreamCreate(&s.stream));
     WDG_HIP(hipEventCreateWithFlags(&s.done, hipEventDisableTiming));
+    WDG_HIP(hipEventCreateWithFlags(&s.moved, hipEventDisableTiming));
     WDG_HIP(hipHostMalloc((void**)&s.hres, sizeof(double), hipHostMallocDefault));
     WDG_HIP(hipHostGetDevicePointer((void**)&s.hresDev, s.hres, 0));
     const size_t n = s.L.total;
@@ -1361,6 +1368,7 @@ int wdg_mpnn_destroy(wdg_mpnn* m) {
   for (auto& k : s.kept) k.release();
   if (s.stream) (void)hipStreamSynchronize(s.stream);
   if (s.done) (void)hipEventDestroy(s.done);
+  if (s.moved) (void)hipEventDestroy(s.moved);
   if (s.stream) (void)hipStreamDestroy(s.stream);
   if (s.hres) (void)hipHostFree(s.hres);
   delete m;
@@ -1700,9 +1708,11 @@ int wdg_mpnn_graph_from_ctx(wdg_mpnn* m, wdg_ctx* ctx, double cutoff, double flo
       s.uidUploads = c.uploads;
       s.uidN = nSph;
     }
-    // the network's next kernels (its own stream) start after the graph is built
+    // the network's next kernels (its own stream) start after the graph is built, and so after a learned
+    // step queued before it on the same stream
     WDG_HIP(hipEventRecord(s.done, c.stream));
     WDG_HIP(hipStreamWaitEvent(s.stream, s.done, 0));
+    if (s.movedCtx == &c) s.movedCtx = nullptr;
     // output rows (spheres in user-id order) are found when an output is asked for
     s.outRow.clear();
     s.fromCtx = &c;
@@ -1734,9 +1744,8 @@ int wdg_mpnn_advance(wdg_mpnn* m, wdg_ctx* ctx, double dT) {
                          c.field.gravity[1], c.field.gravity[2], c.pos[0].p, c.pos[1].p, c.pos[2].p, c.vel[0].p, c.vel[1].p,
                          c.vel[2].p, (const uint32_t*)c.flags.p);
       WDG_LAUNCH_CHECK();
-      // the next forward pass, of whichever graph, writes the outputs that this step reads
-      WDG_HIP(hipEventRecord(s.done, c.stream));
-      WDG_HIP(hipStreamWaitEvent(s.stream, s.done, 0));
+      WDG_HIP(hipEventRecord(s.moved, c.stream));
+      s.movedCtx = &c;
     }
     c.dirtyKnown = false;
   });
