@@ -107,15 +107,15 @@ def algorithmic_bytes(n, slots, real):
       cellDist (20 B); per particle pos, vel, angVel, radius, mass, material (92 B); per
       real contact its slot index (4 B written, 4 B read), previous state read (trsf columns
       0-1, tangential force, contact point: 88 B), new state written (trsf columns 0-1,
-      local force, uN: 80 B) and the 64 B gather record written.
+      local force, uN: 80 B) and the 48 B gather record written.
     k_leapfrog (force gather fused): per particle flags, adjacency offset, pos/vel/angVel/ori
       read and written, mass, inertia, refresh position (272 B; force/torque are not
       touched while they hold the reset value); per slot two adjacency entries (8 B); per
-      real contact its 64 B gather record.
+      real contact its 48 B gather record and packed cellDist (8 B).
     """
     return {
-        "contact_loop": slots * 20 + n * 92 + real * (4 + 4 + 88 + 80 + 64),
-        "k_leapfrog": n * 272 + slots * 8 + real * 64,
+        "contact_loop": slots * 20 + n * 92 + real * (4 + 4 + 88 + 80 + 48),
+        "k_leapfrog": n * 272 + slots * 8 + real * (48 + 8),
     }
 
 
