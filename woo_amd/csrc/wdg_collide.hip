@@ -1,5 +1,5 @@
 // Broadphase: Verlet-skin refresh test, spatial re-sort of the particle
-// storage, cell-list pair generation over radix-sorted cell keys, and the merge
+// storage by counting per cell, pair generation over the cells, and the merge
 // that carries contact history across refreshes. Replaces
 // InsertionSortCollider::run (InsertionSortCollider.cpp:386-613).
 //
@@ -524,7 +524,7 @@ struct PairArgs {
   const uint32_t *sceneBodyOff, *sceneBody;
   const uint32_t* cbeg;  // k_cell_begin
   const double* bnd;  // enlarged AABB of every boundary body (min3, max3), k_bnd_bounds
-  const float4* pf;  // float candidate records (k_last_pos)
+  const float4* pf;  // float candidate records (k_permute)
   const double* vdS;  // per-scene Verlet distances (batched scenes with per-scene skins), else null
   int stage;          // OUT_STAGE: staged pairs per sphere
   int nbStage;        // OUT_STAGE: staged neighbours per sphere
