@@ -91,8 +91,7 @@ def test_a_forward_pass_waits_for_the_step_before():
         d.set("vel", 3. * d.get("vel"))
         net.graph_from(d)
         a = net.forward()
-        for k in range(40):  # some milliseconds of the engine's stream, none of which waits
-            d.kinetic_energy() if wait else None
+        for k in range(40):  # work on the engine's stream that nothing waits for
             d.contact_loop(step + k, 1e-12, physKind=1, lawKind=1, poisson=.25, en=.6)
         net.advance(d, COARSE * dt)
         if wait:
